@@ -638,3 +638,52 @@ def test_pressure_clamp_fixture_on_gpu():
         assert_close(dstar, z["c_dstar"], f"clamp dQ* ({where})")
         assert_close(dq, z["c_dq"], f"clamp dQ ({where})")
         assert_close(upts, z["c_upts1"], f"clamp upts ({where})")
+
+
+@pytest.mark.parametrize("kind,dims,order", [
+    ("hex", (5, 5, 5), "colour"),       # colours of 63 and 62 cells
+    ("hex", (4, 4, 8), "colour"),       # 64 and 64
+    ("hex", (13, 5, 2), "colour"),      # 65 and 65
+    ("hex", (5, 5, 5), "mesh"), ("hex", (13, 5, 2), "mesh"),
+    ("hex", (56, 54, 54), "mesh"),      # 81648 per colour: one wave per face
+    ("hex", (56, 55, 54), "mesh"),      # 83160 per colour: one thread per cell
+    ("hex", (80, 80, 77), "mesh"),      # 246400 per colour: one wave per face
+    ("quad", (9, 7, 1), "colour"), ("quad", (13, 10, 1), "mesh"),
+    ("tet", (51,), "colour"),           # 397953 per colour: one wave per face
+    ("tet", (52,), "colour"),           # 421824 per colour: one thread per cell
+])
+def test_wave_per_face_and_thread_per_cell_sweeps(kind, dims, order):
+    """Both forms of the sweep kernel at the edges of a 64-cell workgroup and on
+    either side of the sizes that choose between them, bit for bit against the
+    oracle, in the mesh's own numbering and on declared two-colour layouts."""
+    if kind == "tet":
+        mesh = M.tet_mesh(dims[0], seed=5)
+        mesh.key = M.hilbert_keys(mesh, "tet", dims)
+    else:
+        mesh = M.hex_mesh(*dims, seed=5, permute=False)
+    if kind == "quad":
+        mesh = M.Mesh(np.ascontiguousarray(mesh.nei_ele[:4]),
+                      np.ascontiguousarray(mesh.fnorm_vol[:4]),
+                      np.ascontiguousarray(mesh.vec_fnorm[:4, :2]), mesh.orig_id, mesh.key)
+    flow = M.flow_fields(mesh, seed=5)
+    cv = torch_dev()
+    if order == "colour":
+        lay = LY.colored_layout(mesh, flow, coloring="greedy-bfs")
+        mesh, flow, lc, ic = lay.mesh, lay.flow, lay.lcolor, lay.icolor
+    else:
+        _, lc, ic, _ = LY.greedy_coloring(mesh.nei_ele)
+    lcd, icd = cv(np.ascontiguousarray(lc)), cv(np.ascontiguousarray(ic))
+    D = mesh.ndims
+    L.call("ucfd_set_config", D + 2, D + 2, D)
+    try:
+        if order == "colour":
+            L.call("ucfd_declare_colored_layout", mesh.neles, icd, lcd, None)
+        got = colored_pass_lib(mesh, flow, lcd, icd, cv, two_array=order == "colour")
+    finally:
+        L.call("ucfd_set_config", 5, 5, 3)
+        if order == "colour":
+            L.call("ucfd_release_colored_layout", icd, lcd)
+    want = O.colored_pass(mesh.nei_ele, ic, lc, mesh.fnorm_vol, mesh.vec_fnorm, flow.fspr,
+                          flow.dt, flow.upts, flow.rhsb)
+    for g, w, what in zip(got, want, ("diag", "dQ*", "dQ", "upts")):
+        assert np.array_equal(g, w), what

@@ -206,3 +206,23 @@ def test_rans_sweeps_refuse_a_configuration_without_turbulence_rows():
                                           flow.upts.ctypes.data, flow.rhsb.ctypes.data,
                                           flow.dt.ctypes.data, flow.fspr.ctypes.data)
     assert rc == 1
+
+
+@pytest.mark.parametrize("kind, dims, nt", [
+    ("hex", (56, 54, 54), 2),       # 81648 cells a colour: one wave per face
+    ("hex", (56, 55, 54), 2),       # 83160: one thread per cell
+    ("tet", (52,), 1),              # 421824 a colour: one thread per cell when declared
+])
+def test_rans_sweeps_on_both_sides_of_the_kernel_choice(kind, dims, nt):
+    """Both forms of the turbulence-row kernel, declared (every face taken in
+    the second launch) and not, bit for bit against the oracle."""
+    mesh = M.tet_mesh(*dims, seed=7) if kind == "tet" else M.hex_mesh(*dims, seed=7)
+    mesh.key = M.hilbert_keys(mesh, kind, dims)
+    flow = M.flow_fields(mesh, seed=7, nvars=5 + nt)
+    lay = colored_layout(mesh, flow, coloring="greedy-bfs")
+    f2, tfspr = with_turbulence(lay.mesh, lay.flow, nt, 7)
+    L.call("ucfd_set_config", 5 + nt, 5, 3)
+    _, os_, oq = bridge_oracle(lay.mesh, f2, tfspr, 5)
+    for two, declare in ((True, True), (False, False)):
+        _, ds, dq = run_gpu(lay.mesh, f2, tfspr, 5, True, lay, two, True, declare)
+        assert np.array_equal(ds, os_) and np.array_equal(dq[5:], oq), (two, declare)

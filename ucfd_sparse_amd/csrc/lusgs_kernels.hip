@@ -238,6 +238,104 @@ __global__ __launch_bounds__(kSweepBlock) void k_sweep(
     if (RANGE && threadIdx.x == 0 && (sic != ib || slc != lce)) raise_flag(flag, UCFD_KFLAG_LAYOUT);
 }
 
+// The same sweep with one wave per face: a workgroup serves 64 cells with FC
+// waves, wave f computing face f's term of all 64 cells (every array access
+// of a wave is one row over consecutive cells), the terms meet in LDS and
+// wave k sums row k over the faces in index order, as k_sweep does (a face
+// not taken adds +0.0 to a sum that is never -0.0: the same bits).  FC times
+// as many waves with a quarter of the registers, and one round of loads per
+// face instead of FC/G rounds one after the other.
+template <int DIR, int MODE, int ND, int FC>
+__global__ __launch_bounds__(64*FC) void k_sweep_wf(
+    int n0, int cnt, int N, const int *__restrict__ nei, const int *__restrict__ order,
+    const int *__restrict__ lcolor, const double *__restrict__ fnv,
+    const double *__restrict__ vfn, const double *__restrict__ upts, const double *in,
+    double *out, const double *__restrict__ diag, const double *__restrict__ fspr, int *flag,
+    int lce)
+{
+    constexpr int NV = ND + 2, KW = (NV + FC - 1)/FC;
+    constexpr bool RANGE = MODE >= 2, EAGER = MODE == 3;
+    __shared__ double term[FC][NV][64];
+    const int lane = threadIdx.x & 63, f = threadIdx.x >> 6;
+    const int b0 = xcd_block()*64, t = b0 + lane;
+    int sic = 0, slc = 0;
+    if (RANGE) { sic = order[n0 + b0]; slc = lcolor[n0 + b0]; }
+    int i = -1;
+    if (t < cnt) {
+        i = RANGE ? n0 + t : order[n0 + t];
+        if ((unsigned)i >= (unsigned)N) {
+            raise_flag(flag, UCFD_KFLAG_INDEX);
+            i = -1;
+        }
+    }
+    double dg = 1.0, xin[KW], lam = 0.0, fv = 0.0, nf[ND], dfj[NV];
+    int nb = -1, ci = 0;
+    if (i >= 0) {
+        nb = ld_stream(nei + (size_t)f*N + i);
+        if (MODE == 0) ci = lcolor[i];
+        if (EAGER) {
+#pragma unroll
+            for (int d = 0; d < ND; ++d) nf[d] = ld_stream(vfn + (size_t)(f*ND + d)*N + i);
+            fv = ld_stream(fnv + (size_t)f*N + i);
+            lam = ld_stream(fspr + (size_t)f*N + i);
+        }
+        dg = diag[i];
+#pragma unroll
+        for (int q = 0; q < KW; ++q)
+            if (f + q*FC < NV) xin[q] = ld_stream(in + (size_t)(f + q*FC)*N + i);
+    }
+    bool tk = false;
+    if (i >= 0) {
+        if ((unsigned)nb >= (unsigned)N) {
+            raise_flag(flag, UCFD_KFLAG_INDEX);
+        } else if (MODE == 0) {
+            const int cn = lcolor[nb];
+            tk = DIR == 0 ? (cn < ci) : (cn > ci);
+        } else if (MODE == 1) {
+            tk = DIR == 0 ? (nb < i) : (nb > i);
+        } else {
+            tk = DIR == 0 ? (nb < n0) : (nb >= n0 + cnt);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < NV; ++k) dfj[k] = 0.0;
+    if (tk) {
+        double u[NV], du[NV];
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            u[k] = upts[(size_t)k*N + nb];
+            du[k] = out[(size_t)k*N + nb];
+        }
+        if (!EAGER) {
+#pragma unroll
+            for (int d = 0; d < ND; ++d) nf[d] = ld_stream(vfn + (size_t)(f*ND + d)*N + i);
+            fv = ld_stream(fnv + (size_t)f*N + i);
+            lam = ld_stream(fspr + (size_t)f*N + i);
+        }
+        ucfd::diff_flux<double, ND>(u, du, nf, dfj);
+#pragma unroll
+        for (int k = 0; k < NV; ++k) dfj[k] = (dfj[k] - lam*du[k])*fv;
+    }
+#pragma unroll
+    for (int k = 0; k < NV; ++k) term[f][k][lane] = dfj[k];
+    __syncthreads();
+    if (i >= 0) {
+#pragma unroll
+        for (int q = 0; q < KW; ++q) {
+            const int k = f + q*FC;
+            if (k >= NV) continue;
+            double df = 0.0;
+#pragma unroll
+            for (int g = 0; g < FC; ++g) df += term[g][k][lane];
+            const size_t o = (size_t)k*N + i;
+            if (DIR == 0) out[o] = (xin[q] - 0.5*df)/dg;
+            else          out[o] = xin[q] - (0.5*df/dg);
+        }
+    }
+    if (RANGE && threadIdx.x == 0 && (sic != n0 + b0 || slc != lce))
+        raise_flag(flag, UCFD_KFLAG_LAYOUT);
+}
+
 // A colour range where no face can be taken in range mode: the first colour
 // of a lower sweep (n0 == 0: no neighbour id lies below it) and the last of
 // an upper sweep (the range ends at N).  The face sum is empty, so the
@@ -375,10 +473,11 @@ __global__ __launch_bounds__(kSweepBlock) void k_rans_sweep(
     constexpr int NFV = ND + 2;
     const int t = xcd_block()*kSweepBlock + threadIdx.x;
     if (t >= cnt) return;
+    constexpr bool RANGE = MODE >= 2, EAGER = MODE == 3;
     int sic = 0, slc = 0;
     const int ib = n0 + xcd_block()*kSweepBlock;
-    if (MODE == 2) { sic = order[ib]; slc = lcolor[ib]; }
-    const int i = MODE == 2 ? n0 + t : ld_stream(order + n0 + t);
+    if (RANGE) { sic = order[ib]; slc = lcolor[ib]; }
+    const int i = RANGE ? n0 + t : ld_stream(order + n0 + t);
     if ((unsigned)i >= (unsigned)N) {
         raise_flag(flag, UCFD_KFLAG_INDEX);
         return;
@@ -388,6 +487,16 @@ __global__ __launch_bounds__(kSweepBlock) void k_rans_sweep(
     bool tk[FC];
 #pragma unroll
     for (int f = 0; f < FC; ++f) nbv[f] = ld_stream(nei + (size_t)f*N + i);
+    double nf[FC][ND], fv[FC], lam[FC];
+    if (EAGER) {
+#pragma unroll
+        for (int f = 0; f < FC; ++f) {
+#pragma unroll
+            for (int d = 0; d < ND; ++d) nf[f][d] = ld_stream(vfn + (size_t)(f*ND + d)*N + i);
+            fv[f] = ld_stream(fnv + (size_t)f*N + i);
+            lam[f] = ld_stream(tfspr + (size_t)f*N + i);
+        }
+    }
     const double dg = ld_stream(tdiag + i);
     double xin[NT];
 #pragma unroll
@@ -407,7 +516,7 @@ __global__ __launch_bounds__(kSweepBlock) void k_rans_sweep(
             tk[f] = DIR == 0 ? (nb < n0) : (nb >= n0 + cnt);
         }
     }
-    double rho[FC], m[FC][ND], ut[FC][NT], dut[FC][NT], nf[FC][ND], fv[FC], lam[FC];
+    double rho[FC], m[FC][ND], ut[FC][NT], dut[FC][NT];
 #pragma unroll
     for (int f = 0; f < FC; ++f) {
         if (!tk[f]) continue;
@@ -420,10 +529,12 @@ __global__ __launch_bounds__(kSweepBlock) void k_rans_sweep(
             ut[f][k] = upts[(size_t)(NFV + k)*N + nb];
             dut[f][k] = out[(size_t)(NFV + k)*N + nb];
         }
+        if (!EAGER) {
 #pragma unroll
-        for (int d = 0; d < ND; ++d) nf[f][d] = ld_stream(vfn + (size_t)(f*ND + d)*N + i);
-        fv[f] = ld_stream(fnv + (size_t)f*N + i);
-        lam[f] = ld_stream(tfspr + (size_t)f*N + i);
+            for (int d = 0; d < ND; ++d) nf[f][d] = ld_stream(vfn + (size_t)(f*ND + d)*N + i);
+            fv[f] = ld_stream(fnv + (size_t)f*N + i);
+            lam[f] = ld_stream(tfspr + (size_t)f*N + i);
+        }
     }
     double df[NT];
 #pragma unroll
@@ -447,8 +558,135 @@ __global__ __launch_bounds__(kSweepBlock) void k_rans_sweep(
         if (DIR == 0) __builtin_nontemporal_store((xin[k] - 0.5*df[k])/dg, out + o);
         else          __builtin_nontemporal_store(xin[k] - (0.5*df[k]/dg), out + o);
     }
-    if (MODE == 2 && threadIdx.x == 0 && (sic != ib || slc != lce))
+    if (RANGE && threadIdx.x == 0 && (sic != ib || slc != lce))
         raise_flag(flag, UCFD_KFLAG_LAYOUT);
+}
+
+// The turbulence rows with one wave per face (see k_sweep_wf).
+template <int DIR, int MODE, int ND, int NT, int FC>
+__global__ __launch_bounds__(64*FC) void k_rans_wf(
+    int n0, int cnt, int N, const int *__restrict__ nei, const int *__restrict__ order,
+    const int *__restrict__ lcolor, const double *__restrict__ fnv,
+    const double *__restrict__ vfn, const double *__restrict__ upts, const double *in,
+    double *out, const double *__restrict__ tdiag, const double *__restrict__ tfspr, int *flag,
+    int lce)
+{
+    constexpr int NFV = ND + 2;
+    constexpr bool RANGE = MODE >= 2, EAGER = MODE == 3;
+    static_assert(NT <= FC, "a wave per turbulence row");
+    __shared__ double term[FC][NT][64];
+    const int lane = threadIdx.x & 63, f = threadIdx.x >> 6;
+    const int b0 = xcd_block()*64, t = b0 + lane;
+    int sic = 0, slc = 0;
+    if (RANGE) { sic = order[n0 + b0]; slc = lcolor[n0 + b0]; }
+    int i = -1;
+    if (t < cnt) {
+        i = RANGE ? n0 + t : order[n0 + t];
+        if ((unsigned)i >= (unsigned)N) {
+            raise_flag(flag, UCFD_KFLAG_INDEX);
+            i = -1;
+        }
+    }
+    double dg = 1.0, xin = 0.0, lam = 0.0, fv = 0.0, nf[ND];
+    int nb = -1, ci = 0;
+    if (i >= 0) {
+        nb = ld_stream(nei + (size_t)f*N + i);
+        if (MODE == 0) ci = lcolor[i];
+        if (EAGER) {
+#pragma unroll
+            for (int d = 0; d < ND; ++d) nf[d] = ld_stream(vfn + (size_t)(f*ND + d)*N + i);
+            fv = ld_stream(fnv + (size_t)f*N + i);
+            lam = ld_stream(tfspr + (size_t)f*N + i);
+        }
+        if (f < NT) {
+            dg = tdiag[i];
+            xin = ld_stream(in + (size_t)(NFV + f)*N + i);
+        }
+    }
+    bool tk = false;
+    if (i >= 0) {
+        if ((unsigned)nb >= (unsigned)N) {
+            raise_flag(flag, UCFD_KFLAG_INDEX);
+        } else if (MODE == 0) {
+            const int cn = lcolor[nb];
+            tk = DIR == 0 ? (cn < ci) : (cn > ci);
+        } else if (MODE == 1) {
+            tk = DIR == 0 ? (nb < i) : (nb > i);
+        } else {
+            tk = DIR == 0 ? (nb < n0) : (nb >= n0 + cnt);
+        }
+    }
+    double tm[NT];
+#pragma unroll
+    for (int k = 0; k < NT; ++k) tm[k] = 0.0;
+    if (tk) {
+        double m[ND], ut[NT], dut[NT];
+        const double rho = upts[nb];
+#pragma unroll
+        for (int d = 0; d < ND; ++d) m[d] = upts[(size_t)(d + 1)*N + nb];
+#pragma unroll
+        for (int k = 0; k < NT; ++k) {
+            ut[k] = upts[(size_t)(NFV + k)*N + nb];
+            dut[k] = out[(size_t)(NFV + k)*N + nb];
+        }
+        if (!EAGER) {
+#pragma unroll
+            for (int d = 0; d < ND; ++d) nf[d] = ld_stream(vfn + (size_t)(f*ND + d)*N + i);
+            fv = ld_stream(fnv + (size_t)f*N + i);
+            lam = ld_stream(tfspr + (size_t)f*N + i);
+        }
+        double th = 0.0;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) th += m[d]*nf[d];
+        th /= rho;
+#pragma unroll
+        for (int k = 0; k < NT; ++k) {
+            const double dfj = (dut[k] + ut[k])*th - ut[k]*th;
+            tm[k] = (dfj - lam*dut[k])*fv;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < NT; ++k) term[f][k][lane] = tm[k];
+    __syncthreads();
+    if (i >= 0 && f < NT) {
+        double df = 0.0;
+#pragma unroll
+        for (int g = 0; g < FC; ++g) df += term[g][f][lane];
+        const size_t o = (size_t)(NFV + f)*N + i;
+        if (DIR == 0) out[o] = (xin - 0.5*df)/dg;
+        else          out[o] = xin - (0.5*df/dg);
+    }
+    if (RANGE && threadIdx.x == 0 && (sic != n0 + b0 || slc != lce))
+        raise_flag(flag, UCFD_KFLAG_LAYOUT);
+}
+
+// Which of the two forms serves a launch of cnt cells.  Small launches are a
+// chain of memory round trips on few CUs, and one wave per face shortens the
+// chain and spreads it.  Large launches of tets on a declared layout are bound
+// by the rate of their mixed streams and gathers, where the thread per cell
+// with every load of the cell in flight is ahead.  On a caller's own numbering
+// (MODE 0, 1) it is not: each launch touches most lines of every array, and the
+// extra waves hide more of it.  Times of a whole pass, us, thread per cell ->
+// wave per face (flow rows; cells in the mesh, two colours unless said):
+//   tets, declared: 197K 40.7 -> 37.2, 547K 88.0 -> 84.1, 1.6M (4-5 colours)
+//     277.7 -> 273.1; 1.6M 217.9 -> 220.4, 5.3M 655 -> 689
+//   tets, own numbering (4 colours): 48K 95 -> 55, 197K 143 -> 106,
+//     547K 264 -> 242, 3.1M 1344 -> 1265
+//   hexes, declared: 101K 32.9 -> 31.5, 486K 90.1 -> 87.9, 2.1M 350 -> 342
+//   hexes, own numbering: 101K 48.6 -> 45.1, 246K 81.7 -> 84.3,
+//     486K 150.9 -> 148.7, 1.0M 303 -> 291
+//   sequential sweeps of a 41x37x33 grid: 20.1 -> 10.0 us per level
+// kWfRound: the cells the chip holds at once as six-wave workgroups (5 per
+// CU); between one and three such rounds of hexes the last, partly filled one
+// costs what the extra waves bring.  With turbulence rows hexes gain below one
+// round only (101K 57.0 -> 53.8, 246K 89.0 -> 88.7, 1.0M 303.7 -> 309.7).
+constexpr int kWfRound = 256*5*64;
+constexpr int kWfTets = 400000;
+
+inline bool wave_per_face(int mode, int nface, int cnt)
+{
+    if (nface == 6) return mode >= 2 || cnt <= kWfRound || cnt >= 3*kWfRound;
+    return mode < 2 || cnt <= kWfTets;
 }
 
 template <int DIR, int MODE, int ND, int NT>
@@ -458,6 +696,20 @@ int launch_rans_f(hipStream_t s, int n0, int cnt, int N, int nface, const int *n
                   const double *tfspr, int *flag, int lce)
 {
     const dim3 g((cnt + kSweepBlock - 1)/kSweepBlock), b(kSweepBlock);
+    if (nface == 6 ? cnt <= kWfRound : wave_per_face(MODE, nface, cnt)) {
+        const dim3 gw((cnt + 63)/64);
+#define RW(FC) hipLaunchKernelGGL((k_rans_wf<DIR, MODE, ND, NT, FC>), gw, dim3(64*FC), 0, s, n0, \
+                                  cnt, N, nei, order, lcolor, fnv, vfn, upts, in, out, tdiag, \
+                                  tfspr, flag, lce)
+        switch (nface) {
+        case 3: RW(3); break;
+        case 4: RW(4); break;
+        case 6: RW(6); break;
+        default: return UCFD_ERR_ARG;
+        }
+#undef RW
+        return hipGetLastError() == hipSuccess ? UCFD_OK : UCFD_ERR_HIP;
+    }
 #define RL(FC) hipLaunchKernelGGL((k_rans_sweep<DIR, MODE, ND, NT, FC>), g, b, 0, s, n0, cnt, N, \
                                   nei, order, lcolor, fnv, vfn, upts, in, out, tdiag, tfspr, flag, lce)
     switch (nface) {
@@ -523,20 +775,30 @@ int launch_sweep_f(hipStream_t s, int n0, int cnt, int N, int nface, const int *
 {
     const dim3 grid((cnt + kBlock - 1)/kBlock), block(kBlock);
     const dim3 sgrid((cnt + kSweepBlock - 1)/kSweepBlock), sblock(kSweepBlock);
+    const dim3 wgrid((cnt + 63)/64);
+#define SW(K, FC, G, B, ...) hipLaunchKernelGGL((K<DIR, MODE, ND, FC>), G, B, 0, s, n0, cnt, N, \
+                                                ##__VA_ARGS__, nei, order, lcolor, fnv, vfn, \
+                                                upts, in, out, diag, fspr, flag, lce)
     switch (nface) {
     case 4:
-        hipLaunchKernelGGL((k_sweep<DIR, MODE, ND, 4>), sgrid, sblock, 0, s, n0, cnt, N, nface, nei,
-                           order, lcolor, fnv, vfn, upts, in, out, diag, fspr, flag, lce);
+        if (wave_per_face(MODE, 4, cnt)) SW(k_sweep_wf, 4, wgrid, dim3(256));
+        else SW(k_sweep, 4, sgrid, sblock, nface);
         break;
     case 6:
-        hipLaunchKernelGGL((k_sweep<DIR, MODE, ND, 6>), sgrid, sblock, 0, s, n0, cnt, N, nface, nei,
-                           order, lcolor, fnv, vfn, upts, in, out, diag, fspr, flag, lce);
+        // range launches of hexes always take the wave-per-face kernel
+        if constexpr (MODE >= 2) {
+            SW(k_sweep_wf, 6, wgrid, dim3(384));
+        } else {
+            if (wave_per_face(MODE, 6, cnt)) SW(k_sweep_wf, 6, wgrid, dim3(384));
+            else SW(k_sweep, 6, sgrid, sblock, nface);
+        }
         break;
     default:
         hipLaunchKernelGGL((k_sweep_any<DIR, MODE, ND>), grid, block, 0, s, n0, cnt, N, nface,
                            nei, order, lcolor, fnv, vfn, upts, in, out, diag, fspr, flag, lce);
         break;
     }
+#undef SW
     return hipGetLastError() == hipSuccess ? UCFD_OK : UCFD_ERR_HIP;
 }
 
@@ -690,6 +952,8 @@ int ucfd_launch_rans_sweep(hipStream_t s, int dir, int mode, int n0, int ne, int
                                             tfspr, flag, lc_expect)
     if (mode == UCFD_SWEEP_COLORED) { if (dir == 0) RM(0, 0); RM(1, 0); }
     if (mode == UCFD_SWEEP_ORDERED) { if (dir == 0) RM(0, 1); RM(1, 1); }
+    // every face taken, as in ucfd_launch_sweep
+    if (dir == 0 ? ne == neles : n0 == 0) { if (dir == 0) RM(0, 3); RM(1, 3); }
     if (dir == 0) RM(0, 2);
     RM(1, 2);
 #undef RM
