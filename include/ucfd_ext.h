@@ -200,6 +200,15 @@ int ucfd_adjoint_destroy(void *handle);
 int ucfd_lusgs_adjoint(void *handle, double factor, const double *dt, const double *fspr,
                        const double *dstar, const double *dq, const double *w, double *rhsbar,
                        double *dtbar, double *fsprbar);
+/* The forward pass itself on the handle's mesh, in one call (with the default
+ * synchronous stream: one wait): parallel_pre_lusgs into diag, then
+ * ns_parallel_lower_sweep for every colour (rhsb -> dstar), then
+ * ns_parallel_upper_sweep in reverse (dstar -> dq).  dstar NULL: the in-place
+ * sweeps on dq (first a copy of rhsb); dq NULL: pre and the lower sweeps only.
+ * icolor / lcolor as in those calls (the declared pointers of the layout). */
+int ucfd_lusgs_pass(void *handle, double factor, const int *icolor, const int *lcolor,
+                    const double *dt, const double *fspr, const double *rhsb, double *dstar,
+                    double *dq, double *diag);
 
 #ifdef __cplusplus
 }

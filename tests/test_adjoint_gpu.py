@@ -114,3 +114,38 @@ def test_non_coloured_layout_is_rejected():
     rc = lib.ucfd_adjoint_create(ctypes.byref(h), mesh.neles, mesh.nface, 1, off.ctypes.data,
                                  nei.data_ptr(), None, None, None)
     assert rc != 0
+
+
+@pytest.mark.parametrize("coloring", ["greedy", "greedy-bfs"])
+def test_one_call_pass_equals_the_separate_calls(coloring):
+    """ucfd_lusgs_pass (both forms, and the lower half alone) against
+    parallel_pre_lusgs and the per-colour sweep calls, bit for bit."""
+    import torch
+
+    from ucfd_sparse_amd import lib as L
+    from ucfd_sparse_amd import mesh as M
+    from ucfd_sparse_amd.autograd import ColoredSystem
+    from ucfd_sparse_amd.layout import colored_layout
+    L.call("ucfd_set_config", 5, 5, 3)
+    mesh = M.tet_mesh(6, seed=4)
+    lay = colored_layout(mesh, M.flow_fields(mesh, seed=4), coloring=coloring)
+    S = ColoredSystem(lay)
+    rhsb, dt, fspr = (torch.from_numpy(a).cuda() for a in (lay.flow.rhsb, lay.flow.dt,
+                                                           lay.flow.fspr))
+    diag, dstar, dq = torch.zeros_like(dt), torch.zeros_like(rhsb), torch.zeros_like(rhsb)
+    mesh_args = (S.N, S.F, S.nei, S.icolor, S.lcolor, S.fnv, S.vfn, S.upts)
+    L.call("parallel_pre_lusgs", S.N, S.F, 1.5, S.fnv, dt, diag, fspr)
+    for c in range(len(S.off) - 1):
+        L.call("ns_parallel_lower_sweep", S.off[c], S.off[c + 1], *mesh_args, rhsb, dstar, diag,
+               fspr)
+    for c in reversed(range(len(S.off) - 1)):
+        L.call("ns_parallel_upper_sweep", S.off[c], S.off[c + 1], *mesh_args, dq, dstar, diag, fspr)
+    got = S.forward_arrays(rhsb, dt, fspr, 1.5)
+    assert all(torch.equal(g, w) for g, w in zip(got, (dq, dstar, diag)))
+    assert torch.equal(S.forward_inplace(rhsb, dt, fspr, 1.5), dq)
+    assert torch.equal(S.recompute_dstar(rhsb, dt, fspr, 1.5), dstar)
+    with pytest.raises(L.UCFDError):
+        S.nei[2, 5] = S.N + 3
+        S.forward_arrays(rhsb, dt, fspr)
+    S.nei[2, 5] = 5
+    S.forward_arrays(rhsb, dt, fspr)        # the raised error was cleared

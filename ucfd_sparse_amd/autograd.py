@@ -3,9 +3,10 @@ dQ = upper(lower(pre(dt, fspr), rhsb)) as a torch.autograd.Function whose
 backward is the library's hand-written adjoint (ucfd_lusgs_adjoint,
 include/ucfd_ext.h).
 
-The forward runs the legacy API (parallel_pre_lusgs, ns_parallel_lower_sweep
-per colour, ns_parallel_upper_sweep per colour in reverse) on device tensors
-of a colour-contiguous layout, on torch's current stream.  The lower sweep's
+The forward runs the legacy API's pass (parallel_pre_lusgs, ns_parallel_lower_sweep
+per colour, ns_parallel_upper_sweep per colour in reverse, as one library
+call) on device tensors of a colour-contiguous layout, on torch's current
+stream.  The lower sweep's
 output dQ* is either kept for the backward (two-array sweeps: rhsb -> dQ*,
 dQ* -> dQ) or, with recompute=True, never kept: the forward runs the
 in-place sweeps on one buffer (rhsb copy -> dQ* -> dQ) and the backward
@@ -50,7 +51,7 @@ class ColoredSystem:
 
         def up(a):
             return torch.from_numpy(np.ascontiguousarray(a)).to(dev)
-        self.N, self.F = m.neles, m.nface
+        self.N, self.F, self.rows = m.neles, m.nface, m.ndims + 2
         self.nei, self.fnv, self.vfn = up(m.nei_ele), up(m.fnorm_vol), up(m.vec_fnorm)
         self.upts = up(f.upts)
         self.icolor, self.lcolor = up(lay.icolor), up(lay.lcolor)
@@ -79,68 +80,41 @@ class ColoredSystem:
             if v is not None:
                 L.arr(v, np.float64, sizes[k], k, device=True)
 
+    def _out(self, like):
+        """An output of the pass: the sweeps write every cell of the NFVARS rows,
+        only rows beyond them start from zero."""
+        return (torch.empty_like if like.numel() == self.rows * self.N else torch.zeros_like)(like)
+
+    def _pass(self, rhsb, dt, fspr, factor, dstar, dq, diag=None):
+        """ucfd_lusgs_pass on torch's current stream; returns diag."""
+        diag = torch.empty(self.N, dtype=torch.float64, device=rhsb.device) if diag is None else diag
+        with _Stream(self.lib):
+            L.check(self.lib.ucfd_lusgs_pass(
+                self.handle, float(factor), self.icolor.data_ptr(), self.lcolor.data_ptr(),
+                dt.data_ptr(), fspr.data_ptr(), rhsb.data_ptr(),
+                None if dstar is None else dstar.data_ptr(),
+                None if dq is None else dq.data_ptr(), diag.data_ptr()), "ucfd_lusgs_pass")
+        return diag
+
     def forward_arrays(self, rhsb, dt, fspr, factor=1.0, dq=None, dstar=None, diag=None):
         """pre + lower + upper on torch's current stream; returns (dq, dstar, diag)."""
-        lib, N, F = self.lib, self.N, self.F
         self.check_inputs(rhsb, dt, fspr, dq=dq, dstar=dstar, diag=diag)
-        diag = torch.empty(N, dtype=torch.float64, device=rhsb.device) if diag is None else diag
-        dstar = torch.zeros_like(rhsb) if dstar is None else dstar
-        dq = torch.zeros_like(rhsb) if dq is None else dq
-        p = dict(nei=self.nei.data_ptr(), ic=self.icolor.data_ptr(), lc=self.lcolor.data_ptr(),
-                 fnv=self.fnv.data_ptr(), vfn=self.vfn.data_ptr(), up=self.upts.data_ptr())
-        with _Stream(lib):
-            L.check(lib.parallel_pre_lusgs(N, F, float(factor), p["fnv"], dt.data_ptr(),
-                                           diag.data_ptr(), fspr.data_ptr()), "pre")
-            self._lower(p, rhsb, dstar, diag, fspr)
-            for c in reversed(range(len(self.off) - 1)):
-                L.check(lib.ns_parallel_upper_sweep(
-                    self.off[c], self.off[c + 1], N, F, p["nei"], p["ic"], p["lc"], p["fnv"],
-                    p["vfn"], p["up"], dq.data_ptr(), dstar.data_ptr(), diag.data_ptr(),
-                    fspr.data_ptr()), "upper")
-        return dq, dstar, diag
-
-    def _lower(self, p, rhsb, dstar, diag, fspr):
-        lib, N, F = self.lib, self.N, self.F
-        for c in range(len(self.off) - 1):
-            L.check(lib.ns_parallel_lower_sweep(
-                self.off[c], self.off[c + 1], N, F, p["nei"], p["ic"], p["lc"], p["fnv"],
-                p["vfn"], p["up"], rhsb.data_ptr(), dstar.data_ptr(), diag.data_ptr(),
-                fspr.data_ptr()), "lower")
+        dstar = self._out(rhsb) if dstar is None else dstar
+        dq = self._out(rhsb) if dq is None else dq
+        return dq, dstar, self._pass(rhsb, dt, fspr, factor, dstar, dq, diag)
 
     def forward_inplace(self, rhsb, dt, fspr, factor=1.0):
         """pre + lower + upper with the in-place C sweeps on one buffer;
         returns dQ (dQ* is overwritten by the upper sweep)."""
-        lib, N, F = self.lib, self.N, self.F
         self.check_inputs(rhsb, dt, fspr)
-        diag = torch.empty(N, dtype=torch.float64, device=rhsb.device)
-        dub = rhsb.clone()
-        p = dict(nei=self.nei.data_ptr(), ic=self.icolor.data_ptr(), lc=self.lcolor.data_ptr(),
-                 fnv=self.fnv.data_ptr(), vfn=self.vfn.data_ptr(), up=self.upts.data_ptr())
-        with _Stream(lib):
-            L.check(lib.parallel_pre_lusgs(N, F, float(factor), p["fnv"], dt.data_ptr(),
-                                           diag.data_ptr(), fspr.data_ptr()), "pre")
-            nc = len(self.off) - 1
-            for c in range(nc):
-                L.check(lib.parallel_ns_lower_sweep(
-                    self.off[c], self.off[c + 1], N, F, p["nei"], p["ic"], p["lc"], p["fnv"],
-                    p["vfn"], p["up"], dub.data_ptr(), diag.data_ptr(), fspr.data_ptr()), "lower")
-            for c in reversed(range(nc)):
-                L.check(lib.parallel_ns_upper_sweep(
-                    self.off[c], self.off[c + 1], N, F, p["nei"], p["ic"], p["lc"], p["fnv"],
-                    p["vfn"], p["up"], dub.data_ptr(), diag.data_ptr(), fspr.data_ptr()), "upper")
+        dub = torch.empty_like(rhsb) if rhsb.numel() == self.rows * self.N else rhsb.clone()
+        self._pass(rhsb, dt, fspr, factor, None, dub)
         return dub
 
     def recompute_dstar(self, rhsb, dt, fspr, factor=1.0):
-        lib = self.lib
         self.check_inputs(rhsb, dt, fspr)
-        diag = torch.empty(self.N, dtype=torch.float64, device=rhsb.device)
-        dstar = torch.zeros_like(rhsb)
-        p = dict(nei=self.nei.data_ptr(), ic=self.icolor.data_ptr(), lc=self.lcolor.data_ptr(),
-                 fnv=self.fnv.data_ptr(), vfn=self.vfn.data_ptr(), up=self.upts.data_ptr())
-        with _Stream(lib):
-            L.check(lib.parallel_pre_lusgs(self.N, self.F, float(factor), p["fnv"],
-                                           dt.data_ptr(), diag.data_ptr(), fspr.data_ptr()), "pre")
-            self._lower(p, rhsb, dstar, diag, fspr)
+        dstar = self._out(rhsb)
+        self._pass(rhsb, dt, fspr, factor, dstar, None)
         return dstar
 
     def adjoint(self, dt, fspr, dstar, dq, w, factor=1.0, overwrite_dstar=False):
@@ -148,7 +122,7 @@ class ColoredSystem:
         the rhsb gradient is written into dstar's buffer and returned."""
         w = w.contiguous()
         self.check_inputs(None, dt, fspr, dq=dq, dstar=dstar, w=w)
-        rb = dstar if overwrite_dstar else torch.zeros_like(dq)
+        rb = dstar if overwrite_dstar else self._out(dq)
         dtb = torch.empty_like(dt)
         fb = torch.empty_like(fspr)
         with _Stream(self.lib):

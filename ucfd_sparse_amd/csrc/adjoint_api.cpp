@@ -153,3 +153,59 @@ UCFD_API int ucfd_lusgs_adjoint(void *handle, double factor, const double *dt, c
                                (double *)sg.dev(irb), (double *)sg.dev(idb), (double *)sg.dev(ifb));
     return sg.leave(rc);
 }
+
+// The forward the adjoint belongs to, in one call: pre, the lower sweeps of
+// every colour and the upper sweeps in reverse, on the handle's mesh.  dstar
+// and dq given: rhsb -> dstar -> dq; dstar NULL: in place on dq (a copy of
+// rhsb first); dq NULL: pre and the lower sweeps only.
+UCFD_API int ucfd_lusgs_pass(void *handle, double factor, const int *icolor, const int *lcolor,
+                             const double *dt, const double *fspr, const double *rhsb,
+                             double *dstar, double *dq, double *diag)
+{
+    const char *fn = "ucfd_lusgs_pass";
+    Adjoint *A = (Adjoint *)handle;
+    if (!A || (!dstar && !dq)) return ucfd_report(UCFD_ERR_ARG, fn, "NULL handle or outputs");
+    const UcfdConfig &cfg = ucfd_config();
+    if (cfg.ndims != A->ndims || cfg.nfvars != A->ndims + 2)
+        return ucfd_report(UCFD_ERR_STATE, fn, "configuration changed since create");
+    const int N = A->neles, F = A->nface, nc = (int)A->off.size() - 1;
+    const size_t n = (size_t)N, vec = sizeof(double)*(size_t)cfg.nfvars*n,
+                 row = sizeof(double)*n, ids = sizeof(int)*n;
+    UcfdStage sg(fn);
+    const int inei = sg.add(A->nei, ids*F, UCFD_IN);
+    const int iic = sg.add(icolor, ids, UCFD_IN), ilc = sg.add(lcolor, ids, UCFD_IN);
+    const int ifnv = sg.add(A->fnv, row*F, UCFD_IN), ivfn = sg.add(A->vfn, row*F*A->ndims, UCFD_IN);
+    const int iup = sg.add(A->upts, vec, UCFD_IN), idt = sg.add(dt, row, UCFD_IN);
+    const int ifs = sg.add(fspr, row*F, UCFD_IN), irh = sg.add(rhsb, vec, UCFD_IN);
+    const int ids_ = dstar ? sg.add(dstar, vec, UCFD_OUT) : -1;
+    const int idq = dq ? sg.add(dq, vec, UCFD_OUT) : -1;
+    const int idg = sg.add(diag, row, UCFD_OUT);
+    int rc = sg.enter();
+    if (rc) return rc;
+    const hipStream_t s = ucfd_stream();
+    const int *nei = (const int *)sg.dev(inei), *ic = (const int *)sg.dev(iic),
+              *lc = (const int *)sg.dev(ilc);
+    const double *fnv = (const double *)sg.dev(ifnv), *vfn = (const double *)sg.dev(ivfn),
+                 *up = (const double *)sg.dev(iup), *fs = (const double *)sg.dev(ifs),
+                 *rh = (const double *)sg.dev(irh);
+    double *dg = (double *)sg.dev(idg), *q = dq ? (double *)sg.dev(idq) : nullptr;
+    double *ds = dstar ? (double *)sg.dev(ids_) : q;
+    if (!dstar) {
+        rc = ucfd_check_hip(hipMemcpyAsync(q, rh, vec, hipMemcpyDeviceToDevice, s), fn,
+                            "hipMemcpyAsync(rhsb)");
+        rh = q;
+    }
+    if (!rc) rc = ucfd_launch_pre(s, N, F, factor, fnv, (const double *)sg.dev(idt), dg, fs);
+    for (int k = 0; k < 2*nc && !rc; ++k) {
+        const bool upper = k >= nc;
+        if (upper && !q) break;
+        const int c = upper ? 2*nc - 1 - k : k, n0 = A->off[c], ne = A->off[c + 1];
+        int lv = 0;
+        const int mode = ucfd_colored_mode(icolor, lcolor, N, n0, ne, &lv);
+        rc = ucfd_launch_sweep(s, upper, mode, n0, ne, N, F, A->ndims, cfg.nfvars, nei, ic, lc,
+                               fnv, vfn, up, upper ? ds : rh, upper ? q : ds, dg, fs,
+                               ucfd_device_flag(), lv);
+    }
+    if (rc) ucfd_report(rc, fn, "kernel launch failed");
+    return sg.leave(rc);
+}

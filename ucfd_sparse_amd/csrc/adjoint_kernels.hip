@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include "adjoint_internal.h"
+#include "error_word.h"
 #include "flux.h"
 
 namespace {
@@ -37,11 +38,11 @@ __global__ __launch_bounds__(AB) void k_pairs(int64_t N, int F, const int *__res
         const int64_t nb = nei[f*N + i];
         int pf = -1;
         if ((uint64_t)nb >= (uint64_t)N) {
-            atomicOr(flag, UCFD_KFLAG_INDEX);
+            ucfd::raise(flag, UCFD_KFLAG_INDEX);
         } else if (nb != i) {
             for (int g = 0; g < F; ++g)
                 if (nei[g*N + nb] == i) { pf = g; break; }
-            if (pf < 0) atomicOr(flag, UCFD_KFLAG_INDEX);
+            if (pf < 0) ucfd::raise(flag, UCFD_KFLAG_INDEX);
         }
         pair[f*N + i] = pf;
     }

@@ -11,6 +11,7 @@
 #include <type_traits>
 
 #include "block_lu.h"
+#include "error_word.h"
 #include "flowsys_internal.h"
 #include "flux.h"
 #include "wave_rows.h"
@@ -59,7 +60,7 @@ __global__ __launch_bounds__(64) void k_pack(int neles, int nlocal, int nvars, i
     if (lane < nact) {
         r = cell_ids[e];
         if ((unsigned)r >= (unsigned)nlocal) {
-            atomicOr(flag, UCFD_KFLAG_INDEX);
+            ucfd::raise(flag, UCFD_KFLAG_INDEX);
             r = -1;
         }
         dg = 1/dt[e] + a0;
@@ -109,7 +110,7 @@ __global__ __launch_bounds__(FB) void k_bpack_rec(int neles, int nlocal, double 
     if (e >= neles) return;
     const int r = cell_ids[e];
     if ((unsigned)r >= (unsigned)nlocal) {
-        atomicOr(flag, UCFD_KFLAG_INDEX);
+        ucfd::raise(flag, UCFD_KFLAG_INDEX);
         return;
     }
     inv[r] = e;
@@ -191,7 +192,7 @@ __global__ __launch_bounds__(FB) void k_tpack(int neles, int nlocal, int nvars, 
     if (e >= neles) return;
     const int r = cell_ids[e];
     if ((unsigned)r >= (unsigned)nlocal) {
-        atomicOr(flag, UCFD_KFLAG_INDEX);
+        ucfd::raise(flag, UCFD_KFLAG_INDEX);
         return;
     }
     if (NT > 0) {
@@ -240,7 +241,7 @@ __global__ __launch_bounds__(FB) void k_update(int neles, int nlocal, int nvars,
     if (e >= neles) return;
     const int r = cell_ids[e];
     if ((unsigned)r >= (unsigned)nlocal) {
-        atomicOr(flag, UCFD_KFLAG_INDEX);
+        ucfd::raise(flag, UCFD_KFLAG_INDEX);
         return;
     }
     for (int k = 0; k < nvars; ++k) upts[e + (int64_t)k*neles] += du[k + (int64_t)r*nvars];
@@ -258,7 +259,7 @@ __global__ __launch_bounds__(FB) void k_subres(int neles, int nlocal, int nvars,
     if (e >= neles) return;
     const int r = cell_ids[e];
     if ((unsigned)r >= (unsigned)nlocal) {
-        atomicOr(flag, UCFD_KFLAG_INDEX);
+        ucfd::raise(flag, UCFD_KFLAG_INDEX);
         return;
     }
     for (int k = 0; k < nvars; ++k) {
@@ -428,7 +429,7 @@ __global__ __launch_bounds__(64) void k_prep_diag(int nlocal, int64_t nfaces,
 #pragma unroll
         for (int c = 0; c < NV; ++c) m[rr*NV + c] = __shfl(dm[c], g*NV + rr, 64);
     if (!act) return;
-    if (!ucfd::ludcmp<NV>(m) && row == 0) atomicOr(flag, UCFD_KFLAG_PIVOT);
+    if (!ucfd::ludcmp<NV>(m) && row == 0) ucfd::raise(flag, UCFD_KFLAG_PIVOT);
     // this lane's row, selected with constant indices (an index that depends
     // on the lane would place m in scratch memory)
     double o[NV];
@@ -672,10 +673,10 @@ __global__ __launch_bounds__(FB) void k_lpack_inv(int neles, int nlocal,
     if (e >= neles) return;
     const int r = cell_ids[e];
     if ((unsigned)r >= (unsigned)nlocal) {
-        atomicOr(flag, UCFD_KFLAG_INDEX);
+        ucfd::raise(flag, UCFD_KFLAG_INDEX);
         return;
     }
-    if (atomicExch(inv + r, e) >= 0) atomicOr(flag, UCFD_KFLAG_DUP);
+    if (atomicExch(inv + r, e) >= 0) ucfd::raise(flag, UCFD_KFLAG_DUP);
 }
 
 __global__ __launch_bounds__(FB) void k_lpack_rank(int neles, int nlocal, int nvars, int nfvars,
@@ -738,10 +739,10 @@ __global__ __launch_bounds__(FB) void k_lpack_rec(int neles, int nlocal, int nfv
     if (e >= neles) return;
     const int r = cell_ids[e];
     if ((unsigned)r >= (unsigned)nlocal) {
-        atomicOr(flag, UCFD_KFLAG_INDEX);
+        ucfd::raise(flag, UCFD_KFLAG_INDEX);
         return;
     }
-    if (atomicExch(inv + r, e) >= 0) atomicOr(flag, UCFD_KFLAG_DUP);
+    if (atomicExch(inv + r, e) >= 0) ucfd::raise(flag, UCFD_KFLAG_DUP);
     const double dte = dt[e];
     double v[W];
 #pragma unroll
@@ -812,7 +813,7 @@ __global__ __launch_bounds__(FB) void k_lupdate_from_rec(int neles, int nlocal,
     if (e >= neles) return;
     const int r = cell_ids[e];
     if ((unsigned)r >= (unsigned)nlocal) {
-        atomicOr(flag, UCFD_KFLAG_INDEX);
+        ucfd::raise(flag, UCFD_KFLAG_INDEX);
         return;
     }
     const fs_d2 *in = (const fs_d2 *)(rec + (int64_t)r*W);
@@ -837,7 +838,7 @@ __global__ __launch_bounds__(FB) void k_lupdate(int neles, int nlocal, int nvars
     if (e >= neles) return;
     const int r = cell_ids[e];
     if ((unsigned)r >= (unsigned)nlocal) {
-        atomicOr(flag, UCFD_KFLAG_INDEX);
+        ucfd::raise(flag, UCFD_KFLAG_INDEX);
         return;
     }
     for (int k = 0; k < nvars; ++k) upts[e + (int64_t)k*neles] += du[r + (int64_t)k*nlocal];

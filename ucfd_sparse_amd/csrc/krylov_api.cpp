@@ -985,7 +985,7 @@ UCFD_API ucfd_status_t UCFDSolve(Solver solver, Precon pc, SpMat A, UCFDReal *x,
         rc = gmres(solver, pc, A, md, pd, xd, bd, ucfd_stream(), fn);
     else
         rc = bicgstab(solver, pc, A, md, pd, xd, bd, ucfd_stream(), fn);
-    // a solve is synchronous: the result and the device error word are final on return
+    // a solve is synchronous: the result and the error word are final on return
     if (!rc) rc = ucfd_sync_and_check(fn);
     return status(sg.leave(rc));
 }

@@ -15,6 +15,7 @@
 #include <type_traits>
 
 #include "block_lu.h"
+#include "error_word.h"
 #include "krylov_internal.h"
 #include "wave_rows.h"
 
@@ -74,7 +75,7 @@ __global__ __launch_bounds__(KB) void k_spmv_bsr(int bn, const int *__restrict__
         const int64_t o = (int64_t)idx*B + k;
         y[o] = alpha*arr[k] + beta*y[o];
     }
-    if (bad) atomicOr(flag, UCFD_KFLAG_INDEX);
+    if (bad) ucfd::raise(flag, UCFD_KFLAG_INDEX);
 }
 
 // Block sizes 2..7: one wave per G = 64/B block rows (wave_rows.h).  The
@@ -177,7 +178,7 @@ __global__ __launch_bounds__(64) void k_spmv_bsr_w(int bn, const int *__restrict
         const int64_t o = (int64_t)i*B + r;
         y[o] = alpha*arr + beta*y[o];
     }
-    if (bad) atomicOr(flag, UCFD_KFLAG_INDEX);
+    if (bad) ucfd::raise(flag, UCFD_KFLAG_INDEX);
 }
 
 __global__ __launch_bounds__(KB) void k_spmv_csr(int n, const int *__restrict__ rowptr,
@@ -196,7 +197,7 @@ __global__ __launch_bounds__(KB) void k_spmv_csr(int n, const int *__restrict__ 
         else bad = true;
     }
     y[i] = alpha*s + beta*y[i];
-    if (bad) atomicOr(flag, UCFD_KFLAG_INDEX);
+    if (bad) ucfd::raise(flag, UCFD_KFLAG_INDEX);
 }
 
 template <int B>
@@ -210,7 +211,7 @@ __global__ __launch_bounds__(KB) void k_prepare(int bn, const int *__restrict__ 
     const double *src = values + (int64_t)diagslots[i]*B*B;
 #pragma unroll
     for (int q = 0; q < B*B; ++q) a[q] = src[q];
-    if (!ucfd::ludcmp<B>(a)) atomicOr(flag, UCFD_KFLAG_PIVOT);
+    if (!ucfd::ludcmp<B>(a)) ucfd::raise(flag, UCFD_KFLAG_PIVOT);
 #pragma unroll
     for (int q = 0; q < B*B; ++q) dv[(int64_t)i*B*B + q] = a[q];
 }
@@ -292,7 +293,7 @@ __global__ __launch_bounds__(KB) void k_ilu_factor(int base, int cnt, const int 
     }
 #pragma unroll
     for (int q = 0; q < B2; ++q) dv[(int64_t)i*B2 + q] = d[q];
-    if (bad) atomicOr(flag, UCFD_KFLAG_PIVOT);
+    if (bad) ucfd::raise(flag, UCFD_KFLAG_PIVOT);
 }
 
 // The block form on one wave per G = 64/B rows of a level: lane (g, r) owns
@@ -379,7 +380,7 @@ __global__ __launch_bounds__(64) void k_ilu_factor_w(int base, int cnt,
 #pragma unroll
         for (int c = 0; c < B; ++c) d[rr*B + c] = __shfl(dr[c], g*B + rr, 64);
     if (!act) return;
-    if (!ucfd::ludcmp<B>(d) && r == 0) atomicOr(flag, UCFD_KFLAG_PIVOT);
+    if (!ucfd::ludcmp<B>(d) && r == 0) ucfd::raise(flag, UCFD_KFLAG_PIVOT);
     double o[B];
 #pragma unroll
     for (int c = 0; c < B; ++c) o[c] = d[c];

@@ -64,6 +64,17 @@ bool whole_colour_of_declared(const int *icolor, const int *lcolor, int neles, i
     return false;
 }
 
+}  // namespace
+
+int ucfd_colored_mode(const int *icolor, const int *lcolor, int neles, int n0, int ne,
+                      int *lc_value)
+{
+    return whole_colour_of_declared(icolor, lcolor, neles, n0, ne, lc_value) ? UCFD_SWEEP_RANGE
+                                                                             : UCFD_SWEEP_COLORED;
+}
+
+namespace {
+
 int do_pre(const char *fn, int neles, int nface, double factor, const double *fnorm_vol,
            const double *dt, double *diag, const double *fspr)
 {
@@ -131,8 +142,7 @@ int do_colored(const char *fn, int dir, int n0, int ne, int neles, int nface, co
     const int a_dg = sg.add(diag, N*8, UCFD_IN);
     const int a_sp = sg.add(fspr, F*N*8, UCFD_IN);
     int lc_value = 0;
-    const int mode = whole_colour_of_declared(icolor, lcolor, neles, n0, ne, &lc_value)
-                         ? UCFD_SWEEP_RANGE : UCFD_SWEEP_COLORED;
+    const int mode = ucfd_colored_mode(icolor, lcolor, neles, n0, ne, &lc_value);
     int rc = sg.enter();
     if (rc) return rc;
     if (rans)

@@ -11,8 +11,9 @@
 // -ffp-contract=off so no FMA is introduced.
 //
 // Every gathered index is bounds checked; an out-of-range entry raises
-// UCFD_KFLAG_INDEX in the device error word and the face (or cell) is
+// UCFD_KFLAG_INDEX in the error words and the face (or cell) is
 // skipped, so a malformed index array cannot make the kernel fault.
+#include "error_word.h"
 #include "flux.h"
 #include "ucfd_internal.h"
 
@@ -23,11 +24,6 @@ constexpr int kBlock = 256;
 // three such workgroups (12 waves).  Measured on the 2.65M-cell heavy
 // launch: 201 us against 210 us with 128 threads and 218 us with 64.
 constexpr int kSweepBlock = 256;
-
-__device__ __forceinline__ void raise_flag(int *flag, int bit)
-{
-    atomicOr(flag, bit);
-}
 
 __global__ __launch_bounds__(kBlock) void k_pre(int N, int nface, double factor,
                                                 const double *__restrict__ fnv,
@@ -145,7 +141,7 @@ __global__ __launch_bounds__(kSweepBlock) void k_sweep(
     if (RANGE) { sic = order[ib]; slc = lcolor[ib]; }
     const int i = RANGE ? n0 + t : ld_stream(order + n0 + t);
     if ((unsigned)i >= (unsigned)N) {
-        raise_flag(flag, UCFD_KFLAG_INDEX);
+        ucfd::raise(flag, UCFD_KFLAG_INDEX);
         return;
     }
     int ci = 0;
@@ -175,7 +171,7 @@ __global__ __launch_bounds__(kSweepBlock) void k_sweep(
     for (int f = 0; f < FC; ++f) {
         const int nb = nbv[f];
         if ((unsigned)nb >= (unsigned)N) {
-            raise_flag(flag, UCFD_KFLAG_INDEX);
+            ucfd::raise(flag, UCFD_KFLAG_INDEX);
             tk[f] = false;
         } else if (MODE == 0) {
             const int cn = lcolor[nb];
@@ -235,7 +231,7 @@ __global__ __launch_bounds__(kSweepBlock) void k_sweep(
         if (DIR == 0) __builtin_nontemporal_store((xin[k] - 0.5*df[k])/dg, out + o);
         else          __builtin_nontemporal_store(xin[k] - (0.5*df[k]/dg), out + o);
     }
-    if (RANGE && threadIdx.x == 0 && (sic != ib || slc != lce)) raise_flag(flag, UCFD_KFLAG_LAYOUT);
+    if (RANGE && threadIdx.x == 0 && (sic != ib || slc != lce)) ucfd::raise(flag, UCFD_KFLAG_LAYOUT);
 }
 
 // The same sweep with one wave per face: a workgroup serves 64 cells with FC
@@ -264,7 +260,7 @@ __global__ __launch_bounds__(64*FC) void k_sweep_wf(
     if (t < cnt) {
         i = RANGE ? n0 + t : order[n0 + t];
         if ((unsigned)i >= (unsigned)N) {
-            raise_flag(flag, UCFD_KFLAG_INDEX);
+            ucfd::raise(flag, UCFD_KFLAG_INDEX);
             i = -1;
         }
     }
@@ -287,7 +283,7 @@ __global__ __launch_bounds__(64*FC) void k_sweep_wf(
     bool tk = false;
     if (i >= 0) {
         if ((unsigned)nb >= (unsigned)N) {
-            raise_flag(flag, UCFD_KFLAG_INDEX);
+            ucfd::raise(flag, UCFD_KFLAG_INDEX);
         } else if (MODE == 0) {
             const int cn = lcolor[nb];
             tk = DIR == 0 ? (cn < ci) : (cn > ci);
@@ -333,7 +329,7 @@ __global__ __launch_bounds__(64*FC) void k_sweep_wf(
         }
     }
     if (RANGE && threadIdx.x == 0 && (sic != n0 + b0 || slc != lce))
-        raise_flag(flag, UCFD_KFLAG_LAYOUT);
+        ucfd::raise(flag, UCFD_KFLAG_LAYOUT);
 }
 
 // A colour range where no face can be taken in range mode: the first colour
@@ -385,7 +381,7 @@ __global__ __launch_bounds__(kBlock) void k_sweep_none(int n0, int cnt, int N,
             else          out[o] = xin[c][k] - (0.5*df/dg[c]);
         }
     }
-    if (threadIdx.x == 0 && (sic != ib || slc != lce)) raise_flag(flag, UCFD_KFLAG_LAYOUT);
+    if (threadIdx.x == 0 && (sic != ib || slc != lce)) ucfd::raise(flag, UCFD_KFLAG_LAYOUT);
 }
 
 // Any other face count: one face at a time.
@@ -402,11 +398,11 @@ __global__ __launch_bounds__(kBlock) void k_sweep_any(
     if (t >= cnt) return;
     if (MODE >= 2 && threadIdx.x == 0) {
         const int ib = n0 + xcd_block()*kBlock;
-        if (order[ib] != ib || lcolor[ib] != lce) raise_flag(flag, UCFD_KFLAG_LAYOUT);
+        if (order[ib] != ib || lcolor[ib] != lce) ucfd::raise(flag, UCFD_KFLAG_LAYOUT);
     }
     const int i = MODE >= 2 ? n0 + t : order[n0 + t];
     if ((unsigned)i >= (unsigned)N) {
-        raise_flag(flag, UCFD_KFLAG_INDEX);
+        ucfd::raise(flag, UCFD_KFLAG_INDEX);
         return;
     }
     int ci = 0;
@@ -417,7 +413,7 @@ __global__ __launch_bounds__(kBlock) void k_sweep_any(
     for (int f = 0; f < nface; ++f) {
         const int nb = nei[(size_t)f*N + i];
         if ((unsigned)nb >= (unsigned)N) {
-            raise_flag(flag, UCFD_KFLAG_INDEX);
+            ucfd::raise(flag, UCFD_KFLAG_INDEX);
             continue;
         }
         bool take;
@@ -479,7 +475,7 @@ __global__ __launch_bounds__(kSweepBlock) void k_rans_sweep(
     if (RANGE) { sic = order[ib]; slc = lcolor[ib]; }
     const int i = RANGE ? n0 + t : ld_stream(order + n0 + t);
     if ((unsigned)i >= (unsigned)N) {
-        raise_flag(flag, UCFD_KFLAG_INDEX);
+        ucfd::raise(flag, UCFD_KFLAG_INDEX);
         return;
     }
     const int ci = MODE == 0 ? lcolor[i] : 0;
@@ -505,7 +501,7 @@ __global__ __launch_bounds__(kSweepBlock) void k_rans_sweep(
     for (int f = 0; f < FC; ++f) {
         const int nb = nbv[f];
         if ((unsigned)nb >= (unsigned)N) {
-            raise_flag(flag, UCFD_KFLAG_INDEX);
+            ucfd::raise(flag, UCFD_KFLAG_INDEX);
             tk[f] = false;
         } else if (MODE == 0) {
             const int cn = lcolor[nb];
@@ -559,7 +555,7 @@ __global__ __launch_bounds__(kSweepBlock) void k_rans_sweep(
         else          __builtin_nontemporal_store(xin[k] - (0.5*df[k]/dg), out + o);
     }
     if (RANGE && threadIdx.x == 0 && (sic != ib || slc != lce))
-        raise_flag(flag, UCFD_KFLAG_LAYOUT);
+        ucfd::raise(flag, UCFD_KFLAG_LAYOUT);
 }
 
 // The turbulence rows with one wave per face (see k_sweep_wf).
@@ -583,7 +579,7 @@ __global__ __launch_bounds__(64*FC) void k_rans_wf(
     if (t < cnt) {
         i = RANGE ? n0 + t : order[n0 + t];
         if ((unsigned)i >= (unsigned)N) {
-            raise_flag(flag, UCFD_KFLAG_INDEX);
+            ucfd::raise(flag, UCFD_KFLAG_INDEX);
             i = -1;
         }
     }
@@ -606,7 +602,7 @@ __global__ __launch_bounds__(64*FC) void k_rans_wf(
     bool tk = false;
     if (i >= 0) {
         if ((unsigned)nb >= (unsigned)N) {
-            raise_flag(flag, UCFD_KFLAG_INDEX);
+            ucfd::raise(flag, UCFD_KFLAG_INDEX);
         } else if (MODE == 0) {
             const int cn = lcolor[nb];
             tk = DIR == 0 ? (cn < ci) : (cn > ci);
@@ -657,7 +653,7 @@ __global__ __launch_bounds__(64*FC) void k_rans_wf(
         else          out[o] = xin - (0.5*df/dg);
     }
     if (RANGE && threadIdx.x == 0 && (sic != n0 + b0 || slc != lce))
-        raise_flag(flag, UCFD_KFLAG_LAYOUT);
+        ucfd::raise(flag, UCFD_KFLAG_LAYOUT);
 }
 
 // Which of the two forms serves a launch of cnt cells.  Small launches are a

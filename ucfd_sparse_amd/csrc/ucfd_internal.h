@@ -20,8 +20,9 @@ enum {
     UCFD_ERR_NUMERIC = 6     // non-finite value or zero pivot detected
 };
 
-// Bits raised by kernels in the device error word.
+// Error bits raised by kernels, one word each (error_word.h).
 enum { UCFD_KFLAG_INDEX = 1, UCFD_KFLAG_PIVOT = 2, UCFD_KFLAG_LAYOUT = 4, UCFD_KFLAG_DUP = 8 };
+constexpr int UCFD_KFLAG_COUNT = 4;
 
 // Flow-variable configuration of the legacy API (compile-time in the
 // reference: NVARS / NFVARS / NDIMS, Makefile.inc:21-24).
@@ -37,11 +38,11 @@ UCFD_HIDDEN int ucfd_check_hip(hipError_t e, const char *fn, const char *what);
 UCFD_HIDDEN hipStream_t ucfd_stream();
 UCFD_HIDDEN bool ucfd_stream_is_user();
 UCFD_HIDDEN const UcfdConfig &ucfd_config();
-UCFD_HIDDEN int *ucfd_device_flag();          // device error word (per process)
+UCFD_HIDDEN int *ucfd_device_flag();          // error words (per process)
 UCFD_HIDDEN int ucfd_ensure_device(const char *fn);
 UCFD_HIDDEN bool ucfd_is_device_ptr(const void *p);
-// Wait for the library stream; a raised device error word becomes a status
-// (and is cleared).  Call with the runtime lock held or outside any staging.
+// Wait for the library stream; a raised error bit becomes a status (and is
+// cleared).  Call with the runtime lock held or outside any staging.
 UCFD_HIDDEN int ucfd_sync_and_check(const char *fn);
 
 // Staging of host arrays for one call.  Device (or managed) pointers are used
@@ -64,6 +65,13 @@ struct UcfdStage {
     int leave(int status);
     void *dev(int idx) const { return args[idx].dev; }
 };
+
+// ---- legacy API (legacy_api.cpp)
+// Sweep mode of a coloured call on cells [n0, ne): UCFD_SWEEP_RANGE (and the
+// colour's lcolor value) when they are one whole colour of a layout declared
+// with these pointers, else UCFD_SWEEP_COLORED.
+UCFD_HIDDEN int ucfd_colored_mode(const int *icolor, const int *lcolor, int neles, int n0, int ne,
+                                  int *lc_value);
 
 // ---- kernel launchers (lusgs_kernels.hip)
 enum { UCFD_SWEEP_COLORED = 0, UCFD_SWEEP_ORDERED = 1, UCFD_SWEEP_RANGE = 2 };

@@ -78,6 +78,7 @@ _SIGS = {
     "ucfd_adjoint_create": [c_void_p, c_int, c_int, c_int] + [c_void_p] * 5,
     "ucfd_adjoint_destroy": [c_void_p],
     "ucfd_lusgs_adjoint": [c_void_p, c_double] + [c_void_p] * 8,
+    "ucfd_lusgs_pass": [c_void_p, c_double] + [c_void_p] * 8,
     # Krylov API (include/ucfdmat.h, ucfdprecon.h, ucfdsolver.h); handles are
     # passed by address (SpMat*, Precon*, Solver*) or by value (void*)
     "UCFDMatInit": [c_void_p],
