@@ -3,6 +3,7 @@ against the CPU adjoint oracle on the same inputs, and the
 torch.autograd.Function (ucfd_sparse_amd.autograd.LUSGSPass) against central
 differences of the GPU forward (h = 1e-6, FP64), with dQ* stored and
 recomputed (identical gradients)."""
+import ctypes
 import math
 
 import numpy as np
@@ -10,6 +11,7 @@ import pytest
 
 from oracle import pyoracle as O
 from ucfd_sparse_amd import layout as LY
+from ucfd_sparse_amd import lib as L
 from ucfd_sparse_amd import mesh as M
 
 pytestmark = pytest.mark.gpu
@@ -120,15 +122,10 @@ def test_non_coloured_layout_is_rejected():
 def test_one_call_pass_equals_the_separate_calls(coloring):
     """ucfd_lusgs_pass (both forms, and the lower half alone) against
     parallel_pre_lusgs and the per-colour sweep calls, bit for bit."""
-    import torch
-
-    from ucfd_sparse_amd import lib as L
-    from ucfd_sparse_amd import mesh as M
     from ucfd_sparse_amd.autograd import ColoredSystem
-    from ucfd_sparse_amd.layout import colored_layout
     L.call("ucfd_set_config", 5, 5, 3)
     mesh = M.tet_mesh(6, seed=4)
-    lay = colored_layout(mesh, M.flow_fields(mesh, seed=4), coloring=coloring)
+    lay = LY.colored_layout(mesh, M.flow_fields(mesh, seed=4), coloring=coloring)
     S = ColoredSystem(lay)
     rhsb, dt, fspr = (torch.from_numpy(a).cuda() for a in (lay.flow.rhsb, lay.flow.dt,
                                                            lay.flow.fspr))
@@ -149,3 +146,40 @@ def test_one_call_pass_equals_the_separate_calls(coloring):
         S.forward_arrays(rhsb, dt, fspr)
     S.nei[2, 5] = 5
     S.forward_arrays(rhsb, dt, fspr)        # the raised error was cleared
+
+
+@pytest.mark.parametrize("kind,dims", [("hex", (5, 5, 5)), ("hex", (4, 4, 8)), ("hex", (13, 5, 2)),
+                                       ("quad", (13, 10, 1)), ("quad", (9, 7, 1)), ("tet", (4,))])
+def test_adjoint_at_workgroup_edges(kind, dims):
+    """Colours of 62 to 65 cells (one 64-cell workgroup, just under and just
+    over) and every face count the meshes have, against the adjoint oracle."""
+    mesh = M.tet_mesh(*dims, seed=9) if kind == "tet" else M.hex_mesh(*dims, seed=9)
+    if kind == "quad":
+        mesh = M.Mesh(np.ascontiguousarray(mesh.nei_ele[:4]),
+                      np.ascontiguousarray(mesh.fnorm_vol[:4]),
+                      np.ascontiguousarray(mesh.vec_fnorm[:4, :2]), mesh.orig_id, mesh.key)
+    lay = LY.colored_layout(mesh, M.flow_fields(mesh, seed=9), coloring="greedy-bfs")
+    m, f = lay.mesh, lay.flow
+    N, F, D = m.neles, m.nface, m.ndims
+    rng = np.random.default_rng(9)
+    w = rng.normal(size=(D + 2, N))
+    _, ds, dq, _ = O.colored_pass(m.nei_ele, lay.icolor, lay.lcolor, m.fnorm_vol, m.vec_fnorm,
+                                  f.fspr, f.dt, f.upts, f.rhsb)
+    want = O.lusgs_adjoint(m.nei_ele, lay.off, m.fnorm_vol, m.vec_fnorm, f.fspr, f.dt, f.upts, ds,
+                           dq, w)
+    off = np.ascontiguousarray(lay.off, np.int32)
+    mesh_d = [dev(a) for a in (m.nei_ele, m.fnorm_vol, m.vec_fnorm, f.upts)]
+    dt, fspr, dqd, wd = dev(f.dt), dev(f.fspr), dev(dq), dev(w)
+    dtb, fb, h = torch.zeros_like(dt), torch.zeros_like(fspr), ctypes.c_void_p()
+    L.call("ucfd_set_config", D + 2, D + 2, D)
+    try:
+        L.call("ucfd_adjoint_create", h, N, F, len(off) - 1, off, *mesh_d)
+        for alias in (False, True):
+            dsd = dev(ds)
+            rb = dsd if alias else torch.zeros_like(dsd)
+            L.call("ucfd_lusgs_adjoint", h.value, 1.0, dt, fspr, dsd, dqd, wd, rb, dtb, fb)
+            for g, o, what in zip((rb, dtb, fb), want, ("rhsb", "dt", "fspr")):
+                assert np.abs(g.cpu().numpy() - o).max() <= 1e-13 * np.abs(o).max(), (what, alias)
+    finally:
+        L.load().ucfd_adjoint_destroy(h)
+        L.call("ucfd_set_config", 5, 5, 3)

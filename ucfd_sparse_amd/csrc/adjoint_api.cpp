@@ -23,8 +23,7 @@ struct Adjoint {
     const int *nei = nullptr;
     const double *fnv = nullptr, *vfn = nullptr, *upts = nullptr;
     int *pair = nullptr;           // device [nface, neles]
-    double *diag = nullptr;        // device [neles]
-    double *work = nullptr;        // device [nfvars, neles]
+    double *rec = nullptr;         // device, one record per cell (adjoint and diagonal)
 };
 
 }  // namespace
@@ -66,13 +65,11 @@ UCFD_API int ucfd_adjoint_create(void **handle, int neles, int nface, int ncolor
     A->fnv = fnorm_vol;
     A->vfn = vec_fnorm;
     A->upts = upts;
-    const size_t nf = (size_t)cfg.nfvars*neles;
+    const size_t nrec = adj_rec_doubles(cfg.ndims)*neles;
     if ((rc = ucfd_check_hip(hipMalloc((void **)&A->pair, sizeof(int)*(size_t)nface*neles), fn,
                              "hipMalloc(pair)")) ||
-        (rc = ucfd_check_hip(hipMalloc((void **)&A->diag, sizeof(double)*neles), fn,
-                             "hipMalloc(diag)")) ||
-        (rc = ucfd_check_hip(hipMalloc((void **)&A->work, sizeof(double)*nf), fn,
-                             "hipMalloc(work)"))) {
+        (rc = ucfd_check_hip(hipMalloc((void **)&A->rec, sizeof(double)*nrec), fn,
+                             "hipMalloc(records)"))) {
         ucfd_adjoint_destroy(A);
         return rc;
     }
@@ -100,8 +97,7 @@ UCFD_API int ucfd_adjoint_destroy(void *handle)
     if (!A) return UCFD_OK;
     (void)hipStreamSynchronize(ucfd_stream());
     if (A->pair) (void)hipFree(A->pair);
-    if (A->diag) (void)hipFree(A->diag);
-    if (A->work) (void)hipFree(A->work);
+    if (A->rec) (void)hipFree(A->rec);
     delete A;
     return UCFD_OK;
 }
@@ -137,19 +133,18 @@ UCFD_API int ucfd_lusgs_adjoint(void *handle, double factor, const double *dt, c
     const int *nei = (const int *)sg.dev(inei);
     const double *fnv = (const double *)sg.dev(ifnv), *vfn = (const double *)sg.dev(ivfn);
     const double *fs = (const double *)sg.dev(ifs), *dtd = (const double *)sg.dev(idt);
-    rc = ucfd_launch_pre(s, A->neles, A->nface, factor, fnv, dtd, A->diag, fs);
     const int nc = (int)A->off.size() - 1;
     for (int c = 0; c < nc && !rc; ++c)
         rc = adj_launch_colour(s, 0, A->off[c], A->off[c + 1], A->neles, A->nface, A->ndims, nei,
-                               A->pair, fnv, vfn, fs, dtd, factor, A->diag,
-                               (const double *)sg.dev(iup), (const double *)sg.dev(ids),
-                               (const double *)sg.dev(idq), (const double *)sg.dev(iw), A->work,
+                               A->pair, fnv, vfn, fs, dtd, factor, (const double *)sg.dev(iup),
+                               (const double *)sg.dev(ids), (const double *)sg.dev(idq),
+                               (const double *)sg.dev(iw), A->rec,
                                nullptr, nullptr, nullptr);
     for (int c = nc - 1; c >= 0 && !rc; --c)
         rc = adj_launch_colour(s, 1, A->off[c], A->off[c + 1], A->neles, A->nface, A->ndims, nei,
-                               A->pair, fnv, vfn, fs, dtd, factor, A->diag,
-                               (const double *)sg.dev(iup), (const double *)sg.dev(ids),
-                               (const double *)sg.dev(idq), (const double *)sg.dev(iw), A->work,
+                               A->pair, fnv, vfn, fs, dtd, factor, (const double *)sg.dev(iup),
+                               (const double *)sg.dev(ids), (const double *)sg.dev(idq),
+                               (const double *)sg.dev(iw), A->rec,
                                (double *)sg.dev(irb), (double *)sg.dev(idb), (double *)sg.dev(ifb));
     return sg.leave(rc);
 }
