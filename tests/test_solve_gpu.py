@@ -148,3 +148,27 @@ def test_solver_rejects_invalid_colouring():
     with pytest.raises(L.UCFDError):
         LUSGSSolver(m.neles, 4, bad, m.nei_ele, m.fnorm_vol, m.vec_fnorm, f.fspr, f.dt,
                     np.ascontiguousarray(f.upts[:5]))
+
+
+@pytest.mark.parametrize("kind,dims", [("hex", (5, 5, 5)), ("hex", (4, 4, 8)), ("hex", (13, 5, 2)),
+                                       ("tet", (58,)),      # 585336 a colour: one wave per face
+                                       ("tet", (59,))])     # 616137: one thread per cell
+def test_solves_at_workgroup_edges_and_on_both_sides_of_the_kernel_choice(kind, dims):
+    """Colours of 62 to 65 cells and the two kernel forms at their boundary: both
+    precision forms reach 1e-10 by the oracle's residual, and agree."""
+    mesh = M.tet_mesh(*dims, seed=11) if kind == "tet" else M.hex_mesh(*dims, seed=11)
+    mesh.key = M.hilbert_keys(mesh, kind, dims)
+    lay = colored_layout(mesh, M.flow_fields(mesh, seed=11), coloring="greedy-bfs")
+    m, f = lay.mesh, lay.flow
+    s = LUSGSSolver.from_layout(lay)
+    b, out = dev(f.rhsb[:5]), []
+    for mode in ("fp64", "mixed"):
+        dq = dev(np.zeros((5, m.neles)))
+        st = s.solve(b, dq, mode, 1e-10, 200)
+        assert st.converged and st.rel_residual <= 1e-10
+        out.append(dq.cpu().numpy())
+        _, no = O.residual(m.nei_ele, m.fnorm_vol, m.vec_fnorm, f.fspr, f.dt, f.upts, f.rhsb,
+                           out[-1])
+        assert no <= 2e-10 * np.linalg.norm(f.rhsb[:5])
+    assert np.abs(out[1] - out[0]).max() <= 1e-8 * np.abs(out[0]).max()
+    s.close()

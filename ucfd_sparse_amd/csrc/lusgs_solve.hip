@@ -443,6 +443,176 @@ __global__ __launch_bounds__(kSB) void k_upper_upd_res(
     block_sum<kSB>(ss, part, pofs + b);
 }
 
+// ---- the same launches with one wave per face (wave_per_face says when): a
+// small colour is a chain of round trips on part of the chip, which FC times the
+// waves with one face's loads each shorten and spread.  A workgroup serves 64 cells with FC
+// waves, wave f forming face f's terms; they meet in LDS, and wave k updates
+// component k (k, k + FC, ...) of the cells with the expressions of the kernels
+// above, summing the faces in index order (a face not taken adds +0.0 to a sum
+// that is never -0.0), so the vectors are the same bits.  Partial sums of the
+// norm are one per 64 cells.
+constexpr int kWF = 64;
+
+// component q of cell i in the split layout
+template <typename T> __device__ __forceinline__ T *at_split(T *p, int N, int i, int q)
+{
+    return q < 4 ? p + 4*(size_t)i + q : p + 4*(size_t)N + i;
+}
+
+// sum over the workgroup's waves of the lanes' sums, in a fixed order
+template <int WAVES>
+__device__ __forceinline__ void wf_sum(double v, double *part, int slot)
+{
+    __shared__ double red[WAVES];
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double s = 0.0;
+        for (int q = 0; q < WAVES; ++q) s += red[q];
+        part[slot] = s;
+    }
+}
+
+template <typename T, int FC, bool WITH_RES, bool LAST>
+__global__ __launch_bounds__(64*FC) void k_lower_res_wf(
+    int n0, int cnt, int N, const int *__restrict__ nei, const Face4<T> *__restrict__ geo,
+    const T *__restrict__ diag, const T *__restrict__ qb, const T *__restrict__ rhs, T *e,
+    T *dstar, double *part, int pofs, T *delta)
+{
+    constexpr int KW = (NV + FC - 1)/FC;
+    __shared__ T slow[FC][NV][64], sres[WITH_RES ? FC : 1][NV][64];
+    const int lane = threadIdx.x & 63, f = threadIdx.x >> 6;
+    const int b = xcd_remap(), t = b*64 + lane, i = n0 + t;
+    const bool act = t < cnt;
+    T dg = T(1), rh[KW], ei[KW], low[NV], res[NV];
+#pragma unroll
+    for (int q = 0; q < NV; ++q) low[q] = res[q] = T(0);
+    if (act) {
+        const int nb = nei[(size_t)f*N + i];
+        dg = diag[i];
+#pragma unroll
+        for (int w = 0; w < KW; ++w) {
+            const int q = f + w*FC;
+            if (q >= NV) continue;
+            rh[w] = rhs[(size_t)q*N + i];
+            ei[w] = WITH_RES || LAST ? *at_split(e, N, i, q) : T(0);
+        }
+        const bool res_f = WITH_RES && nb != i, low_f = nb < n0;
+        if (res_f || low_f) {
+            T U[NV], dr[NV], dl[NV];
+            const Face4<T> g = ldg_nt(geo + (size_t)f*N + i);
+            ld_split<false>(qb, N, nb, U);
+            if (res_f) ld_split<false>(e, N, nb, dr);
+            if (low_f) ld_split<false>(dstar, N, nb, dl);
+            if (res_f) face_term<T>(U, dr, g, res);
+            if (low_f) face_term<T>(U, dl, g, low);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+        slow[f][q][lane] = low[q];
+        if (WITH_RES) sres[f][q][lane] = res[q];
+    }
+    __syncthreads();
+    double ss = 0.0;
+    if (act) {
+#pragma unroll
+        for (int w = 0; w < KW; ++w) {
+            const int q = f + w*FC;
+            if (q >= NV) continue;
+            T s = rh[w], acc = T(0);
+            if (WITH_RES) {
+                T r = T(0);
+#pragma unroll
+                for (int g = 0; g < FC; ++g) r += sres[WITH_RES ? g : 0][q][lane];
+                s = s - (dg*ei[w] + T(0.5)*r);
+            }
+            ss += (double)s*(double)s;
+#pragma unroll
+            for (int g = 0; g < FC; ++g) acc += slow[g][q][lane];
+            const T o = (s - T(0.5)*acc)/dg;
+            if (LAST) {
+                const T acc0 = T(0), dlt = o - T(0.5)*acc0/dg;
+                *at_split(delta, N, i, q) = dlt;
+                *at_split(e, N, i, q) = ei[w] + dlt;
+            } else {
+                *at_split(dstar, N, i, q) = o;
+            }
+        }
+    }
+    wf_sum<FC>(ss, part, pofs + b);
+}
+
+// RES: the first colour ([n0, n0+cnt) = [0, cnt)), with the next pass's
+// residual and dstar (k_upper_upd_res); otherwise k_upper_upd
+template <typename T, int FC, bool RES>
+__global__ __launch_bounds__(64*FC) void k_upper_wf(
+    int n0, int cnt, int N, const int *__restrict__ nei, const Face4<T> *__restrict__ geo,
+    const T *__restrict__ diag, const T *__restrict__ qb, T *dstar, T *delta, T *e,
+    const T *__restrict__ rhs, double *part, int pofs)
+{
+    constexpr int KW = (NV + FC - 1)/FC;
+    __shared__ T sup[FC][NV][64], sres[RES ? FC : 1][NV][64];
+    const int lane = threadIdx.x & 63, f = threadIdx.x >> 6;
+    const int b = xcd_remap(), t = b*64 + lane, i = n0 + t, ne = n0 + cnt;
+    const bool act = t < cnt;
+    T dg = T(1), rh[KW], ds[KW], ei[KW], up[NV], res[NV];
+#pragma unroll
+    for (int q = 0; q < NV; ++q) up[q] = res[q] = T(0);
+    if (act) {
+        const int nb = nei[(size_t)f*N + i];
+        dg = diag[i];
+#pragma unroll
+        for (int w = 0; w < KW; ++w) {
+            const int q = f + w*FC;
+            if (q >= NV) continue;
+            if (RES) rh[w] = rhs[(size_t)q*N + i];
+            ds[w] = *at_split(dstar, N, i, q);
+            ei[w] = *at_split(e, N, i, q);
+        }
+        if (nb >= ne) {
+            T U[NV], d[NV], en[NV];
+            const Face4<T> g = ldg_nt(geo + (size_t)f*N + i);
+            ld_split<false>(qb, N, nb, U);
+            ld_split<false>(delta, N, nb, d);
+            if (RES) ld_split<false>(e, N, nb, en);
+            face_term<T>(U, d, g, up);
+            if (RES) face_term<T>(U, en, g, res);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+        sup[f][q][lane] = up[q];
+        if (RES) sres[f][q][lane] = res[q];
+    }
+    __syncthreads();
+    double ss = 0.0;
+    if (act) {
+#pragma unroll
+        for (int w = 0; w < KW; ++w) {
+            const int q = f + w*FC;
+            if (q >= NV) continue;
+            T acc = T(0);
+#pragma unroll
+            for (int g = 0; g < FC; ++g) acc += sup[g][q][lane];
+            const T dl = ds[w] - T(0.5)*acc/dg, en = ei[w] + dl;
+            *at_split(e, N, i, q) = en;
+            if (!RES) {
+                *at_split(delta, N, i, q) = dl;
+                continue;
+            }
+            T r = T(0);
+#pragma unroll
+            for (int g = 0; g < FC; ++g) r += sres[RES ? g : 0][q][lane];
+            const T sq = rh[w] - (dg*en + T(0.5)*r), acc0 = T(0);
+            ss += (double)sq*(double)sq;
+            *at_split(dstar, N, i, q) = (sq - T(0.5)*acc0)/dg;
+        }
+    }
+    if (RES) wf_sum<FC>(ss, part, pofs + b);
+}
+
 // ---- FP64 residual r = b - A(dq) on base Q (split layout) over all cells;
 // dq in the split layout (DQS: the solver's own increment) or [var][cell]
 // (a caller's array).  Optionally writes fl32(r) ([var][cell]) and the FP32
@@ -518,10 +688,11 @@ __global__ __launch_bounds__(kSB) void k_residual64(
 // Sum of the block partials in a fixed order (thread t sums t, t+1024, ...
 // with eight loads in flight, then a fixed tree), so the norm and every
 // convergence decision are reproducible run to run.
-// The result goes to out (device) and to hout (pinned host memory, read by
-// the host after a stream synchronisation: no copy kernel).
+// The result goes to out (device) and to hout (pinned host memory: the value,
+// then the launch's sequence number, which the host polls while the launches
+// behind this one run: no copy kernel and no wait for the stream).
 __global__ __launch_bounds__(1024) void k_sum_parts(const double *part, int n, double *out,
-                                                    double *hout)
+                                                    double *hout, unsigned long long seq)
 {
     constexpr int U = 8;
     __shared__ double red[16];
@@ -543,7 +714,11 @@ __global__ __launch_bounds__(1024) void k_sum_parts(const double *part, int n, d
         double t = 0.0;
         for (int w = 0; w < 16; ++w) t += red[w];
         *out = t;
-        if (hout) *hout = t;
+        if (hout) {
+            __hip_atomic_store(hout, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store((unsigned long long *)hout + 1, seq, __ATOMIC_RELEASE,
+                               __HIP_MEMORY_SCOPE_SYSTEM);
+        }
     }
 }
 
@@ -717,6 +892,7 @@ struct ucfd_lusgs_solver {
           *delta32 = nullptr;
     double *part = nullptr, *norm = nullptr, *hnorm = nullptr;
     double *hnorm_dev = nullptr;   // device address of the pinned hnorm
+    unsigned long long seq = 0;    // launches of k_sum_parts so far
     int nparts = 0;
     std::vector<void *> allocs;
 };
@@ -743,6 +919,19 @@ int copy_in(void *dst, const void *src, size_t bytes, hipStream_t st, const char
                           "hipMemcpyAsync(in)");
 }
 
+// Whether a colour of cnt cells is launched with one wave per face.  Solves to
+// 1e-10 on two colours (four: "4c"), thread per cell -> wave per face, us:
+//   FP64:  9K hexes 326 -> 217, 262K 1094 -> 958, 913K 4344 -> 3619, 2.2M
+//     12172 -> 10884; 197K tets 854 -> 736, 1M 3774 -> 3704 (4c 5406 -> 4632);
+//     2.2M 9141 -> 10177 (4c 12263 -> 12359), 5.3M 27494 -> 30107
+//   mixed: 9K hexes 332 -> 266, 913K 2194 -> 2062; 197K tets 701 -> 615, 1M
+//     2432 -> 2415 (4c 3621 -> 3145); 2.2M 5400 -> 5799, 5.3M 14479 -> 17480
+// A thread per cell of a hex keeps six faces' loads (256 VGPRs, one wave per
+// SIMD); large colours of tets are ahead with all of a cell's loads in one
+// wave, as in the sweep kernels of the legacy API.
+constexpr int kWfTets = 600000;
+inline bool wave_per_face(int F, int cnt) { return F == 6 || cnt <= kWfTets; }
+
 // lower (with residual) over all colours, norm of s to *norm.  pre0: the
 // previous pass's upper launch formed the first colour's residual, block
 // partials and dstar (k_upper_upd_res), so the pass starts at the second
@@ -756,15 +945,19 @@ int lower_pass(ucfd_lusgs_solver *s, hipStream_t st, bool with_res, const T *qb,
     for (int c = 0; c < s->nc; ++c) {
         const int n0 = s->off[c], cnt = s->off[c + 1] - n0;
         if (cnt <= 0) continue;
-        const dim3 g((cnt + kSB - 1)/kSB);
+        const bool wf = wave_per_face(s->F, cnt);
+        const dim3 g((cnt + (wf ? kWF : kSB) - 1)/(wf ? kWF : kSB));
         if (c == 0 && pre0) {
             pofs += (int)g.x;
             continue;
         }
         const bool last = s->nc > 1 && c == s->nc - 1;
-#define LR(FC, RES, LAST) hipLaunchKernelGGL((k_lower_res<T, FC, RES, LAST>), g, dim3(kSB), 0, st, \
-                                             n0, cnt, s->N, s->nei, geo, diag, qb, rhs, e, dstar, \
-                                             s->part, pofs, delta)
+#define LRK(K, B) hipLaunchKernelGGL(K, g, dim3(B), 0, st, n0, cnt, s->N, s->nei, geo, diag, qb, \
+                                     rhs, e, dstar, s->part, pofs, delta)
+// hexes always take the wave-per-face form
+#define LR(FC, RES, LAST) do { \
+        if (FC == 6 || wf) LRK((k_lower_res_wf<T, FC, RES, LAST>), 64*FC); \
+        else if constexpr (FC == 4) LRK((k_lower_res<T, 4, RES, LAST>), kSB); } while (0)
         if (s->F == 4) {
             if (last) { if (with_res) LR(4, true, true); else LR(4, false, true); }
             else      { if (with_res) LR(4, true, false); else LR(4, false, false); }
@@ -773,10 +966,11 @@ int lower_pass(ucfd_lusgs_solver *s, hipStream_t st, bool with_res, const T *qb,
             else      { if (with_res) LR(6, true, false); else LR(6, false, false); }
         }
 #undef LR
+#undef LRK
         pofs += (int)g.x;
     }
     hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(1024), 0, st, s->part, pofs, s->norm,
-                       s->hnorm_dev);
+                       s->hnorm_dev, ++s->seq);
     return hipGetLastError() == hipSuccess ? UCFD_OK : UCFD_ERR_HIP;
 }
 
@@ -793,22 +987,23 @@ int upper_pass(ucfd_lusgs_solver *s, hipStream_t st, const T *qb, T *dstar, T *d
         const int n0 = s->off[c], cnt = s->off[c + 1] - n0;
         if (cnt <= 0) continue;
         if (s->nc > 1 && c == s->nc - 1) continue;
-        const dim3 g((cnt + kSB - 1)/kSB);
-        if (c == 0 && rhs) {
-            if (s->F == 4)
-                hipLaunchKernelGGL((k_upper_upd_res<T, 4>), g, dim3(kSB), 0, st, cnt, s->N, s->nei,
-                                   geo, diag, qb, dstar, delta, e, rhs, s->part, 0);
-            else
-                hipLaunchKernelGGL((k_upper_upd_res<T, 6>), g, dim3(kSB), 0, st, cnt, s->N, s->nei,
-                                   geo, diag, qb, dstar, delta, e, rhs, s->part, 0);
-            continue;
+        const bool wf = wave_per_face(s->F, cnt), res = c == 0 && rhs;
+        const dim3 g((cnt + (wf ? kWF : kSB) - 1)/(wf ? kWF : kSB));
+#define UPW(FC, RES) hipLaunchKernelGGL((k_upper_wf<T, FC, RES>), g, dim3(64*FC), 0, st, n0, cnt, \
+                                        s->N, s->nei, geo, diag, qb, dstar, delta, e, rhs, \
+                                        s->part, 0)
+        if (s->F == 6) {
+            if (res) UPW(6, true); else UPW(6, false);
+        } else if (wf) {
+            if (res) UPW(4, true); else UPW(4, false);
+        } else if (res) {
+            hipLaunchKernelGGL((k_upper_upd_res<T, 4>), g, dim3(kSB), 0, st, cnt, s->N, s->nei,
+                               geo, diag, qb, dstar, delta, e, rhs, s->part, 0);
+        } else {
+            hipLaunchKernelGGL((k_upper_upd<T, 4>), g, dim3(kSB), 0, st, n0, cnt, s->N, s->nei,
+                               geo, diag, qb, dstar, delta, e);
         }
-        if (s->F == 4)
-            hipLaunchKernelGGL((k_upper_upd<T, 4>), g, dim3(kSB), 0, st, n0, cnt, s->N, s->nei, geo,
-                               diag, qb, dstar, delta, e);
-        else
-            hipLaunchKernelGGL((k_upper_upd<T, 6>), g, dim3(kSB), 0, st, n0, cnt, s->N, s->nei, geo,
-                               diag, qb, dstar, delta, e);
+#undef UPW
     }
     return hipGetLastError() == hipSuccess ? UCFD_OK : UCFD_ERR_HIP;
 }
@@ -841,16 +1036,30 @@ int residual64(ucfd_lusgs_solver *s, hipStream_t st, const double *b, const doub
         pofs += (int)g.x;
     }
     hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(1024), 0, st, s->part, pofs, s->norm,
-                       s->hnorm_dev);
+                       s->hnorm_dev, ++s->seq);
     return hipGetLastError() == hipSuccess ? UCFD_OK : UCFD_ERR_HIP;
 }
 
+// The norm of the last k_sum_parts launch, as soon as that kernel has written
+// it: the upper launches enqueued behind it run while the host decides and
+// enqueues the next pass.  The poll ends with the value, or with the stream
+// (finished without it, or failed).
 int read_norm(ucfd_lusgs_solver *s, hipStream_t st, double *out, const char *fn)
 {
-    // the last k_sum_parts wrote the norm into the pinned hnorm
-    int rc = ucfd_check_hip(hipStreamSynchronize(st), fn, "hipStreamSynchronize");
-    *out = sqrt(*s->hnorm);
-    return rc;
+    const unsigned long long *word = (const unsigned long long *)s->hnorm + 1;
+    for (;;) {
+        for (int k = 0; k < 4096; ++k) {
+            if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == s->seq) {
+                *out = sqrt(*(volatile double *)s->hnorm);
+                return UCFD_OK;
+            }
+            __builtin_ia32_pause();
+        }
+        const hipError_t q = hipStreamQuery(st);
+        if (q == hipErrorNotReady) continue;
+        if (q == hipSuccess && __atomic_load_n(word, __ATOMIC_ACQUIRE) == s->seq) continue;
+        return ucfd_check_hip(q == hipSuccess ? hipErrorUnknown : q, fn, "norm of the residual");
+    }
 }
 
 }  // namespace
@@ -898,7 +1107,8 @@ UCFD_API int ucfd_lusgs_solver_create(ucfd_lusgs_solver **out, int neles, int nf
     s->off.assign(color_off, color_off + ncolors + 1);
     int maxparts = 0;
     for (int c = 0; c < ncolors; ++c) maxparts += (s->off[c + 1] - s->off[c] + kSB - 1)/kSB;
-    s->nparts = std::max(maxparts, (neles + kSB - 1)/kSB) + 8;
+    // one partial per 64 or per kSB cells
+    s->nparts = std::max(maxparts, (neles + kWF - 1)/kWF + ncolors) + 8;
     const hipStream_t st = ucfd_stream();
     double *tfnv = nullptr, *tvfn = nullptr, *tsp = nullptr, *tdt = nullptr, *tq = nullptr;
     if ((rc = dalloc(s, &s->nei, F*N, fn)) || (rc = dalloc(s, &s->g64, F*N, fn)) ||
@@ -924,6 +1134,7 @@ UCFD_API int ucfd_lusgs_solver_create(ucfd_lusgs_solver **out, int neles, int nf
         delete s;
         return rc;
     }
+    memset(s->hnorm, 0, 64);    // no sequence number of an earlier solver's memory
     rc = copy_in(s->nei, hn.data(), F*N*4, st, fn);
     if (!rc) rc = copy_in(tfnv, fnorm_vol, F*N*8, st, fn);
     if (!rc) rc = copy_in(tvfn, vec_fnorm, 3*F*N*8, st, fn);
@@ -1246,7 +1457,7 @@ UCFD_API int ucfd_lusgs_residual_noalloc(int neles, int nface, int ncolors, cons
         pofs += (int)g.x;
     }
     hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(1024), 0, st, S->part, pofs, S->norm,
-                       (double *)nullptr);
+                       (double *)nullptr, 0ull);
     if ((rc = ucfd_check_hip(hipGetLastError(), fn, "kernel launch"))) return rc;
     double nrm2 = 0.0;
     int f = 0;
