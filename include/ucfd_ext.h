@@ -171,7 +171,7 @@ int ucfd_lusgs_solve(ucfd_lusgs_solver *solver, int mode, const double *b, doubl
  * colour's launch also does that colour's upper step and update), ms[1]
  * upper sweep with update of the other colours (FP64; the first colour's
  * launch also forms that colour's residual and lower step for the next
- * pass), ms[2] / ms[3] the same
+ * pass, and the first launch sums the pass's norm), ms[2] / ms[3] the same
  * kernels in FP32 (the inner kernels of UCFD_SOLVE_MIXED), ms[4] the FP64
  * residual and its norm.  b is a device array [5][neles]; the solver's work
  * arrays are overwritten. */

@@ -200,6 +200,63 @@ __device__ __forceinline__ void block_sum(double v, double *part, int slot)
     }
 }
 
+// Sum of n partials by one workgroup of BS threads in a fixed order (thread t
+// sums t, t + BS, ... with eight loads in flight, then a fixed tree), so the
+// norm and every convergence decision are reproducible run to run; valid in
+// thread 0.
+template <int BS>
+__device__ __forceinline__ double sum_parts(const double *part, int n)
+{
+    constexpr int U = 8;
+    __shared__ double red[BS/64];
+    double s = 0.0;
+    for (int j0 = threadIdx.x; j0 < n; j0 += BS*U) {
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int j = j0 + u*BS;
+            v[u] = j < n ? part[j] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) s += v[u];
+    }
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (threadIdx.x % 64 == 0) red[threadIdx.x/64] = s;
+    __syncthreads();
+    double t = 0.0;
+    if (threadIdx.x == 0)
+        for (int w = 0; w < BS/64; ++w) t += red[w];
+    return t;
+}
+
+// The norm of a pass: partials of the launches before this one, and where the
+// result goes: pinned host memory, the value and then the sequence number that
+// the host polls while the launches behind run (no copy, no wait for the
+// stream).  n = 0: nothing to sum.
+struct NormJob {
+    const double *part;
+    int n;
+    double *hout;
+    unsigned long long seq;
+};
+
+__device__ __forceinline__ void publish(const NormJob &job, double t)
+{
+    __hip_atomic_store(job.hout, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store((unsigned long long *)job.hout + 1, job.seq, __ATOMIC_RELEASE,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The first upper launch of a pass sums the lower launches' partials in its
+// first workgroup: a launch of its own took 4.7 us of a 67 us FP32 pass (1M
+// tets), 2.5 us and its gap of a 21 us FP64 one (9K hexes).
+template <int BS> __device__ __forceinline__ void first_block_norm(const NormJob &job)
+{
+    if (blockIdx.x != 0 || job.n == 0) return;
+    const double t = sum_parts<BS>(job.part, job.n);
+    if (threadIdx.x == 0) publish(job, t);
+}
+
 // Every kernel below issues all loads a thread needs (its own rows, the face
 // records and the neighbour states of every face it uses) before the first
 // arithmetic, so the gathers of all faces are in flight together.
@@ -307,8 +364,9 @@ template <typename T, int FC>
 __global__ __launch_bounds__(kSB) void k_upper_upd(
     int n0, int cnt, int N, const int *__restrict__ nei, const Face4<T> *__restrict__ geo,
     const T *__restrict__ diag, const T *__restrict__ qb, const T *__restrict__ dstar,
-    T *delta, T *e)
+    T *delta, T *e, NormJob job)
 {
+    first_block_norm<kSB>(job);
     const int t = xcd_remap()*kSB + threadIdx.x;
     if (t >= cnt) return;
     const int i = n0 + t, ne = n0 + cnt;
@@ -370,8 +428,9 @@ template <typename T, int FC>
 __global__ __launch_bounds__(kSB) void k_upper_upd_res(
     int cnt, int N, const int *__restrict__ nei, const Face4<T> *__restrict__ geo,
     const T *__restrict__ diag, const T *__restrict__ qb, T *dstar, T *delta, T *e,
-    const T *__restrict__ rhs, double *part, int pofs)
+    const T *__restrict__ rhs, double *part, int pofs, NormJob job)
 {
+    first_block_norm<kSB>(job);
     const int b = xcd_remap();
     const int t = b*kSB + threadIdx.x;
     double ss = 0.0;
@@ -550,10 +609,11 @@ template <typename T, int FC, bool RES>
 __global__ __launch_bounds__(64*FC) void k_upper_wf(
     int n0, int cnt, int N, const int *__restrict__ nei, const Face4<T> *__restrict__ geo,
     const T *__restrict__ diag, const T *__restrict__ qb, T *dstar, T *delta, T *e,
-    const T *__restrict__ rhs, double *part, int pofs)
+    const T *__restrict__ rhs, double *part, int pofs, NormJob job)
 {
     constexpr int KW = (NV + FC - 1)/FC;
     __shared__ T sup[FC][NV][64], sres[RES ? FC : 1][NV][64];
+    first_block_norm<64*FC>(job);
     const int lane = threadIdx.x & 63, f = threadIdx.x >> 6;
     const int b = xcd_remap(), t = b*64 + lane, i = n0 + t, ne = n0 + cnt;
     const bool act = t < cnt;
@@ -685,40 +745,14 @@ __global__ __launch_bounds__(kSB) void k_residual64(
     block_sum<kSB>(ss, part, pofs + blk);
 }
 
-// Sum of the block partials in a fixed order (thread t sums t, t+1024, ...
-// with eight loads in flight, then a fixed tree), so the norm and every
-// convergence decision are reproducible run to run.
-// The result goes to out (device) and to hout (pinned host memory: the value,
-// then the launch's sequence number, which the host polls while the launches
-// behind this one run: no copy kernel and no wait for the stream).
-__global__ __launch_bounds__(1024) void k_sum_parts(const double *part, int n, double *out,
-                                                    double *hout, unsigned long long seq)
+// The residual's norm, in a launch of its own: to out (device) and, if given,
+// to the host.
+__global__ __launch_bounds__(1024) void k_sum_parts(NormJob job, double *out)
 {
-    constexpr int U = 8;
-    __shared__ double red[16];
-    double s = 0.0;
-    for (int j0 = threadIdx.x; j0 < n; j0 += 1024*U) {
-        double v[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int j = j0 + u*1024;
-            v[u] = j < n ? part[j] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) s += v[u];
-    }
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if (threadIdx.x % 64 == 0) red[threadIdx.x/64] = s;
-    __syncthreads();
+    const double t = sum_parts<1024>(job.part, job.n);
     if (threadIdx.x == 0) {
-        double t = 0.0;
-        for (int w = 0; w < 16; ++w) t += red[w];
         *out = t;
-        if (hout) {
-            __hip_atomic_store(hout, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            __hip_atomic_store((unsigned long long *)hout + 1, seq, __ATOMIC_RELEASE,
-                               __HIP_MEMORY_SCOPE_SYSTEM);
-        }
+        if (job.hout) publish(job, t);
     }
 }
 
@@ -890,9 +924,12 @@ struct ucfd_lusgs_solver {
            *delta64 = nullptr;
     float *d32 = nullptr, *qb32 = nullptr, *r32 = nullptr, *e32 = nullptr, *dstar32 = nullptr,
           *delta32 = nullptr;
-    double *part = nullptr, *norm = nullptr, *hnorm = nullptr;
+    // block partials of the norm: the pass's (parts[cur]) and, from its upper
+    // launch on, the next pass's (parts[cur ^ 1])
+    double *parts[2] = {nullptr, nullptr}, *norm = nullptr, *hnorm = nullptr;
+    int cur = 0, np = 0;           // np: partials of the pass
     double *hnorm_dev = nullptr;   // device address of the pinned hnorm
-    unsigned long long seq = 0;    // launches of k_sum_parts so far
+    unsigned long long seq = 0;    // norms requested so far
     int nparts = 0;
     std::vector<void *> allocs;
 };
@@ -932,7 +969,7 @@ int copy_in(void *dst, const void *src, size_t bytes, hipStream_t st, const char
 constexpr int kWfTets = 600000;
 inline bool wave_per_face(int F, int cnt) { return F == 6 || cnt <= kWfTets; }
 
-// lower (with residual) over all colours, norm of s to *norm.  pre0: the
+// lower (with residual) over all colours; upper_pass sums the norm of s.  pre0: the
 // previous pass's upper launch formed the first colour's residual, block
 // partials and dstar (k_upper_upd_res), so the pass starts at the second
 // colour.  With more than one colour the last colour's launch also does that
@@ -953,7 +990,7 @@ int lower_pass(ucfd_lusgs_solver *s, hipStream_t st, bool with_res, const T *qb,
         }
         const bool last = s->nc > 1 && c == s->nc - 1;
 #define LRK(K, B) hipLaunchKernelGGL(K, g, dim3(B), 0, st, n0, cnt, s->N, s->nei, geo, diag, qb, \
-                                     rhs, e, dstar, s->part, pofs, delta)
+                                     rhs, e, dstar, s->parts[s->cur], pofs, delta)
 // hexes always take the wave-per-face form
 #define LR(FC, RES, LAST) do { \
         if (FC == 6 || wf) LRK((k_lower_res_wf<T, FC, RES, LAST>), 64*FC); \
@@ -969,42 +1006,50 @@ int lower_pass(ucfd_lusgs_solver *s, hipStream_t st, bool with_res, const T *qb,
 #undef LRK
         pofs += (int)g.x;
     }
-    hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(1024), 0, st, s->part, pofs, s->norm,
-                       s->hnorm_dev, ++s->seq);
+    s->np = pofs;
     return hipGetLastError() == hipSuccess ? UCFD_OK : UCFD_ERR_HIP;
 }
 
 // upper sweep and update over all colours (last colour first).  rhs given:
 // the first colour's launch also forms the next pass's residual of its
-// cells, their block partials (at the start of part) and their dstar for
-// the next pass.  The last colour's upper step was done by the lower pass
+// cells, their block partials (at the start of the other buffer) and their
+// dstar for the next pass.  The first launch sums the pass's norm.  The last colour's upper step was done by the lower pass
 // (more than one colour).
 template <typename T>
 int upper_pass(ucfd_lusgs_solver *s, hipStream_t st, const T *qb, T *dstar, T *delta, T *e,
                const Face4<T> *geo, const T *diag, const T *rhs = nullptr)
 {
+    NormJob job{s->parts[s->cur], s->np, s->hnorm_dev, ++s->seq};
+    double *next = s->parts[s->cur ^ 1];
+    bool summed = false;
     for (int c = s->nc - 1; c >= 0; --c) {
         const int n0 = s->off[c], cnt = s->off[c + 1] - n0;
         if (cnt <= 0) continue;
         if (s->nc > 1 && c == s->nc - 1) continue;
+        if (summed) job.n = 0;
+        summed = true;
         const bool wf = wave_per_face(s->F, cnt), res = c == 0 && rhs;
         const dim3 g((cnt + (wf ? kWF : kSB) - 1)/(wf ? kWF : kSB));
 #define UPW(FC, RES) hipLaunchKernelGGL((k_upper_wf<T, FC, RES>), g, dim3(64*FC), 0, st, n0, cnt, \
                                         s->N, s->nei, geo, diag, qb, dstar, delta, e, rhs, \
-                                        s->part, 0)
+                                        next, 0, job)
         if (s->F == 6) {
             if (res) UPW(6, true); else UPW(6, false);
         } else if (wf) {
             if (res) UPW(4, true); else UPW(4, false);
         } else if (res) {
             hipLaunchKernelGGL((k_upper_upd_res<T, 4>), g, dim3(kSB), 0, st, cnt, s->N, s->nei,
-                               geo, diag, qb, dstar, delta, e, rhs, s->part, 0);
+                               geo, diag, qb, dstar, delta, e, rhs, next, 0, job);
         } else {
             hipLaunchKernelGGL((k_upper_upd<T, 4>), g, dim3(kSB), 0, st, n0, cnt, s->N, s->nei,
-                               geo, diag, qb, dstar, delta, e);
+                               geo, diag, qb, dstar, delta, e, job);
         }
 #undef UPW
     }
+    // every cell in the last colour: no upper launch to do it
+    if (!summed)
+        hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(1024), 0, st, job, s->norm);
+    s->cur ^= 1;
     return hipGetLastError() == hipSuccess ? UCFD_OK : UCFD_ERR_HIP;
 }
 
@@ -1020,7 +1065,7 @@ int residual64(ucfd_lusgs_solver *s, hipStream_t st, const double *b, const doub
         const dim3 g((cnt + kSB - 1)/kSB);
 #define R(FC, O, Z, S) hipLaunchKernelGGL((k_residual64<FC, O, Z, S>), g, dim3(kSB), 0, st, n0, \
                                           cnt, s->N, s->nei, s->g64, s->d64, s->q64, b, dq, r, \
-                                          s->r32, s->qb32, s->part, pofs)
+                                          s->r32, s->qb32, s->parts[s->cur], pofs)
         if (s->F == 4) {
             if (out32 && zero_dq) R(4, true, true, true);
             else if (out32) R(4, true, false, true);
@@ -1035,13 +1080,13 @@ int residual64(ucfd_lusgs_solver *s, hipStream_t st, const double *b, const doub
 #undef R
         pofs += (int)g.x;
     }
-    hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(1024), 0, st, s->part, pofs, s->norm,
-                       s->hnorm_dev, ++s->seq);
+    hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(1024), 0, st,
+                       NormJob{s->parts[s->cur], pofs, s->hnorm_dev, ++s->seq}, s->norm);
     return hipGetLastError() == hipSuccess ? UCFD_OK : UCFD_ERR_HIP;
 }
 
-// The norm of the last k_sum_parts launch, as soon as that kernel has written
-// it: the upper launches enqueued behind it run while the host decides and
+// The norm last requested, as soon as the kernel that sums it has written it:
+// the rest of that launch and those behind it run while the host decides and
 // enqueues the next pass.  The poll ends with the value, or with the stream
 // (finished without it, or failed).
 int read_norm(ucfd_lusgs_solver *s, hipStream_t st, double *out, const char *fn)
@@ -1118,7 +1163,8 @@ UCFD_API int ucfd_lusgs_solver_create(ucfd_lusgs_solver **out, int neles, int nf
         (rc = dalloc(s, &s->delta64, NV*N, fn)) || (rc = dalloc(s, &s->qb32, NV*N, fn)) ||
         (rc = dalloc(s, &s->r32, NV*N, fn)) || (rc = dalloc(s, &s->e32, NV*N, fn)) ||
         (rc = dalloc(s, &s->dstar32, NV*N, fn)) || (rc = dalloc(s, &s->delta32, NV*N, fn)) ||
-        (rc = dalloc(s, &s->part, (size_t)s->nparts, fn)) || (rc = dalloc(s, &s->norm, 8, fn)) ||
+        (rc = dalloc(s, &s->parts[0], (size_t)s->nparts, fn)) ||
+        (rc = dalloc(s, &s->parts[1], (size_t)s->nparts, fn)) || (rc = dalloc(s, &s->norm, 8, fn)) ||
         (rc = dalloc(s, &tfnv, F*N, fn)) || (rc = dalloc(s, &tvfn, 3*F*N, fn)) ||
         (rc = dalloc(s, &tsp, F*N, fn)) || (rc = dalloc(s, &tdt, N, fn)) ||
         (rc = dalloc(s, &tq, NV*N, fn))) {
@@ -1292,7 +1338,8 @@ UCFD_API int ucfd_lusgs_solve(ucfd_lusgs_solver *s, int mode, const double *b, d
 // pass each (every colour), averaged over reps, on the library stream:
 // ms[0] lower sweep with residual (FP64; the first colour's residual comes
 // from the previous pass, as in the solve), ms[1] upper sweep with update
-// and the first colour's next residual (FP64), ms[2] / ms[3] the same in
+// and the first colour's next residual, with the sum of the pass's norm (FP64),
+// ms[2] / ms[3] the same in
 // FP32 (the inner kernels of the mixed form), ms[4] the FP64 residual (all
 // colours) and its norm.  The state is a
 // first outer step (dq = 0 with right-hand side b); the solver's work arrays
@@ -1456,8 +1503,8 @@ UCFD_API int ucfd_lusgs_residual_noalloc(int neles, int nface, int ncolors, cons
                                flag);
         pofs += (int)g.x;
     }
-    hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(1024), 0, st, S->part, pofs, S->norm,
-                       (double *)nullptr, 0ull);
+    hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(1024), 0, st,
+                       NormJob{S->part, pofs, nullptr, 0ull}, S->norm);
     if ((rc = ucfd_check_hip(hipGetLastError(), fn, "kernel launch"))) return rc;
     double nrm2 = 0.0;
     int f = 0;
