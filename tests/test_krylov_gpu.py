@@ -501,3 +501,19 @@ def test_prepare_again_with_new_values(K):
     f = O.ilu_prepare(A2, "pbilu")
     assert np.array_equal(Di.values.cpu().numpy(), f.reshape(A.values.shape))
     assert np.array_equal(b.cpu().numpy(), O.ilu_apply(A2, f, x, "pbilu", off))
+
+
+@pytest.mark.parametrize("dims", [(3, 17, 257), (4, 29, 113)])
+@pytest.mark.parametrize("kind", ["gmres", "bicgstab"])
+def test_solves_on_both_sides_of_the_reduction_choice(K, dims, kind):
+    """65535 and 65540 unknowns: 256 partials a row (summed by the kernel that
+    uses them) and 257 (summed to one value first)."""
+    mesh = M.hex_mesh(*dims, seed=13)
+    A = M.block_system(mesh, M.flow_fields(mesh, seed=13), blk=5, seed=13)
+    b = M.normal_fill(A.bn * 5, 13)
+    x = np.zeros_like(b)
+    s = K.Solver(kind, A.bn * 5, 200, 1e-10, m=30, right=True)
+    status, _, _ = s.solve(K.Precon.from_bsr(A), K.SpMat.from_bsr(A), x, b)
+    assert status == K.CONVERGED
+    r = b - A.to_scipy() @ x
+    assert np.linalg.norm(r) <= 2e-10 * np.linalg.norm(b)

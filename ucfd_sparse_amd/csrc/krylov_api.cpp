@@ -63,7 +63,9 @@ struct _Precon {
 namespace {
 
 constexpr int HCAP = 64;      // Krylov dimension limit of the device reductions
-constexpr int DB_H = 0, DB_H2 = 64, DB_NSQ = 128, DB_Y = 136, DB_N = 208;
+// scalars on their way to the host: h, h2 (or the BiCGSTAB dots), a norm, and the
+// sequence word of the last posted group
+constexpr int DB_H = 0, DB_H2 = 64, DB_NSQ = 128, DB_SEQ = 136, DB_N = 144;
 
 }  // namespace
 
@@ -80,9 +82,10 @@ struct _Solver {
     double *V, *w, *r, *z;   // GMRES
     double *Z;               // GMRES, right mode: the preconditioned basis M^-1 v_j
     double *rt, *p, *pt, *v, *s, *shat, *t;   // BiCGSTAB (r shared)
-    double *part;            // reduction partials
+    double *part, *part2;    // reduction partials (two sets: a kernel may read one and write the other)
     double *dbuf;            // device scalars
-    double *hbuf;            // pinned host scalars
+    double *hbuf, *hbuf_dev; // pinned host scalars and their device address
+    unsigned long long seq;  // groups of scalars posted so far
 };
 
 namespace {
@@ -390,12 +393,32 @@ ucfd_status_t set_block(Precon *precon, UCFDInt bn, UCFDInt block, PreconType ty
 
 // --------------------------------------------------------------- solvers
 
-int d2h(Solver S, int off, int count, hipStream_t s, const char *fn)
+// Where a kernel posts scalars; last: with the next sequence number
+KryPost post_at(Solver S, int off, bool last)
 {
-    int rc = hip(hipMemcpyAsync(S->hbuf + off, S->dbuf + off, sizeof(double)*count,
-                                hipMemcpyDeviceToHost, s), fn, "hipMemcpyAsync(scalars)");
-    if (rc) return rc;
-    return hip(hipStreamSynchronize(s), fn, "hipStreamSynchronize");
+    KryPost h;
+    h.out = S->hbuf_dev + off;
+    if (last) {
+        h.word = (unsigned long long *)(S->hbuf_dev + DB_SEQ);
+        h.seq = ++S->seq;
+    }
+    return h;
+}
+
+// The last posted group is in hbuf
+int await(Solver S, hipStream_t s, const char *fn)
+{
+    return ucfd_poll((const unsigned long long *)(S->hbuf + DB_SEQ), S->seq, s, fn,
+                     "scalars of the iteration");
+}
+
+// x.y on the host
+int dot_host(Solver S, hipStream_t s, const double *x, const double *y, double *out, const char *fn)
+{
+    int rc = kry_dot(s, S->n, x, y, S->part, S->dbuf, post_at(S, DB_NSQ, true));
+    if (!rc) rc = await(S, s, fn);
+    *out = S->hbuf[DB_NSQ];
+    return rc;
 }
 
 void record(Solver S, int iter, double res)
@@ -415,38 +438,31 @@ int gmres(Solver S, Precon pc, SpMat A, const MatDev &ma, const PcDev &mp, doubl
     const double tol = S->tol, haptol = S->haptol;
     const int64_t N = n;
     std::vector<double> H((size_t)ld*m, 0.0), y(ld, 0.0), cs(ld, 0.0), sn(ld, 0.0);
-    double *V = S->V, *w = S->w, *r = S->r, *part = S->part, *db = S->dbuf;
-    double *hb = S->hbuf;
+    double *V = S->V, *w = S->w, *r = S->r, *part = S->part, *part2 = S->part2;
+    const double *hb = S->hbuf;
     int rc, iter = 0, k = 0;
-    double abeta = 0.0, tolv = tol;
+    double abeta = 0.0, tolv = tol, sq = 0.0;
     if (S->right) {
-        if ((rc = kry_dot(s, N, b, b, part, db + DB_NSQ)) || (rc = d2h(S, DB_NSQ, 1, s, fn)))
-            return rc;
-        tolv = tol*sqrt(hb[DB_NSQ]);
+        if ((rc = dot_host(S, s, b, b, &sq, fn))) return rc;
+        tolv = tol*sqrt(sq);
     }
     while (iter < S->maxiter) {
         if ((rc = kry_copy(s, N, b, r)) || (rc = spmv(s, A, ma, -1.0, x, 1.0, r))) return rc;
-        if ((rc = kry_dot(s, N, r, r, part, db + DB_NSQ)) || (rc = d2h(S, DB_NSQ, 1, s, fn)))
-            return rc;
-        abeta = sqrt(hb[DB_NSQ]);
+        if ((rc = dot_host(S, s, r, r, &sq, fn))) return rc;
+        abeta = sqrt(sq);
         record(S, iter, abeta);
         if (abeta <= tolv) {
             S->stat = CONVERGED;
             break;
         }
         double beta = abeta;
-        int nsq_slot = DB_NSQ;
         if (!S->right) {
-            if ((rc = pc_apply(s, pc, mp, r))) return rc;
-            nsq_slot = DB_NSQ + 1;
-            if ((rc = kry_dot(s, N, r, r, part, db + nsq_slot)) || (rc = d2h(S, nsq_slot, 1, s, fn)))
-                return rc;
-            beta = sqrt(hb[nsq_slot]);
+            if ((rc = pc_apply(s, pc, mp, r)) || (rc = dot_host(S, s, r, r, &sq, fn))) return rc;
+            beta = sqrt(sq);
         }
         y[0] = beta;
         // right mode: z_0 starts as a copy of v_0 (M^-1 is applied in place)
-        if ((rc = kry_scale_by_inv_sqrt(s, N, r, db + nsq_slot, V, S->right ? S->Z : nullptr)))
-            return rc;
+        if ((rc = kry_scale_by_inv_sqrt(s, N, r, part, V, S->right ? S->Z : nullptr))) return rc;
         k = 0;
         bool happy = false;
         for (int j = 0; j < m; ++j) {
@@ -464,14 +480,18 @@ int gmres(Solver S, Precon pc, SpMat A, const MatDev &ma, const PcDev &mp, doubl
                     return rc;
             }
             // CGS2 (gmres.c:20-29); the first update and the second projection
-            // share one pass over V
-            if ((rc = kry_gemvt(s, N, kk, V, N, w, part, db + DB_H)) ||
-                (rc = kry_gemv_gemvt(s, N, kk, V, N, -1.0, db + DB_H, w, part, db + DB_H2)) ||
-                (rc = kry_gemv(s, N, kk, V, N, -1.0, db + DB_H2, w, part, db + DB_NSQ)) ||
-                (rc = kry_scale_by_inv_sqrt(s, N, w, db + DB_NSQ, V + (size_t)(j + 1)*n,
+            // share one pass over V.  Each kernel sums the partials of the one
+            // before it and posts them; the host reads all three while the
+            // normalisation runs.
+            if ((rc = kry_gemvt(s, N, kk, V, N, w, part)) ||
+                (rc = kry_gemv_gemvt(s, N, kk, V, N, -1.0, part, w, part2,
+                                     post_at(S, DB_H, false))) ||
+                (rc = kry_gemv(s, N, kk, V, N, -1.0, part2, w, part, post_at(S, DB_H2, false))) ||
+                (rc = kry_scale_by_inv_sqrt(s, N, w, part, V + (size_t)(j + 1)*n,
                                             S->right && j + 1 < m ? S->Z + (size_t)(j + 1)*n
-                                                                  : nullptr)) ||
-                (rc = d2h(S, 0, DB_NSQ + 1, s, fn)))
+                                                                  : nullptr,
+                                            post_at(S, DB_NSQ, true))) ||
+                (rc = await(S, s, fn)))
                 return rc;
             double *Hcol = H.data() + (size_t)j*ld;
             for (int i = 0; i < kk; ++i) Hcol[i] = hb[DB_H + i] + 1.0*hb[DB_H2 + i];
@@ -506,17 +526,9 @@ int gmres(Solver S, Precon pc, SpMat A, const MatDev &ma, const PcDev &mp, doubl
             y[i] = sum/H[i + (size_t)i*ld];
         }
         if (k > 0) {
-            memcpy(hb + DB_Y, y.data(), sizeof(double)*k);
-            if ((rc = hip(hipMemcpyAsync(db + DB_Y, hb + DB_Y, sizeof(double)*k,
-                                         hipMemcpyHostToDevice, s), fn, "hipMemcpyAsync(y)")))
-                return rc;
-            if (S->right) {
-                if ((rc = kry_gemv(s, N, k, S->Z, N, 1.0, db + DB_Y, x, part, nullptr)))
-                    return rc;
-            } else if ((rc = kry_gemv(s, N, k, V, N, 1.0, db + DB_Y, x, part, nullptr))) {
-                return rc;
-            }
-            // the host buffer of y is rewritten only after the next synchronisation
+            KryCoef c;
+            memcpy(c.v, y.data(), sizeof(double)*k);
+            if ((rc = kry_gemv_y(s, N, k, S->right ? S->Z : V, N, c, x))) return rc;
         }
         if (happy) S->stat = HAPPYBREAKDOWN;
         iter++;
@@ -533,19 +545,17 @@ int bicgstab(Solver S, Precon pc, SpMat A, const MatDev &ma, const PcDev &mp, do
 {
     const int64_t N = S->n;
     double *r = S->r, *rt = S->rt, *p = S->p, *pt = S->pt, *v = S->v, *sv = S->s;
-    double *shat = S->shat, *t = S->t, *part = S->part, *db = S->dbuf, *hb = S->hbuf;
+    double *shat = S->shat, *t = S->t, *part = S->part, *part2 = S->part2;
+    const double *hb = S->hbuf;
     int rc, iter = 0;
-    double rho, rhoprev, alpha, beta, omega, resnorm = 0.0, tolv = S->tol;
+    double rho, rhoprev, alpha, beta, omega, resnorm = 0.0, tolv = S->tol, sq = 0.0;
     if (S->right) {
-        if ((rc = kry_dot(s, N, b, b, part, db + DB_NSQ)) || (rc = d2h(S, DB_NSQ, 1, s, fn)))
-            return rc;
-        tolv = S->tol*sqrt(hb[DB_NSQ]);
+        if ((rc = dot_host(S, s, b, b, &sq, fn))) return rc;
+        tolv = S->tol*sqrt(sq);
     }
     if ((rc = kry_copy(s, N, b, r)) || (rc = spmv(s, A, ma, -1.0, x, 1.0, r)) ||
-        (rc = kry_copy(s, N, r, rt)) || (rc = kry_dot(s, N, rt, r, part, db + DB_NSQ)) ||
-        (rc = d2h(S, DB_NSQ, 1, s, fn)))
+        (rc = kry_copy(s, N, r, rt)) || (rc = dot_host(S, s, rt, r, &rho, fn)))
         return rc;
-    rho = hb[DB_NSQ];
     rhoprev = 1.0;
     alpha = 1.0;
     omega = 1.0;
@@ -560,26 +570,27 @@ int bicgstab(Solver S, Precon pc, SpMat A, const MatDev &ma, const PcDev &mp, do
             beta = (rho/rhoprev)*(alpha/omega);
             if ((rc = kry_bicg_p(s, N, beta, omega, r, v, p, pt))) return rc;
         }
-        // pi = rt.v stays on the device: s = r - (rho/pi) v is formed there, and
-        // pi comes back with the five dots in one copy (one host wait per
-        // iteration).  A pi breakdown then stops before x and r change.
+        // pi = rt.v and the five dots stay on the device, where alpha = rho/pi
+        // and omega are formed for the updates; the last kernel posts them, and
+        // the host, forming the same quotients, decides while it runs.  A pi
+        // breakdown leaves x and r unchanged.
         if ((rc = pc_apply(s, pc, mp, pt)) || (rc = spmv(s, A, ma, 1.0, pt, 0.0, v)) ||
-            (rc = kry_dot(s, N, rt, v, part, db + DB_NSQ)) ||
-            (rc = kry_bicg_s(s, N, rho, db + DB_NSQ, r, v, sv, shat)) ||
+            (rc = kry_dot(s, N, rt, v, part, nullptr)) ||
+            (rc = kry_bicg_s(s, N, rho, part, r, v, sv, shat)) ||
             (rc = pc_apply(s, pc, mp, shat)) || (rc = spmv(s, A, ma, 1.0, shat, 0.0, t)) ||
-            (rc = kry_dot5(s, N, rt, sv, t, part, db + DB_H)) ||
-            (rc = d2h(S, DB_H, DB_NSQ + 1 - DB_H, s, fn)))
+            (rc = kry_dot5(s, N, rt, sv, t, part2)) ||
+            (rc = kry_bicg_xr(s, N, rho, part, part2, pt, shat, sv, t, x, r,
+                              post_at(S, DB_H, true))) ||
+            (rc = await(S, s, fn)))
             return rc;
-        const double pi = hb[DB_NSQ];
+        const double phi = hb[DB_H], rtt = hb[DB_H + 1], ts = hb[DB_H + 2], tt = hb[DB_H + 3],
+                     ss = hb[DB_H + 4], pi = hb[DB_H + 5];
         if (fabs(pi) < 1e-30) {
             S->stat = PIBREAKDOWN;
             break;
         }
         alpha = rho/pi;
-        const double phi = hb[DB_H], rtt = hb[DB_H + 1], ts = hb[DB_H + 2], tt = hb[DB_H + 3],
-                     ss = hb[DB_H + 4];
         omega = ts/tt;
-        if ((rc = kry_bicg_xr(s, N, alpha, pt, omega, shat, sv, t, x, r))) return rc;
         const double rho_new = phi - omega*rtt;
         resnorm = sqrt(fabs(ss - 2.0*omega*ts + omega*omega*tt));
         record(S, iter, resnorm);
@@ -615,14 +626,17 @@ ucfd_status_t solver_create(Solver *solver, SolverType type, UCFDInt n, UCFDInt 
     S->tol = tol;
     S->maxiter = maxiter;
     const size_t nv = strcmp(type, GMRES) == 0 ? (size_t)(m + 1) + 3 : 8;
-    const size_t bytes = sizeof(double)*((size_t)n*nv + (size_t)HCAP*1024 + DB_N);
+    const size_t bytes = sizeof(double)*((size_t)n*nv + 2*(size_t)HCAP*KRY_MAXPART + 8);
     if ((rc = hip(hipMalloc((void **)&S->vec, bytes), fn, "hipMalloc(work vectors)")) ||
         (rc = hip(hipMemset(S->vec, 0, bytes), fn, "hipMemset(work vectors)")) ||
         (rc = hip(hipHostMalloc((void **)&S->hbuf, sizeof(double)*DB_N, hipHostMallocDefault), fn,
-                  "hipHostMalloc(scalars)"))) {
+                  "hipHostMalloc(scalars)")) ||
+        (rc = hip(hipHostGetDevicePointer((void **)&S->hbuf_dev, S->hbuf, 0), fn,
+                  "hipHostGetDevicePointer(scalars)"))) {
         UCFDSolverDestroy(solver);
         return UCFD_FAILED;
     }
+    memset(S->hbuf, 0, sizeof(double)*DB_N);
     double *q = S->vec;
     auto take = [&](size_t cnt) { double *o = q; q += cnt; return o; };
     if (strcmp(type, GMRES) == 0) {
@@ -640,8 +654,9 @@ ucfd_status_t solver_create(Solver *solver, SolverType type, UCFDInt n, UCFDInt 
         S->shat = take(n);
         S->t = take(n);
     }
-    S->part = take((size_t)HCAP*1024);
-    S->dbuf = take(DB_N);
+    S->part = take((size_t)HCAP*KRY_MAXPART);
+    S->part2 = take((size_t)HCAP*KRY_MAXPART);
+    S->dbuf = take(8);
     return UCFD_SUCCESS;
 }
 

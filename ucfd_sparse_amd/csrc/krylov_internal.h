@@ -63,45 +63,66 @@ UCFD_HIDDEN int kry_bsgs_sweep32(hipStream_t s, int upper, int blk, int base, in
                                  const int *diagslots, const float *vals32,
                                  const double *diagvalues, float *x32, double *b, int maxw);
 
-// BLAS-1/2 on device vectors.  Reductions write to out (device) in a fixed
-// order; part must hold kry_parts(n) doubles per reduced quantity.
-UCFD_HIDDEN int kry_parts(int64_t n);
+// Scalars posted to the host by the kernel that forms them: values at out (the
+// device address of pinned memory), then seq at word (0: not yet the last).
+// out NULL: nothing posted.
+struct KryPost {
+    double *out = nullptr;
+    unsigned long long *word = nullptr, seq = 0;
+};
+struct KryCoef {
+    double v[64];
+};
+
+// BLAS-1/2 on device vectors.  A reduction leaves its partials, or the one sum
+// where they would be many, in row q at part + q*KRY_MAXPART; the kernel that
+// uses it (over vectors of the same length) sums the row in a fixed order.
+enum { KRY_MAXPART = 1024 };
+// x.y: partials, and with out also the sum (device, posted)
 UCFD_HIDDEN int kry_dot(hipStream_t s, int64_t n, const double *x, const double *y, double *part,
-                        double *out);
+                        double *out, const KryPost &h = KryPost());
 UCFD_HIDDEN int kry_axpy(hipStream_t s, int64_t n, double a, const double *x, double *y);
 UCFD_HIDDEN int kry_axpby(hipStream_t s, int64_t n, double a, const double *x, double b,
                           double *y);  // y = a x + b y
-// dst = src * (1/sqrt(*normsq)); the same values also into dst2 when given
+// dst = src/sqrt(the sum of the partials nsq_part, posted); the same values also
+// into dst2 when given
 UCFD_HIDDEN int kry_scale_by_inv_sqrt(hipStream_t s, int64_t n, const double *src,
-                                      const double *normsq, double *dst,
-                                      double *dst2 = nullptr);
-// h[j] = sum_i V[j*ldv + i] w[i], j < k (k <= 64): out[j] (device)
+                                      const double *nsq_part, double *dst, double *dst2,
+                                      const KryPost &h = KryPost());
+// partials of h[j] = sum_i V[j*ldv + i] w[i], j < k (k <= 64)
 UCFD_HIDDEN int kry_gemvt(hipStream_t s, int64_t n, int k, const double *V, int64_t ldv,
-                          const double *w, double *part, double *out);
-// w[i] += alpha * sum_j V[j*ldv + i] h[j], h on the device; with normsq != NULL
-// also writes sum_i w_new[i]^2 to *normsq
+                          const double *w, double *part);
+// w[i] += alpha * sum_j V[j*ldv + i] h[j], h the sums of the partials hpart
+// (posted); with part also the partials of sum_i w_new[i]^2.  part is not hpart.
 UCFD_HIDDEN int kry_gemv(hipStream_t s, int64_t n, int k, const double *V, int64_t ldv,
-                         double alpha, const double *h, double *w, double *part,
-                         double *normsq);
+                         double alpha, const double *hpart, double *w, double *part,
+                         const KryPost &h = KryPost());
 // kry_gemv (no norm) followed by kry_gemvt on the updated w, in one pass over
-// V when k <= 32: w[i] += alpha * sum_j V[j*ldv + i] h[j]; out[j] = V_j . w
+// V when k <= 32.  part is not hpart.
 UCFD_HIDDEN int kry_gemv_gemvt(hipStream_t s, int64_t n, int k, const double *V, int64_t ldv,
-                               double alpha, const double *h, double *w, double *part,
-                               double *out);
-// BiCGSTAB fused reduction (bicgstab.c:5-22): out[0..4] = (rt.s, rt.t, t.s, t.t, s.s)
+                               double alpha, const double *hpart, double *w, double *part,
+                               const KryPost &h = KryPost());
+// x += V y
+UCFD_HIDDEN int kry_gemv_y(hipStream_t s, int64_t n, int k, const double *V, int64_t ldv,
+                           const KryCoef &y, double *x);
+// BiCGSTAB fused reduction (bicgstab.c:5-22): partials of (rt.s, rt.t, t.s, t.t,
+// s.s) in rows 0..4
 UCFD_HIDDEN int kry_dot5(hipStream_t s, int64_t n, const double *rt, const double *sv,
-                         const double *t, double *part, double *out);
+                         const double *t, double *part);
 // p = r + beta*(p - omega*v); pt = p
 UCFD_HIDDEN int kry_bicg_p(hipStream_t s, int64_t n, double beta, double omega, const double *r,
                            const double *v, double *p, double *pt);
-// s = r - alpha*v; shat = s, with alpha = rho / *pi (pi on the device)
-UCFD_HIDDEN int kry_bicg_s(hipStream_t s, int64_t n, double rho, const double *pi,
+// s = r - alpha*v; shat = s, with alpha = rho / pi, pi the sum of pi_part
+UCFD_HIDDEN int kry_bicg_s(hipStream_t s, int64_t n, double rho, const double *pi_part,
                            const double *r, const double *v, double *sv, double *shat);
 // b = (float)a
 UCFD_HIDDEN int kry_cast32(hipStream_t s, int64_t n, const double *a, float *b);
-// x += alpha*pt + omega*shat; r = s - omega*t
-UCFD_HIDDEN int kry_bicg_xr(hipStream_t s, int64_t n, double alpha, const double *pt,
-                            double omega, const double *shat, const double *sv, const double *t,
-                            double *x, double *r);
+// pi and the five dots from their partials (posted as dots 0..4, pi), then
+// x += alpha*pt + omega*shat; r = s - omega*t with alpha = rho/pi, omega =
+// t.s/t.t; |pi| < 1e-30 leaves x and r alone
+UCFD_HIDDEN int kry_bicg_xr(hipStream_t s, int64_t n, double rho, const double *pi_part,
+                            const double *dots, const double *pt, const double *shat,
+                            const double *sv, const double *t, double *x, double *r,
+                            const KryPost &h);
 UCFD_HIDDEN int kry_copy(hipStream_t s, int64_t n, const double *x, double *y);
 UCFD_HIDDEN int kry_fill(hipStream_t s, int64_t n, double v, double *y);

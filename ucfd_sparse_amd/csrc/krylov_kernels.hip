@@ -22,7 +22,7 @@
 namespace {
 
 constexpr int KB = KRY_BLOCK;
-constexpr int KMAXPART = 1024;
+constexpr int KMAXPART = KRY_MAXPART;
 
 __device__ __forceinline__ int kxcd()
 {
@@ -761,22 +761,81 @@ __device__ __forceinline__ double block_reduce(double v)
     return s;
 }
 
-// out[q] = sum of part[q*stride + 0..np-1], one block per q, fixed order
-__global__ __launch_bounds__(1024) void k_sum_rows(const double *part, int np, int stride,
-                                                   double *out)
+// Sum of row part[0 .. np-1] (np <= KMAXPART) by one wave, in every lane: the
+// sums of 64 consecutive partials (a fixed tree), added in order.
+__device__ __forceinline__ double wave_row_sum(const double *__restrict__ part, int np)
+{
+    constexpr int U = 8;
+    const int lane = threadIdx.x & 63;
+    double t = 0.0;
+    for (int q0 = 0; q0 < np; q0 += 64*U) {
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int j = q0 + u*64 + lane;
+            v[u] = j < np ? part[j] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (q0 + u*64 >= np) break;
+            for (int o = 32; o > 0; o >>= 1) v[u] += __shfl_xor(v[u], o, 64);
+            t += v[u];
+        }
+    }
+    return t;
+}
+
+// hs[j] = the sum of row j of the partials, j < k, by the workgroup.  A kernel
+// that needs the result of a reduction sums its partials itself, every
+// workgroup for itself, when there are at most KFUSE a row: 21K unknowns, 83
+// partials a row, save a launch and its gap (2.3 + 1.5 us) for under 1 us.  With
+// 1024 a row the sums cost 8 us (k = 4) to 17 us (k = 10) where the launch costs
+// 4.7, so longer rows are summed to one value by k_sum_rows first.
+constexpr int KFUSE = 256;
+
+__device__ __forceinline__ void block_row_sums(double *hs, const double *__restrict__ part, int np,
+                                               int k)
+{
+    for (int j = threadIdx.x >> 6; j < k; j += KB/64) {
+        const double t = wave_row_sum(part + (int64_t)j*KMAXPART, np);
+        if ((threadIdx.x & 63) == 0) hs[j] = t;
+    }
+    __syncthreads();
+}
+
+// Scalars for the host: written to pinned memory by the first workgroup, the
+// sequence number last (KryPost::seq 0: more values follow from a later kernel)
+__device__ __forceinline__ void post(const KryPost &h, const double *v, int k)
+{
+    if (blockIdx.x != 0 || threadIdx.x != 0 || !h.out) return;
+    for (int j = 0; j < k; ++j)
+        __hip_atomic_store(h.out + j, v[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (h.seq)
+        __hip_atomic_store(h.word, h.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// one workgroup per row: the row's sum replaces its first partial
+__global__ __launch_bounds__(1024) void k_sum_rows(double *part, int np)
 {
     __shared__ double red[16];
-    const double *p = part + (int64_t)blockIdx.x*stride;
-    double s = 0.0;
-    for (int j = threadIdx.x; j < np; j += 1024) s += p[j];
+    double *p = part + (int64_t)blockIdx.x*KMAXPART;
+    double s = (int)threadIdx.x < np ? p[threadIdx.x] : 0.0;
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
     if (threadIdx.x % 64 == 0) red[threadIdx.x/64] = s;
     __syncthreads();
     if (threadIdx.x == 0) {
         double t = 0.0;
         for (int w = 0; w < 16; ++w) t += red[w];
-        out[blockIdx.x] = t;
+        p[0] = t;
     }
+}
+
+// one row's sum, to out (device) and to the host
+__global__ __launch_bounds__(64) void k_sum_row(const double *part, int np, double *out, KryPost h)
+{
+    const double t = wave_row_sum(part, np);
+    if (threadIdx.x == 0) *out = t;
+    post(h, &t, 1);
 }
 
 __global__ __launch_bounds__(KB) void k_dot(int64_t n, const double *__restrict__ x,
@@ -828,13 +887,16 @@ __global__ __launch_bounds__(KB) void k_gemvt8(int64_t n, int k, int j0, const d
     }
 }
 
+// w += alpha V h, h the sums of the partials hpart (posted to the host), and
+// with part the partials of |w|^2.  Any k <= 64.
 __global__ __launch_bounds__(KB) void k_gemv(int64_t n, int k, const double *__restrict__ V,
-                                             int64_t ldv, double alpha, const double *__restrict__ h,
-                                             double *__restrict__ w, double *part)
+                                             int64_t ldv, double alpha,
+                                             const double *__restrict__ hpart, int np,
+                                             double *__restrict__ w, double *part, KryPost post_h)
 {
     __shared__ double hs[64];
-    if (threadIdx.x < k) hs[threadIdx.x] = h[threadIdx.x];
-    __syncthreads();
+    block_row_sums(hs, hpart, np, k);
+    post(post_h, hs, k);
     double ss = 0.0;
     const int64_t st = (int64_t)gridDim.x*KB;
     for (int64_t i = (int64_t)blockIdx.x*KB + threadIdx.x; i < n; i += st) {
@@ -856,12 +918,13 @@ __global__ __launch_bounds__(KB) void k_gemv(int64_t n, int k, const double *__r
 template <int KM>
 __global__ __launch_bounds__(KB) void k_gemv_r(int64_t n, int k, const double *__restrict__ V,
                                                int64_t ldv, double alpha,
-                                               const double *__restrict__ h,
-                                               double *__restrict__ w, double *part)
+                                               const double *__restrict__ hpart, int np,
+                                               double *__restrict__ w, double *part,
+                                               KryPost post_h)
 {
     __shared__ double hs[KM];
-    if (threadIdx.x < k) hs[threadIdx.x] = h[threadIdx.x];
-    __syncthreads();
+    block_row_sums(hs, hpart, np, k);
+    post(post_h, hs, k);
     double ss = 0.0;
     const int64_t st = (int64_t)gridDim.x*KB;
     for (int64_t i = (int64_t)blockIdx.x*KB + threadIdx.x; i < n; i += st) {
@@ -879,6 +942,27 @@ __global__ __launch_bounds__(KB) void k_gemv_r(int64_t n, int k, const double *_
     if (part) {
         ss = block_reduce(ss);
         if (threadIdx.x == 0) part[blockIdx.x] = ss;
+    }
+}
+
+// x += V y with the coefficients in the launch's arguments (no copy to the
+// device): k_gemv's sums, KM columns at a time with their loads issued together
+template <int KM>
+__global__ __launch_bounds__(KB) void k_gemv_y(int64_t n, int k, const double *__restrict__ V,
+                                               int64_t ldv, KryCoef y, double *__restrict__ x)
+{
+    const int64_t st = (int64_t)gridDim.x*KB;
+    for (int64_t i = (int64_t)blockIdx.x*KB + threadIdx.x; i < n; i += st) {
+        double sum = 0.0;
+        for (int j = 0; j < k; j += KM) {
+            double vr[KM];
+#pragma unroll
+            for (int q = 0; q < KM; ++q) vr[q] = j + q < k ? V[(int64_t)(j + q)*ldv + i] : 0.0;
+#pragma unroll
+            for (int q = 0; q < KM; ++q)
+                if (j + q < k) sum += vr[q]*y.v[j + q];
+        }
+        x[i] = 1.0*sum + 1.0*x[i];
     }
 }
 
@@ -917,12 +1001,14 @@ __global__ __launch_bounds__(KB) void k_gemvt_all(int64_t n, int k, const double
 template <int KM>
 __global__ __launch_bounds__(KB) void k_gemv_gemvt(int64_t n, int k,
                                                    const double *__restrict__ V, int64_t ldv,
-                                                   double alpha, const double *__restrict__ h,
-                                                   double *__restrict__ w, double *part)
+                                                   double alpha,
+                                                   const double *__restrict__ hpart, int np,
+                                                   double *__restrict__ w, double *part,
+                                                   KryPost post_h)
 {
     __shared__ double hs[KM];
-    if (threadIdx.x < k) hs[threadIdx.x] = h[threadIdx.x];
-    __syncthreads();
+    block_row_sums(hs, hpart, np, k);
+    post(post_h, hs, k);
     double acc[KM];
 #pragma unroll
     for (int q = 0; q < KM; ++q) acc[q] = 0.0;
@@ -949,12 +1035,16 @@ __global__ __launch_bounds__(KB) void k_gemv_gemvt(int64_t n, int k,
         }
 }
 
+// dst = src/sqrt(sum of the partials nsq), the sum posted to the host
 __global__ __launch_bounds__(KB) void k_scale_isqrt(int64_t n, const double *__restrict__ src,
-                                                    const double *__restrict__ nsq,
+                                                    const double *__restrict__ nsq, int np,
                                                     double *__restrict__ dst,
-                                                    double *__restrict__ dst2)
+                                                    double *__restrict__ dst2, KryPost post_n)
 {
-    const double inv = 1.0/sqrt(*nsq);
+    __shared__ double hs[1];
+    block_row_sums(hs, nsq, np, 1);
+    post(post_n, hs, 1);
+    const double inv = 1.0/sqrt(hs[0]);
     const int64_t st = (int64_t)gridDim.x*KB;
     for (int64_t i = (int64_t)blockIdx.x*KB + threadIdx.x; i < n; i += st) {
         const double v = inv*src[i];
@@ -991,14 +1081,17 @@ __global__ __launch_bounds__(KB) void k_bicg_p(int64_t n, double beta, double om
 }
 
 // s = r - alpha*v (as copy + axpy); shat = s
-// alpha = rho/pi with pi read on the device (the host forms the same
+// alpha = rho/pi with pi the sum of the partials (the host forms the same
 // quotient once it has pi)
-__global__ __launch_bounds__(KB) void k_bicg_s(int64_t n, double rho, const double *__restrict__ pi,
+__global__ __launch_bounds__(KB) void k_bicg_s(int64_t n, double rho,
+                                               const double *__restrict__ pi_part, int np,
                                                const double *__restrict__ r,
                                                const double *__restrict__ v,
                                                double *__restrict__ sv, double *__restrict__ shat)
 {
-    const double alpha = rho/(*pi);
+    __shared__ double hs[1];
+    block_row_sums(hs, pi_part, np, 1);
+    const double alpha = rho/hs[0];
     const int64_t st = (int64_t)gridDim.x*KB;
     for (int64_t i = (int64_t)blockIdx.x*KB + threadIdx.x; i < n; i += st) {
         const double t = r[i] + (-alpha)*v[i];
@@ -1014,13 +1107,27 @@ __global__ __launch_bounds__(KB) void k_cast32(int64_t n, const double *__restri
     for (int64_t i = (int64_t)blockIdx.x*KB + threadIdx.x; i < n; i += st) b[i] = (float)a[i];
 }
 
-__global__ __launch_bounds__(KB) void k_bicg_xr(int64_t n, double alpha,
-                                                const double *__restrict__ pt, double omega,
+// The end of a BiCGSTAB iteration: pi and the five dots summed from their
+// partials and posted to the host, alpha = rho/pi and omega = (t.s)/(t.t) formed
+// here as the host forms them, then x += alpha pt + omega shat, r = s - omega t.
+// A pi breakdown (bicgstab.c:84) leaves x and r as they are.
+__global__ __launch_bounds__(KB) void k_bicg_xr(int64_t n, double rho,
+                                                const double *__restrict__ pi_part,
+                                                const double *__restrict__ dots, int np,
+                                                const double *__restrict__ pt,
                                                 const double *__restrict__ shat,
                                                 const double *__restrict__ sv,
                                                 const double *__restrict__ t,
-                                                double *__restrict__ x, double *__restrict__ r)
+                                                double *__restrict__ x, double *__restrict__ r,
+                                                KryPost post_d)
 {
+    __shared__ double hs[6];
+    block_row_sums(hs, dots, np, 5);
+    block_row_sums(hs + 5, pi_part, np, 1);
+    post(post_d, hs, 6);
+    const double pi = hs[5];
+    if (fabs(pi) < 1e-30) return;
+    const double alpha = rho/pi, omega = hs[2]/hs[3];
     const int64_t st = (int64_t)gridDim.x*KB;
     for (int64_t i = (int64_t)blockIdx.x*KB + threadIdx.x; i < n; i += st) {
         double xv = x[i] + alpha*pt[i];
@@ -1259,27 +1366,39 @@ int kry_bsgs_sweep32(hipStream_t s, int upper, int blk, int base, int cnt, const
                            diagvalues, x32, b, maxw);
 }
 
-int kry_parts(int64_t n) { return KMAXPART; }
+namespace {
 
-int kry_dot(hipStream_t s, int64_t n, const double *x, const double *y, double *part, double *out)
+// partials a consumer finds per row of a reduction over n elements
+int row_np(int64_t n) { return nblocks(n) <= KFUSE ? nblocks(n) : 1; }
+
+void shorten_rows(hipStream_t s, int64_t n, double *part, int rows)
+{
+    if (nblocks(n) > KFUSE)
+        hipLaunchKernelGGL(k_sum_rows, dim3(rows), dim3(1024), 0, s, part, nblocks(n));
+}
+
+}  // namespace
+
+int kry_dot(hipStream_t s, int64_t n, const double *x, const double *y, double *part, double *out,
+            const KryPost &h)
 {
     const int nb = nblocks(n);
     hipLaunchKernelGGL(k_dot, dim3(nb), dim3(KB), 0, s, n, x, y, part);
-    hipLaunchKernelGGL(k_sum_rows, dim3(1), dim3(1024), 0, s, part, nb, KMAXPART, out);
+    shorten_rows(s, n, part, 1);
+    if (out) hipLaunchKernelGGL(k_sum_row, dim3(1), dim3(64), 0, s, part, row_np(n), out, h);
     return ok();
 }
 
 int kry_dot5(hipStream_t s, int64_t n, const double *rt, const double *sv, const double *t,
-             double *part, double *out)
+             double *part)
 {
-    const int nb = nblocks(n);
-    hipLaunchKernelGGL(k_dot5, dim3(nb), dim3(KB), 0, s, n, rt, sv, t, part);
-    hipLaunchKernelGGL(k_sum_rows, dim3(5), dim3(1024), 0, s, part, nb, KMAXPART, out);
+    hipLaunchKernelGGL(k_dot5, dim3(nblocks(n)), dim3(KB), 0, s, n, rt, sv, t, part);
+    shorten_rows(s, n, part, 5);
     return ok();
 }
 
 int kry_gemvt(hipStream_t s, int64_t n, int k, const double *V, int64_t ldv, const double *w,
-              double *part, double *out)
+              double *part)
 {
     if (k <= 0 || k > 64) return UCFD_ERR_ARG;
     const int nb = nblocks(n);
@@ -1292,54 +1411,69 @@ int kry_gemvt(hipStream_t s, int64_t n, int k, const double *V, int64_t ldv, con
     else
         for (int j0 = 0; j0 < k; j0 += 8)
             hipLaunchKernelGGL(k_gemvt8, dim3(nb), dim3(KB), 0, s, n, k, j0, V, ldv, w, part);
-    hipLaunchKernelGGL(k_sum_rows, dim3(k), dim3(1024), 0, s, part, nb, KMAXPART, out);
+    shorten_rows(s, n, part, k);
     return ok();
 }
 
 int kry_gemv_gemvt(hipStream_t s, int64_t n, int k, const double *V, int64_t ldv, double alpha,
-                   const double *h, double *w, double *part, double *out)
+                   const double *hpart, double *w, double *part, const KryPost &h)
 {
     if (k <= 0 || k > 64) return UCFD_ERR_ARG;
     if (k > 32) {
-        int rc = kry_gemv(s, n, k, V, ldv, alpha, h, w, part, nullptr);
-        return rc ? rc : kry_gemvt(s, n, k, V, ldv, w, part, out);
+        int rc = kry_gemv(s, n, k, V, ldv, alpha, hpart, w, nullptr, h);
+        return rc ? rc : kry_gemvt(s, n, k, V, ldv, w, part);
     }
-    const int nb = nblocks(n);
+    const int nb = nblocks(n), np = row_np(n);
     if (k <= 8)
-        hipLaunchKernelGGL(k_gemv_gemvt<8>, dim3(nb), dim3(KB), 0, s, n, k, V, ldv, alpha, h, w,
-                           part);
+        hipLaunchKernelGGL(k_gemv_gemvt<8>, dim3(nb), dim3(KB), 0, s, n, k, V, ldv, alpha, hpart,
+                           np, w, part, h);
     else if (k <= 16)
-        hipLaunchKernelGGL(k_gemv_gemvt<16>, dim3(nb), dim3(KB), 0, s, n, k, V, ldv, alpha, h, w,
-                           part);
+        hipLaunchKernelGGL(k_gemv_gemvt<16>, dim3(nb), dim3(KB), 0, s, n, k, V, ldv, alpha, hpart,
+                           np, w, part, h);
     else
-        hipLaunchKernelGGL(k_gemv_gemvt<32>, dim3(nb), dim3(KB), 0, s, n, k, V, ldv, alpha, h, w,
-                           part);
-    hipLaunchKernelGGL(k_sum_rows, dim3(k), dim3(1024), 0, s, part, nb, KMAXPART, out);
+        hipLaunchKernelGGL(k_gemv_gemvt<32>, dim3(nb), dim3(KB), 0, s, n, k, V, ldv, alpha, hpart,
+                           np, w, part, h);
+    shorten_rows(s, n, part, k);
     return ok();
 }
 
 int kry_gemv(hipStream_t s, int64_t n, int k, const double *V, int64_t ldv, double alpha,
-             const double *h, double *w, double *part, double *normsq)
+             const double *hpart, double *w, double *part, const KryPost &h)
 {
     if (k <= 0 || k > 64) return UCFD_ERR_ARG;
-    const int nb = nblocks(n);
-    double *pp = normsq ? part : nullptr;
+    const int nb = nblocks(n), np = row_np(n);
     if (k <= 8)
-        hipLaunchKernelGGL(k_gemv_r<8>, dim3(nb), dim3(KB), 0, s, n, k, V, ldv, alpha, h, w, pp);
+        hipLaunchKernelGGL(k_gemv_r<8>, dim3(nb), dim3(KB), 0, s, n, k, V, ldv, alpha, hpart, np,
+                           w, part, h);
     else if (k <= 16)
-        hipLaunchKernelGGL(k_gemv_r<16>, dim3(nb), dim3(KB), 0, s, n, k, V, ldv, alpha, h, w, pp);
+        hipLaunchKernelGGL(k_gemv_r<16>, dim3(nb), dim3(KB), 0, s, n, k, V, ldv, alpha, hpart, np,
+                           w, part, h);
     else if (k <= 32)
-        hipLaunchKernelGGL(k_gemv_r<32>, dim3(nb), dim3(KB), 0, s, n, k, V, ldv, alpha, h, w, pp);
+        hipLaunchKernelGGL(k_gemv_r<32>, dim3(nb), dim3(KB), 0, s, n, k, V, ldv, alpha, hpart, np,
+                           w, part, h);
     else
-        hipLaunchKernelGGL(k_gemv, dim3(nb), dim3(KB), 0, s, n, k, V, ldv, alpha, h, w, pp);
-    if (normsq) hipLaunchKernelGGL(k_sum_rows, dim3(1), dim3(1024), 0, s, part, nb, KMAXPART, normsq);
+        hipLaunchKernelGGL(k_gemv, dim3(nb), dim3(KB), 0, s, n, k, V, ldv, alpha, hpart, np, w,
+                           part, h);
+    if (part) shorten_rows(s, n, part, 1);
     return ok();
 }
 
-int kry_scale_by_inv_sqrt(hipStream_t s, int64_t n, const double *src, const double *normsq,
-                          double *dst, double *dst2)
+int kry_gemv_y(hipStream_t s, int64_t n, int k, const double *V, int64_t ldv, const KryCoef &y,
+               double *x)
 {
-    hipLaunchKernelGGL(k_scale_isqrt, dim3(nblocks(n)), dim3(KB), 0, s, n, src, normsq, dst, dst2);
+    if (k <= 0 || k > 64) return UCFD_ERR_ARG;
+    if (k <= 8)
+        hipLaunchKernelGGL(k_gemv_y<8>, dim3(nblocks(n)), dim3(KB), 0, s, n, k, V, ldv, y, x);
+    else
+        hipLaunchKernelGGL(k_gemv_y<16>, dim3(nblocks(n)), dim3(KB), 0, s, n, k, V, ldv, y, x);
+    return ok();
+}
+
+int kry_scale_by_inv_sqrt(hipStream_t s, int64_t n, const double *src, const double *nsq_part,
+                          double *dst, double *dst2, const KryPost &h)
+{
+    hipLaunchKernelGGL(k_scale_isqrt, dim3(nblocks(n)), dim3(KB), 0, s, n, src, nsq_part, row_np(n),
+                       dst, dst2, h);
     return ok();
 }
 
@@ -1375,10 +1509,11 @@ int kry_bicg_p(hipStream_t s, int64_t n, double beta, double omega, const double
     return ok();
 }
 
-int kry_bicg_s(hipStream_t s, int64_t n, double rho, const double *pi, const double *r,
+int kry_bicg_s(hipStream_t s, int64_t n, double rho, const double *pi_part, const double *r,
                const double *v, double *sv, double *shat)
 {
-    hipLaunchKernelGGL(k_bicg_s, dim3(nblocks(n)), dim3(KB), 0, s, n, rho, pi, r, v, sv, shat);
+    hipLaunchKernelGGL(k_bicg_s, dim3(nblocks(n)), dim3(KB), 0, s, n, rho, pi_part, row_np(n),
+                       r, v, sv, shat);
     return ok();
 }
 
@@ -1389,10 +1524,11 @@ int kry_cast32(hipStream_t s, int64_t n, const double *a, float *b)
     return ok();
 }
 
-int kry_bicg_xr(hipStream_t s, int64_t n, double alpha, const double *pt, double omega,
-                const double *shat, const double *sv, const double *t, double *x, double *r)
+int kry_bicg_xr(hipStream_t s, int64_t n, double rho, const double *pi_part, const double *dots,
+                const double *pt, const double *shat, const double *sv, const double *t, double *x,
+                double *r, const KryPost &h)
 {
-    hipLaunchKernelGGL(k_bicg_xr, dim3(nblocks(n)), dim3(KB), 0, s, n, alpha, pt, omega, shat, sv,
-                       t, x, r);
+    hipLaunchKernelGGL(k_bicg_xr, dim3(nblocks(n)), dim3(KB), 0, s, n, rho, pi_part, dots,
+                       row_np(n), pt, shat, sv, t, x, r, h);
     return ok();
 }

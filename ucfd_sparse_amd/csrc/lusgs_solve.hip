@@ -1087,24 +1087,13 @@ int residual64(ucfd_lusgs_solver *s, hipStream_t st, const double *b, const doub
 
 // The norm last requested, as soon as the kernel that sums it has written it:
 // the rest of that launch and those behind it run while the host decides and
-// enqueues the next pass.  The poll ends with the value, or with the stream
-// (finished without it, or failed).
+// enqueues the next pass.
 int read_norm(ucfd_lusgs_solver *s, hipStream_t st, double *out, const char *fn)
 {
-    const unsigned long long *word = (const unsigned long long *)s->hnorm + 1;
-    for (;;) {
-        for (int k = 0; k < 4096; ++k) {
-            if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == s->seq) {
-                *out = sqrt(*(volatile double *)s->hnorm);
-                return UCFD_OK;
-            }
-            __builtin_ia32_pause();
-        }
-        const hipError_t q = hipStreamQuery(st);
-        if (q == hipErrorNotReady) continue;
-        if (q == hipSuccess && __atomic_load_n(word, __ATOMIC_ACQUIRE) == s->seq) continue;
-        return ucfd_check_hip(q == hipSuccess ? hipErrorUnknown : q, fn, "norm of the residual");
-    }
+    int rc = ucfd_poll((const unsigned long long *)s->hnorm + 1, s->seq, st, fn,
+                       "norm of the residual");
+    *out = sqrt(*(volatile double *)s->hnorm);
+    return rc;
 }
 
 }  // namespace

@@ -165,6 +165,21 @@ int ucfd_sync_and_check(const char *fn)
     return UCFD_OK;
 }
 
+int ucfd_poll(const unsigned long long *word, unsigned long long want, hipStream_t st,
+              const char *fn, const char *what)
+{
+    for (;;) {
+        for (int k = 0; k < 4096; ++k) {
+            if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == want) return UCFD_OK;
+            __builtin_ia32_pause();
+        }
+        const hipError_t q = hipStreamQuery(st);
+        if (q == hipErrorNotReady) continue;
+        if (q == hipSuccess && __atomic_load_n(word, __ATOMIC_ACQUIRE) == want) return UCFD_OK;
+        return ucfd_check_hip(q == hipSuccess ? hipErrorUnknown : q, fn, what);
+    }
+}
+
 int UcfdStage::add(const void *p, size_t bytes, int dir)
 {
     Arg &a = args[nargs];

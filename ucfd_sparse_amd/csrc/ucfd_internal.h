@@ -45,6 +45,13 @@ UCFD_HIDDEN bool ucfd_is_device_ptr(const void *p);
 // cleared).  Call with the runtime lock held or outside any staging.
 UCFD_HIDDEN int ucfd_sync_and_check(const char *fn);
 
+// Wait until a kernel on st has stored want to *word (pinned memory, after the
+// values it announces): polls the word, so the work behind that kernel runs on
+// meanwhile.  Ends with the word, or with the stream (finished without it, or
+// failed).
+UCFD_HIDDEN int ucfd_poll(const unsigned long long *word, unsigned long long want, hipStream_t st,
+                          const char *fn, const char *what);
+
 // Staging of host arrays for one call.  Device (or managed) pointers are used
 // in place; host pointers are copied to a library workspace on entry and
 // copied back on exit when written.  Arguments that alias share one buffer.
