@@ -19,8 +19,7 @@
 namespace {
 
 constexpr int FB = 256;
-constexpr int FSTAGE = 16000;   // LDS bytes of staged blocks per wave
-constexpr int FKP = 4;          // positions per cell whose neighbour rows are fetched first
+constexpr int FKP = 4;          // positions per cell whose loads are issued together
 
 __device__ __forceinline__ int fxcd()
 {
@@ -513,85 +512,16 @@ __global__ __launch_bounds__(FB) void k_sweep(int base, int cnt, const int *__re
 // lane (g, row) = (lane / NV, lane % NV) accumulates component `row` of
 // cell g over every position in the order of k_sweep above; the group
 // exchanges its NV values with lane shuffles and every lane runs the cell's
-// diagonal solve.  The wave's packed blocks and fv values are contiguous
-// (positions of consecutive cells are consecutive) and are staged through
-// LDS with coalesced loads when they fit the launch's cap positions (dynamic
-// LDS, sized from the level's largest wave so that LDS does not limit the
-// waves per SIMD more than needed; at most FSTAGE bytes of blocks);
-// otherwise the lanes read them from HBM directly.  The LU blocks are read
-// from HBM by the row's lanes (staging them would cost LDS, and one wave
-// per SIMD).  Results equal k_sweep's bit for bit.
-
-template <int NV, bool F32, bool STAGED>
-__device__ __forceinline__ void fs_rows(int row, int g, bool act, int r, int st, int ed, int p0w,
-                                        int var0, int nvars, const int *__restrict__ colidx,
-                                        const typename std::conditional<F32, float, double>::type
-                                            *blocks,
-                                        const typename std::conditional<F32, float, double>::type
-                                            *fvs,
-                                        const double *lu_src, const double *__restrict__ rhs,
-                                        double *du, float *du32)
-{
-    using T = typename std::conditional<F32, float, double>::type;
-    constexpr int D2 = NV*NV;
-    T xn[FKP][NV];
-#pragma unroll
-    for (int k = 0; k < FKP; ++k)
-        if (st + k < ed) {
-            const int64_t nb = colidx[st + k];
-#pragma unroll
-            for (int c = 0; c < NV; ++c)
-                xn[k][c] = F32 ? (T)du32[var0 + c + nb*nvars] : (T)du[var0 + c + nb*nvars];
-        }
-    double x = act ? rhs[var0 + row + (int64_t)r*nvars] : 0.0;
-#pragma unroll
-    for (int k = 0; k < FKP; ++k) {
-        const int p = st + k;
-        if (p < ed) {
-            const int64_t q = STAGED ? p - p0w : p;
-            const T *blk = blocks + q*D2 + row*NV;
-            T val = T(0);
-#pragma unroll
-            for (int c = 0; c < NV; ++c) val += blk[c]*xn[k][c];
-            x -= (double)(val*fvs[q]);
-        }
-    }
-    for (int p = st + FKP; p < ed; ++p) {
-        const int64_t nb = colidx[p];
-        const int64_t q = STAGED ? p - p0w : p;
-        const T *blk = blocks + q*D2 + row*NV;
-        T val = T(0);
-#pragma unroll
-        for (int c = 0; c < NV; ++c)
-            val += blk[c]*(F32 ? (T)du32[var0 + c + nb*nvars] : (T)du[var0 + c + nb*nvars]);
-        x -= (double)(val*fvs[q]);
-    }
-    double xv[NV], lu[D2], myrow[NV];
-#pragma unroll
-    for (int c = 0; c < NV; ++c) xv[c] = __shfl(x, g*NV + c, 64);
-    // each lane reads its own row of the LU block; the group's lanes then
-    // exchange the rows, so every lane holds the whole block
-#pragma unroll
-    for (int c = 0; c < NV; ++c) myrow[c] = act ? lu_src[row*NV + c] : 0.0;
-#pragma unroll
-    for (int rr = 0; rr < NV; ++rr)
-#pragma unroll
-        for (int c = 0; c < NV; ++c) lu[rr*NV + c] = __shfl(myrow[c], g*NV + rr, 64);
-    if (!act) return;
-    ucfd::lusub<NV>(lu, xv);
-    const int64_t o = var0 + row + (int64_t)r*nvars;
-    du[o] = xv[row];
-    if (F32) du32[o] = (float)xv[row];
-}
-
-// staged positions per wave: FSTAGE bytes of blocks, at most 8 per cell
-template <int NV, typename T> constexpr int fs_stage_max()
-{
-    return FSTAGE/((int)sizeof(T)*NV*NV) < 8*(64/NV) ? FSTAGE/((int)sizeof(T)*NV*NV) : 8*(64/NV);
-}
-
+// diagonal solve.  Block rows and neighbour rows are read in the widest loads
+// that cover them (wave_rows.h), FKP positions together; each lane reads its own
+// row of the LU block at the start and the group exchanges the rows.  Results
+// equal k_sweep's bit for bit.  NS lower + upper, us, against blocks staged
+// through LDS (FP64 / FP32 products): 4.9K hexes 25.2 -> 15.9, 91K 80.7 -> 60.9 /
+// 54.9 -> 45.4, 25K tets 27.8 -> 20.9, 356K 167.9 -> 158.8 / 123.0 -> 113.7 (FP64
+// 5.2 TB/s); with the whole LU block in every lane from the start 356K tets
+// took 178.7, read at the end 166.1.
 template <int NV, bool F32>
-__global__ __launch_bounds__(64) void k_sweep_w(int base, int cnt, int cap, int var0, int nvars,
+__global__ __launch_bounds__(64) void k_sweep_w(int base, int cnt, int var0, int nvars,
                                                 const int *__restrict__ rowptr,
                                                 const int *__restrict__ colidx,
                                                 const typename std::conditional<F32, float,
@@ -605,55 +535,64 @@ __global__ __launch_bounds__(64) void k_sweep_w(int base, int cnt, int cap, int 
                                                 float *du32)
 {
     using T = typename std::conditional<F32, float, double>::type;
-    constexpr int D2 = NV*NV, G = 64/NV;
-    constexpr int CP = fs_stage_max<NV, T>();
-    constexpr int UJ = (CP*D2 + 63)/64, UF = (CP + 63)/64;
-    // dynamic LDS: cap blocks, then cap fv values (the rows' LU blocks are
-    // read from HBM by each row's lanes)
-    extern __shared__ __align__(16) unsigned char fdyn[];
-    T *sj = (T *)fdyn;
-    T *sf = sj + (size_t)cap*D2;
+    constexpr int D2 = NV*NV, G = 64/NV, KP = FKP;
     const int lane = threadIdx.x;
     const int t0 = ucfd::wave_xcd_index()*G;
     if (t0 >= cnt) return;
     const int g = lane/NV, row = lane%NV;
-    const int nrows = min(G, cnt - t0);
-    const int r0 = base + t0, r = r0 + g;
-    const bool act = g < nrows;
-    const int p0w = rowptr[r0], p1w = rowptr[r0 + nrows];
-    const int st = act ? rowptr[r] : 0, ed = act ? rowptr[r + 1] : 0;
-    if (p1w - p0w > cap) {
-        fs_rows<NV, F32, false>(row, g, act, r, st, ed, 0, var0, nvars, colidx, jp, fvp,
-                                diag + (int64_t)r*D2, rhs, du, du32);
-        return;
+    const int r = base + t0 + g;
+    const bool act = g < G && t0 + g < cnt;
+    int st = 0, ed = 0;
+    double lu[D2], myrow[NV] = {}, x = 0.0;
+    if (act) {
+        st = rowptr[r];
+        ed = rowptr[r + 1];
+        ucfd::ld_values<NV>(diag + (int64_t)r*D2 + row*NV, myrow);
+        x = rhs[var0 + row + (int64_t)r*nvars];
     }
-    const int nj = (p1w - p0w)*D2, nf = p1w - p0w;
-    const T *js = jp + (int64_t)p0w*D2;
-    const T *fs = fvp + p0w;
-    T tj[UJ], tf[UF];
+    for (int p0 = st; p0 < ed; p0 += KP) {
+        int nb[KP];
+        T blk[KP][NV], fv[KP], xn[KP][NV];
 #pragma unroll
-    for (int u = 0; u < UJ; ++u) {
-        const int e = u*64 + lane;
-        tj[u] = e < nj ? __builtin_nontemporal_load(js + e) : T(0);
-    }
+        for (int k = 0; k < KP; ++k)
+            if (p0 + k < ed) {
+                nb[k] = colidx[p0 + k];
+                ucfd::ld_values<NV>(jp + (int64_t)(p0 + k)*D2 + row*NV, blk[k]);
+                fv[k] = fvp[p0 + k];
+            }
 #pragma unroll
-    for (int u = 0; u < UF; ++u) {
-        const int e = u*64 + lane;
-        tf[u] = e < nf ? __builtin_nontemporal_load(fs + e) : T(0);
-    }
+        for (int k = 0; k < KP; ++k)
+            if (p0 + k < ed) {
+                if constexpr (F32)
+                    ucfd::ld_values<NV>(du32 + var0 + (int64_t)nb[k]*nvars, xn[k]);
+                else
+                    ucfd::ld_values<NV>(du + var0 + (int64_t)nb[k]*nvars, xn[k]);
+            }
 #pragma unroll
-    for (int u = 0; u < UJ; ++u) {
-        const int e = u*64 + lane;
-        if (e < nj) sj[e] = tj[u];
-    }
+        for (int k = 0; k < KP; ++k)
+            if (p0 + k < ed) {
+                T val = T(0);
 #pragma unroll
-    for (int u = 0; u < UF; ++u) {
-        const int e = u*64 + lane;
-        if (e < nf) sf[e] = tf[u];
+                for (int c = 0; c < NV; ++c) val += blk[k][c]*xn[k][c];
+                x -= (double)(val*fv[k]);
+            }
     }
-    ucfd::wave_lds_sync();
-    fs_rows<NV, F32, true>(row, g, act, r, st, ed, p0w, var0, nvars, colidx, sj, sf,
-                           diag + (int64_t)(act ? r : r0)*D2, rhs, du, du32);
+    double xv[NV];
+#pragma unroll
+    for (int c = 0; c < NV; ++c) xv[c] = __shfl(x, g*NV + c, 64);
+#pragma unroll
+    for (int rr = 0; rr < NV; ++rr)
+#pragma unroll
+        for (int c = 0; c < NV; ++c) lu[rr*NV + c] = __shfl(myrow[c], g*NV + rr, 64);
+    if (!act) return;
+    ucfd::lusub<NV>(lu, xv);
+    double mine = xv[0];
+#pragma unroll
+    for (int c = 1; c < NV; ++c)
+        if (row == c) mine = xv[c];
+    const int64_t o = var0 + row + (int64_t)r*nvars;
+    du[o] = mine;
+    if (F32) du32[o] = (float)mine;
 }
 
 // ------------------------------------------------------ scalar LU-SGS
@@ -1208,32 +1147,20 @@ template <int NV> struct PrepL {
     }
 };
 
-template <int NV, typename T> size_t sweep_lds(int cap)
-{
-    return (size_t)cap*(NV*NV + 1)*sizeof(T);
-}
-
 template <int NV> struct SweepL {
     static int run(hipStream_t s, bool f32, int base, int cnt, const int *order, int var0,
                    int nvars, const int *rowptr, const int *colidx, const double *jp,
                    const double *fvp, const float *jp32, const float *fv32, const double *rhs,
-                   const double *diag, double *du, float *du32, int maxw)
+                   const double *diag, double *du, float *du32)
     {
         if (!order) {
             const dim3 g((unsigned)((cnt + 64/NV - 1)/(64/NV)));
-            if (f32) {
-                constexpr int CP = fs_stage_max<NV, float>();
-                const int cap = maxw < 0 || maxw > CP ? CP : maxw;
-                const size_t lds = sweep_lds<NV, float>(cap);
-                hipLaunchKernelGGL((k_sweep_w<NV, true>), g, dim3(64), lds, s, base, cnt, cap, var0,
-                                   nvars, rowptr, colidx, jp32, fv32, rhs, diag, du, du32);
-            } else {
-                constexpr int CP = fs_stage_max<NV, double>();
-                const int cap = maxw < 0 || maxw > CP ? CP : maxw;
-                const size_t lds = sweep_lds<NV, double>(cap);
-                hipLaunchKernelGGL((k_sweep_w<NV, false>), g, dim3(64), lds, s, base, cnt, cap,
-                                   var0, nvars, rowptr, colidx, jp, fvp, rhs, diag, du, du32);
-            }
+            if (f32)
+                hipLaunchKernelGGL((k_sweep_w<NV, true>), g, dim3(64), 0, s, base, cnt, var0, nvars,
+                                   rowptr, colidx, jp32, fv32, rhs, diag, du, du32);
+            else
+                hipLaunchKernelGGL((k_sweep_w<NV, false>), g, dim3(64), 0, s, base, cnt, var0,
+                                   nvars, rowptr, colidx, jp, fvp, rhs, diag, du, du32);
             return ok();
         }
         if (f32)
@@ -1344,11 +1271,11 @@ int fs_launch_prepare(hipStream_t s, int nv, int nlocal, int64_t nfaces, int64_t
 int fs_launch_sweep(hipStream_t s, int nv, bool f32, int base, int cnt, const int *order,
                     int var0, int nvars, const int *rowptr, const int *colidx, const double *jp,
                     const double *fvp, const float *jp32, const float *fv32, const double *rhs,
-                    const double *diag, double *du, float *du32, int maxw)
+                    const double *diag, double *du, float *du32)
 {
     if (cnt <= 0) return UCFD_OK;
     return by_nv<SweepL>(nv, s, f32, base, cnt, order, var0, nvars, rowptr, colidx, jp, fvp, jp32,
-                         fv32, rhs, diag, du, du32, maxw);
+                         fv32, rhs, diag, du, du32);
 }
 
 int fs_launch_zero(hipStream_t s, int64_t n, double *a, double *b, float *c)

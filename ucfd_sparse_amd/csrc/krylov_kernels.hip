@@ -78,19 +78,18 @@ __global__ __launch_bounds__(KB) void k_spmv_bsr(int bn, const int *__restrict__
     if (bad) ucfd::raise(flag, UCFD_KFLAG_INDEX);
 }
 
-// Block sizes 2..7: one wave per G = 64/B block rows (wave_rows.h).  The
-// wave's blocks [rowptr[i0], rowptr[i0+G]) are contiguous; they are staged
-// through LDS in chunks of CB = KSPMV/B^2 blocks with all of a chunk's loads
-// in flight, the column indices and x rows of each lane's first KP blocks
-// are fetched before the staging loads, and lane (g, r) sums scalar row r of
-// block row g in the reference order (per block: v = sum_q A[r][q] x[q],
-// then arr += v).
-constexpr int KSTAGE = 1600;    // staged doubles per wave of the block sweeps (12.8 KB of LDS)
-// SpMV chunks: 6.4 KB of LDS per wave leaves room for 4 waves per SIMD (the
-// register limit), against 3 with 12.8 KB chunks; measured 5 % faster on
-// 5x5 blocks
-constexpr int KSPMV = 800;
-
+// Block sizes 2..7: one wave per G = 64/B block rows; lane (g, r) sums scalar row
+// r of block row g in the reference order (per block: v = sum_q A[r][q] x[q],
+// then arr += v).  A lane reads its B values of a block, and the x row it meets,
+// in the widest loads that cover them (wave_rows.h), KP blocks' loads together:
+// 3 + 3 loads a 5x5 block.  Temporal loads: a block's lines serve all B lanes
+// and several loads (non-temporal ones fetched them again: 89 -> 135 us).
+// Against blocks staged through LDS with consecutive lanes on consecutive words
+// (one scalar load per 64 values, then LDS): 64K hex rows 31.8 -> 21.5 us, 384K
+// tet rows 89.6 -> 82.7, 1M 223 -> 216 (4.6 TB/s of matrix values); 4x4 blocks,
+// 384K rows, 57.4 -> 49.1, 7x7 162.6 -> 155.9.  KP: a tet's whole row of five
+// blocks where the registers allow it (5x5: 82.7 us with 5, 87.8 with 3; 7x7:
+// 155.9 with 3, 163 with 5).
 template <int B>
 __global__ __launch_bounds__(64) void k_spmv_bsr_w(int bn, const int *__restrict__ rowptr,
                                                    const int *__restrict__ colidx,
@@ -98,86 +97,43 @@ __global__ __launch_bounds__(64) void k_spmv_bsr_w(int bn, const int *__restrict
                                                    double alpha, const double *__restrict__ x,
                                                    double beta, double *__restrict__ y, int *flag)
 {
-    constexpr int B2 = B*B, G = 64/B, CB = KSPMV/B2, U = (CB*B2 + 63)/64, KP = 5;
-    __shared__ double sv[CB*B2];
-    const int lane = threadIdx.x;
-    const int i0 = ucfd::wave_xcd_index()*G;
-    if (i0 >= bn) return;
-    const int iend = min(i0 + G, bn);
-    const int g = lane/B, r = lane%B;
-    const int i = i0 + g;
-    const bool act = g < G && i < iend;
-    const int s0 = rowptr[i0], s1 = rowptr[iend];
-    const int st = act ? rowptr[i] : 0, ed = act ? rowptr[i + 1] : 0;
+    constexpr int B2 = B*B, G = 64/B, KP = B <= 5 ? 5 : 3;
+    const int lane = threadIdx.x, g = lane/B, r = lane%B;
+    const int i = ucfd::wave_xcd_index()*G + g;
+    if (g >= G || i >= bn) return;
+    const int st = rowptr[i], ed = rowptr[i + 1];
     bool bad = false;
-    double xp[KP][B];
-    int cp[KP];
-#pragma unroll
-    for (int k = 0; k < KP; ++k) {
-        cp[k] = -1;
-        if (st + k < ed) {
-            const int c = colidx[st + k];
-            if ((unsigned)c < (unsigned)bn) {
-                cp[k] = c;
-#pragma unroll
-                for (int q = 0; q < B; ++q) xp[k][q] = x[(int64_t)c*B + q];
-            } else {
-                bad = true;
-            }
-        }
-    }
     double arr = 0.0;
-    for (int c0 = s0; c0 < s1; c0 += CB) {
-        const int c1 = min(c0 + CB, s1);
-        const double *src = values + (int64_t)c0*B2;
-        const int ne = (c1 - c0)*B2;
-        double t[U];
+    for (int j0 = st; j0 < ed; j0 += KP) {
+        int c[KP];
+        double a[KP][B], xv[KP][B];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int e = u*64 + lane;
-            t[u] = e < ne ? __builtin_nontemporal_load(src + e) : 0.0;
-        }
+        for (int k = 0; k < KP; ++k)
+            if (j0 + k < ed) {
+                c[k] = colidx[j0 + k];
+                ucfd::ld_values<B>(values + (int64_t)(j0 + k)*B2 + r*B, a[k]);
+            }
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int e = u*64 + lane;
-            if (e < ne) sv[e] = t[u];
-        }
-        ucfd::wave_lds_sync();
-        if (act) {
-            const int ja = max(st, c0), jb = min(ed, c1);
-#pragma unroll
-            for (int k = 0; k < KP; ++k) {
-                const int j = st + k;
-                if (j >= ja && j < jb && cp[k] >= 0) {
-                    const double *blk = sv + (j - c0)*B2 + r*B;
-                    double v = 0.0;
-#pragma unroll
-                    for (int q = 0; q < B; ++q) v += blk[q]*xp[k][q];
-                    arr += v;
+        for (int k = 0; k < KP; ++k)
+            if (j0 + k < ed) {
+                if ((unsigned)c[k] >= (unsigned)bn) {
+                    bad = true;
+                    c[k] = -1;
+                } else {
+                    ucfd::ld_values<B>(x + (int64_t)c[k]*B, xv[k]);
                 }
             }
-            for (int j = max(ja, st + KP); j < jb; ++j) {
-                const int c = colidx[j];
-                if ((unsigned)c >= (unsigned)bn) {
-                    bad = true;
-                    continue;
-                }
-                const double *blk = sv + (j - c0)*B2 + r*B;
-                double xq[B];
 #pragma unroll
-                for (int q = 0; q < B; ++q) xq[q] = x[(int64_t)c*B + q];
+        for (int k = 0; k < KP; ++k)
+            if (j0 + k < ed && c[k] >= 0) {
                 double v = 0.0;
 #pragma unroll
-                for (int q = 0; q < B; ++q) v += blk[q]*xq[q];
+                for (int q = 0; q < B; ++q) v += a[k][q]*xv[k][q];
                 arr += v;
             }
-        }
-        ucfd::wave_lds_sync();
     }
-    if (act) {
-        const int64_t o = (int64_t)i*B + r;
-        y[o] = alpha*arr + beta*y[o];
-    }
+    const int64_t o = (int64_t)i*B + r;
+    y[o] = alpha*arr + beta*y[o];
     if (bad) ucfd::raise(flag, UCFD_KFLAG_INDEX);
 }
 
@@ -538,96 +494,44 @@ __global__ __launch_bounds__(KB) void k_sweep32(int base, int cnt, const int *__
 // of k_sweep64 / k_sweep32 above; the group then exchanges its B sums with
 // lane shuffles and every lane runs the row's diagonal solve (bit-identical
 // to the thread-per-row kernels).  K selects the FP64 sweep kind (SW_LUSGS
-// or SW_BILU; the mixed form is LU-SGS only).  When the wave's blocks fit
-// the cap words of LDS the launch provides (sized from the level's largest
-// wave) they are staged through LDS (per row, contiguous loads); otherwise
-// the lanes read them from HBM directly.  The rows' LU blocks are read from
-// HBM by the row's lanes (staging them costs LDS, which limits the waves per
-// SIMD).
-template <int B, bool UPPER, bool F32, bool STAGED, int K>
-__device__ __forceinline__ void bsgs_rows(int r, int g, bool act, int i, int j0, int n, int off,
-                                          const int *__restrict__ colidx,
-                                          const typename std::conditional<F32, float, double>::type
-                                              *blocks,
-                                          const double *lu_src, float *x32, double *b)
+// or SW_BILU; the mixed form is LU-SGS only).  Blocks, neighbour rows and the LU
+// block are read in the widest loads that cover them, the LU block with the
+// row's first indices (it depends on nothing else) and KP blocks together, so a
+// row of up to KP blocks is three round trips: indices, blocks and column
+// indices, neighbour rows.  One apply (FP32 products / FP64 / block ILU), blocks
+// staged through LDS -> this: 4.9K hex rows 22/21/18 -> 14/14/13 us, 64K
+// 40.6/35.0/29.3 -> 24.5/29.7/24.8, 384K tet rows, 4 colours, 117/150/133 ->
+// 105/129/111, 1M, 2 colours, 222/305/265 -> 208/286/238; 7x7 blocks, 384K rows,
+// 186/243/201 -> 154/215/171.
+//
+// The LU block: from 5x5 on each lane reads its own row and the group exchanges
+// the rows by shuffles after the sums (every lane holding the whole block from
+// the start: 384K rows 106/135/115 -> 105/129/111 us, 1M 220/300/244 ->
+// 208/286/238, 7x7 173/228/178 -> 154/215/171); smaller blocks are read whole
+// (4x4: 51/67/57 against 53/66/57).
+template <int B> constexpr bool lu_rows() { return B >= 5; }
+
+template <int B> __device__ __forceinline__ void ld_lu(const double *p, int r, double *lu)
 {
-    using T = typename std::conditional<F32, float, double>::type;
-    constexpr int B2 = B*B, KP = 5;
-    static_assert(K == SW_LUSGS || (K == SW_BILU && !F32), "sweep kind");
-    // accumulate with the sign of the reference: LU-SGS adds the upper
-    // products and applies D^-1 to the sum, the others subtract from x_i
-    constexpr bool ADD = UPPER && K == SW_LUSGS;
-    // column x rows of the first KP blocks
-    T xp[KP][B];
+    if (lu_rows<B>()) ucfd::ld_values<B>(p + r*B, lu);   // lu[0 .. B-1]: row r
+    else ucfd::ld_values<B*B>(p, lu);
+}
+
+// the whole block in every lane of group g (all lanes of the wave take part)
+template <int B> __device__ __forceinline__ void share_lu(int g, double *lu)
+{
+    if (!lu_rows<B>()) return;
+    double row[B];
 #pragma unroll
-    for (int k = 0; k < KP; ++k)
-        if (k < n) {
-            const int c = colidx[j0 + k];
+    for (int c = 0; c < B; ++c) row[c] = lu[c];
 #pragma unroll
-            for (int q = 0; q < B; ++q)
-                xp[k][q] = F32 ? (T)x32[(int64_t)c*B + q] : (T)b[(int64_t)c*B + q];
-        }
-    T acc = T(0);
-    double a = 0.0;
-    if (!F32 && !ADD && act) a = b[(int64_t)i*B + r];
+    for (int rr = 0; rr < B; ++rr)
 #pragma unroll
-    for (int k = 0; k < KP; ++k)
-        if (k < n) {
-            const T *blk = blocks + (STAGED ? (int64_t)(off + k)*B2 : (int64_t)(j0 + k)*B2) + r*B;
-            T v = T(0);
-#pragma unroll
-            for (int q = 0; q < B; ++q) v += blk[q]*xp[k][q];
-            if (F32) acc += v;
-            else if (ADD) a += (double)v;
-            else a -= (double)v;
-        }
-    for (int k = KP; k < n; ++k) {
-        const int c = colidx[j0 + k];
-        const T *blk = blocks + (STAGED ? (int64_t)(off + k)*B2 : (int64_t)(j0 + k)*B2) + r*B;
-        T xq[B];
-#pragma unroll
-        for (int q = 0; q < B; ++q) xq[q] = F32 ? (T)x32[(int64_t)c*B + q] : (T)b[(int64_t)c*B + q];
-        T v = T(0);
-#pragma unroll
-        for (int q = 0; q < B; ++q) v += blk[q]*xq[q];
-        if (F32) acc += v;
-        else if (ADD) a += (double)v;
-        else a -= (double)v;
-    }
-    if (K == SW_BILU && !UPPER) {
-        if (act) b[(int64_t)i*B + r] = a;
-        return;
-    }
-    if (F32) {
-        if (UPPER) a = (double)acc;
-        else if (act) a = b[(int64_t)i*B + r] - (double)acc;
-    }
-    // the group's B sums, then the diagonal solve in every lane of the group
-    double arr[B], lu[B2];
-#pragma unroll
-    for (int k = 0; k < B; ++k) arr[k] = __shfl(a, g*B + k, 64);
-    if (!act) return;
-#pragma unroll
-    for (int q = 0; q < B2; ++q) lu[q] = lu_src[q];
-    ucfd::lusub<B>(lu, arr);
-    const int64_t o = (int64_t)i*B + r;
-    if (F32) {
-        if (UPPER) {
-            const double v = (double)x32[o] - arr[r];
-            x32[o] = (float)v;
-            b[o] = v;
-        } else {
-            x32[o] = (float)arr[r];
-        }
-    } else {
-        if (ADD) b[o] -= arr[r];
-        else b[o] = arr[r];
-    }
+        for (int c = 0; c < B; ++c) lu[rr*B + c] = __shfl(row[c], g*B + rr, 64);
 }
 
 template <int B, bool UPPER, bool F32, int K>
-__global__ __launch_bounds__(64) void k_bsgs_w(int base, int cnt, int cap,
-                                               const int *__restrict__ rowptr,
+__global__ __launch_bounds__(64) void k_bsgs_w(int base, int cnt, const int *__restrict__ rowptr,
                                                const int *__restrict__ colidx,
                                                const int *__restrict__ diagslots,
                                                const typename std::conditional<F32, float,
@@ -637,58 +541,87 @@ __global__ __launch_bounds__(64) void k_bsgs_w(int base, int cnt, int cap,
                                                double *b)
 {
     using T = typename std::conditional<F32, float, double>::type;
-    constexpr int B2 = B*B, G = 64/B, PER = (5*B2 + 63)/64;
-    // dynamic LDS: cap staged block words (the rows' LU blocks are read from
-    // HBM by the row's lanes)
-    extern __shared__ __align__(16) unsigned char kdyn[];
-    T *sv = (T *)kdyn;
+    static_assert(K == SW_LUSGS || (K == SW_BILU && !F32), "sweep kind");
+    constexpr int B2 = B*B, G = 64/B, KP = 4;
+    // LU-SGS adds the upper products and applies D^-1 to the sum, the others
+    // subtract from x_i; the lower ILU sweep has no diagonal solve
+    constexpr bool ADD = UPPER && K == SW_LUSGS, SOLVE = K != SW_BILU || UPPER;
     const int lane = threadIdx.x;
     const int t0 = ucfd::wave_xcd_index()*G;
     if (t0 >= cnt) return;
     const int g = lane/B, r = lane%B;
     const int i = base + t0 + g;
     const bool act = g < G && t0 + g < cnt;
-    int j0 = 0, n = 0;
+    const int64_t o = (int64_t)i*B + r;
+    int j0 = 0, j1 = 0;
+    double lu[B2] = {}, own = 0.0;
+    float own32 = 0.0f;
     if (act) {
         const int dd = diagslots[i];
         j0 = UPPER ? dd + 1 : rowptr[i];
-        n = (UPPER ? rowptr[i + 1] : dd) - j0;
+        j1 = UPPER ? rowptr[i + 1] : dd;
+        if (SOLVE) ld_lu<B>(dv + (int64_t)i*B2, r, lu);
+        if (F32 && UPPER) own32 = x32[o];
+        else own = b[o];
     }
-    // block offset of each row in the staged list; the total decides the path
-    const int lead = (act && r == 0) ? n : 0;
-    const int ex = ucfd::wave_excl_scan(lead);
-    const int total = __shfl(ex + lead, 63, 64);
-    const int off = __shfl(ex, g*B < 64 ? g*B : 0, 64);
-    if (total*B2 > cap) {
-        bsgs_rows<B, UPPER, F32, false, K>(r, g, act, i, j0, n, 0, colidx, vals,
-                                        dv + (int64_t)i*B2, x32, b);
+    T acc = T(0);
+    double a = !F32 && !ADD ? own : 0.0;
+    for (int jj = j0; jj < j1; jj += KP) {
+        int c[KP];
+        T blk[KP][B], xc[KP][B];
+#pragma unroll
+        for (int k = 0; k < KP; ++k)
+            if (jj + k < j1) {
+                c[k] = colidx[jj + k];
+                ucfd::ld_values<B>(vals + (int64_t)(jj + k)*B2 + r*B, blk[k]);
+            }
+#pragma unroll
+        for (int k = 0; k < KP; ++k)
+            if (jj + k < j1) {
+                if constexpr (F32) ucfd::ld_values<B>(x32 + (int64_t)c[k]*B, xc[k]);
+                else ucfd::ld_values<B>(b + (int64_t)c[k]*B, xc[k]);
+            }
+#pragma unroll
+        for (int k = 0; k < KP; ++k)
+            if (jj + k < j1) {
+                T v = T(0);
+#pragma unroll
+                for (int q = 0; q < B; ++q) v += blk[k][q]*xc[k][q];
+                if (F32) acc += v;
+                else if (ADD) a += (double)v;
+                else a -= (double)v;
+            }
+    }
+    if (!SOLVE) {
+        if (act) b[o] = a;
         return;
     }
-    // stage: every row's blocks [j0, j0+n) to sv[off*B2 ...]
-    T t[G][PER];
-#pragma unroll
-    for (int gg = 0; gg < G; ++gg) {
-        const int jg = __shfl(j0, gg*B, 64), ng = __shfl(n, gg*B, 64)*B2;
-#pragma unroll
-        for (int k = 0; k < PER; ++k) {
-            const int e = k*64 + lane;
-            t[gg][k] = e < ng ? __builtin_nontemporal_load(vals + (int64_t)jg*B2 + e) : T(0);
-        }
+    if (F32) {
+        if (UPPER) a = (double)acc;
+        else if (act) a = own - (double)acc;
     }
+    // the group's B sums, then the diagonal solve in every lane of the group
+    double arr[B];
 #pragma unroll
-    for (int gg = 0; gg < G; ++gg) {
-        const int jg = __shfl(j0, gg*B, 64), ng = __shfl(n, gg*B, 64)*B2;
-        const int og = __shfl(ex, gg*B, 64)*B2;
+    for (int k = 0; k < B; ++k) arr[k] = __shfl(a, g*B + k, 64);
+    share_lu<B>(g, lu);
+    if (!act) return;
+    ucfd::lusub<B>(lu, arr);
+    double mine = arr[0];
 #pragma unroll
-        for (int k = 0; k < PER; ++k) {
-            const int e = k*64 + lane;
-            if (e < ng) sv[og + e] = t[gg][k];
+    for (int k = 1; k < B; ++k)
+        if (r == k) mine = arr[k];
+    if (F32) {
+        if (UPPER) {
+            const double v = (double)own32 - mine;
+            x32[o] = (float)v;
+            b[o] = v;
+        } else {
+            x32[o] = (float)mine;
         }
-        for (int e = PER*64 + lane; e < ng; e += 64) sv[og + e] = vals[(int64_t)jg*B2 + e];
+    } else {
+        b[o] = ADD ? own - mine : mine;
     }
-    ucfd::wave_lds_sync();
-    bsgs_rows<B, UPPER, F32, true, K>(r, g, act, i, j0, n, off, colidx, sv,
-                                      dv + (int64_t)(act ? i : base + t0)*B2, x32, b);
 }
 
 // A level whose rows take no block in the sweep's direction (the first
@@ -713,12 +646,10 @@ __global__ __launch_bounds__(64) void k_bsgs_diag(int base, int cnt, const doubl
     const int i = base + t0 + g;
     const bool act = g < G && t0 + g < cnt;
     const int64_t o = (int64_t)i*B + r;
-    double lu[B2];
-    double bo = 0.0;
+    double lu[B2] = {}, bo = 0.0;
     float xo = 0.f;
     if (act) {
-#pragma unroll
-        for (int q = 0; q < B2; ++q) lu[q] = dv[(int64_t)i*B2 + q];
+        ld_lu<B>(dv + (int64_t)i*B2, r, lu);
         if (!ADD) bo = b[o];
         if (F32 && UPPER) xo = x32[o];
     }
@@ -731,19 +662,24 @@ __global__ __launch_bounds__(64) void k_bsgs_diag(int base, int cnt, const doubl
     double arr[B];
 #pragma unroll
     for (int k = 0; k < B; ++k) arr[k] = __shfl(a, g*B + k, 64);
+    share_lu<B>(g, lu);
     if (!act) return;
     ucfd::lusub<B>(lu, arr);
+    double mine = arr[0];
+#pragma unroll
+    for (int k = 1; k < B; ++k)
+        if (r == k) mine = arr[k];
     if (F32) {
         if (UPPER) {
-            const double v = (double)xo - arr[r];
+            const double v = (double)xo - mine;
             x32[o] = (float)v;
             b[o] = v;
         } else {
-            x32[o] = (float)arr[r];
+            x32[o] = (float)mine;
         }
     } else {
-        if (ADD) b[o] = b[o] - arr[r];
-        else b[o] = arr[r];
+        if (ADD) b[o] = b[o] - mine;
+        else b[o] = mine;
     }
 }
 
@@ -1199,27 +1135,15 @@ template <int B> struct IluL {
     }
 };
 
-// LDS words for the staged blocks of a wave-staged sweep launch
-template <int B, typename T> int stage_cap(int maxw)
-{
-    const int full = KSTAGE*8/(int)sizeof(T);
-    return maxw < 0 ? full : (maxw*B*B < full ? maxw*B*B : full);
-}
-
-template <int B, typename T> size_t stage_bytes(int cap)
-{
-    return (size_t)(cap > 0 ? cap : 1)*sizeof(T);
-}
-
 template <int B, int K>
 int sweep64_launch(hipStream_t s, int upper, int base, int cnt, const int *ord, const int *rp,
                    const int *ci, const int *ds, const double *v, const double *dv, double *b,
-                   int maxw)
+                   bool empty)
 {
     if constexpr (B > 1) {
         if (!ord) {
             const dim3 g((cnt + 64/B - 1)/(64/B));
-            if (maxw == 0 && K != SW_ILU) {
+            if (empty && K != SW_ILU) {
                 // no row of the level takes a block in this direction
                 if (K == SW_BILU && !upper) return UCFD_OK;
                 if (upper)
@@ -1230,14 +1154,12 @@ int sweep64_launch(hipStream_t s, int upper, int base, int cnt, const int *ord, 
                                        cnt, dv, nullptr, b);
                 return ok();
             }
-            const int cap = stage_cap<B, double>(maxw);
-            const size_t lds = stage_bytes<B, double>(cap);
             if (upper)
-                hipLaunchKernelGGL((k_bsgs_w<B, true, false, K>), g, dim3(64), lds, s, base, cnt,
-                                   cap, rp, ci, ds, v, dv, nullptr, b);
+                hipLaunchKernelGGL((k_bsgs_w<B, true, false, K>), g, dim3(64), 0, s, base, cnt, rp,
+                                   ci, ds, v, dv, nullptr, b);
             else
-                hipLaunchKernelGGL((k_bsgs_w<B, false, false, K>), g, dim3(64), lds, s, base, cnt,
-                                   cap, rp, ci, ds, v, dv, nullptr, b);
+                hipLaunchKernelGGL((k_bsgs_w<B, false, false, K>), g, dim3(64), 0, s, base, cnt, rp,
+                                   ci, ds, v, dv, nullptr, b);
             return ok();
         }
     }
@@ -1254,16 +1176,16 @@ int sweep64_launch(hipStream_t s, int upper, int base, int cnt, const int *ord, 
 template <int B> struct Sw64L {
     static int run(hipStream_t s, int kind, int upper, int base, int cnt, const int *ord,
                    const int *rp, const int *ci, const int *ds, const double *v, const double *dv,
-                   double *b, int maxw)
+                   double *b, bool empty)
     {
         switch (kind) {
         case SW_LUSGS:
-            return sweep64_launch<B, SW_LUSGS>(s, upper, base, cnt, ord, rp, ci, ds, v, dv, b, maxw);
+            return sweep64_launch<B, SW_LUSGS>(s, upper, base, cnt, ord, rp, ci, ds, v, dv, b, empty);
         case SW_BILU:
-            return sweep64_launch<B, SW_BILU>(s, upper, base, cnt, ord, rp, ci, ds, v, dv, b, maxw);
+            return sweep64_launch<B, SW_BILU>(s, upper, base, cnt, ord, rp, ci, ds, v, dv, b, empty);
         case SW_ILU:
             if (B != 1) return UCFD_ERR_ARG;
-            return sweep64_launch<1, SW_ILU>(s, upper, base, cnt, ord, rp, ci, ds, v, dv, b, maxw);
+            return sweep64_launch<1, SW_ILU>(s, upper, base, cnt, ord, rp, ci, ds, v, dv, b, empty);
         default:
             return UCFD_ERR_ARG;
         }
@@ -1273,11 +1195,11 @@ template <int B> struct Sw64L {
 template <int B> struct Sw32L {
     static int run(hipStream_t s, int upper, int base, int cnt, const int *ord, const int *rp,
                    const int *ci, const int *ds, const float *v, const double *dv, float *x32,
-                   double *b, int maxw)
+                   double *b, bool empty)
     {
         if (B > 1 && !ord) {
             const dim3 g((cnt + 64/B - 1)/(64/B));
-            if (maxw == 0) {
+            if (empty) {
                 // no row of the level takes a block in this direction
                 if (upper)
                     hipLaunchKernelGGL((k_bsgs_diag<B, true, true, SW_LUSGS>), g, dim3(64), 0, s,
@@ -1287,14 +1209,12 @@ template <int B> struct Sw32L {
                                        base, cnt, dv, x32, b);
                 return ok();
             }
-            const int cap = stage_cap<B, float>(maxw);
-            const size_t lds = stage_bytes<B, float>(cap);
             if (upper)
-                hipLaunchKernelGGL((k_bsgs_w<B, true, true, SW_LUSGS>), g, dim3(64), lds, s, base,
-                                   cnt, cap, rp, ci, ds, v, dv, x32, b);
+                hipLaunchKernelGGL((k_bsgs_w<B, true, true, SW_LUSGS>), g, dim3(64), 0, s, base, cnt,
+                                   rp, ci, ds, v, dv, x32, b);
             else
-                hipLaunchKernelGGL((k_bsgs_w<B, false, true, SW_LUSGS>), g, dim3(64), lds, s, base,
-                                   cnt, cap, rp, ci, ds, v, dv, x32, b);
+                hipLaunchKernelGGL((k_bsgs_w<B, false, true, SW_LUSGS>), g, dim3(64), 0, s, base,
+                                   cnt, rp, ci, ds, v, dv, x32, b);
             return ok();
         }
         const dim3 g((cnt + KB - 1)/KB);
@@ -1349,21 +1269,21 @@ int kry_ilu_factor(hipStream_t s, int scalar, int rows, int blk, int base, int c
 
 int kry_bsgs_sweep64(hipStream_t s, int kind, int upper, int blk, int base, int cnt,
                      const int *order, const int *rowptr, const int *colidx, const int *diagslots,
-                     const double *values, const double *diagvalues, double *b, int maxw)
+                     const double *values, const double *diagvalues, double *b, bool empty)
 {
     if (cnt <= 0) return UCFD_OK;
     return by_block<Sw64L>(blk, s, kind, upper, base, cnt, order, rowptr, colidx, diagslots,
-                           values, diagvalues, b, maxw);
+                           values, diagvalues, b, empty);
 }
 
 int kry_bsgs_sweep32(hipStream_t s, int upper, int blk, int base, int cnt, const int *order,
                      const int *rowptr, const int *colidx, const int *diagslots,
                      const float *vals32, const double *diagvalues, float *x32, double *b,
-                     int maxw)
+                     bool empty)
 {
     if (cnt <= 0) return UCFD_OK;
     return by_block<Sw32L>(blk, s, upper, base, cnt, order, rowptr, colidx, diagslots, vals32,
-                           diagvalues, x32, b, maxw);
+                           diagvalues, x32, b, empty);
 }
 
 namespace {

@@ -2,15 +2,12 @@
 // block LU-SGS apply, the FlowSys block sweeps).
 //
 // One wave (64 lanes, one wave per workgroup) serves G = 64 / B block rows;
-// lane (g, r) = (lane / B, lane % B) owns scalar row r of block row g.  The
-// wave first copies the blocks its rows use from HBM into LDS with loads in
-// which consecutive lanes read consecutive words (a block row's blocks are
-// contiguous in memory), then every lane reads its own block row's entries
-// from LDS.  A block is row-major, so one lane's scalar row is B contiguous
-// values: a thread-per-block-row kernel makes each lane stream its own 8*B*B
-// bytes, and each wave-wide load touches up to 64 different cache lines;
-// here each load touches 4-5.  Each lane keeps the summation order of its
-// scalar row, so results equal those of a thread-per-row kernel bit for bit.
+// lane (g, r) = (lane / B, lane % B) owns scalar row r of block row g.  A block
+// is row-major, so one lane's scalar row is B contiguous values and the lanes of
+// a group cover the block: with loads of several values each, a wave reads its
+// rows' k-th blocks in two or three instructions.  Each lane keeps the summation
+// order of its scalar row, so results equal those of a thread-per-row kernel bit
+// for bit.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -26,17 +23,43 @@ __device__ __forceinline__ void wave_lds_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
-// exclusive prefix sum of v over the 64 lanes of the wave
-__device__ __forceinline__ int wave_excl_scan(int v)
+// N consecutive values at p (aligned to one value) in the widest loads that
+// cover them
+typedef double wr_d2 __attribute__((ext_vector_type(2), aligned(8)));
+typedef float wr_f4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float wr_f2 __attribute__((ext_vector_type(2), aligned(4)));
+
+template <int N> __device__ __forceinline__ void ld_values(const double *p, double *v)
 {
-    const int lane = threadIdx.x & 63;
-    int x = v;
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
+    for (int q = 0; q + 2 <= N; q += 2) {
+        const wr_d2 *a = (const wr_d2 *)(p + q);
+        const wr_d2 t = *a;
+        v[q] = t.x;
+        v[q + 1] = t.y;
     }
-    return x - v;
+    if (N % 2) v[N - 1] = p[N - 1];
+}
+
+template <int N> __device__ __forceinline__ void ld_values(const float *p, float *v)
+{
+#pragma unroll
+    for (int q = 0; q + 4 <= N; q += 4) {
+        const wr_f4 *a = (const wr_f4 *)(p + q);
+        const wr_f4 t = *a;
+        v[q] = t.x;
+        v[q + 1] = t.y;
+        v[q + 2] = t.z;
+        v[q + 3] = t.w;
+    }
+    constexpr int R = N/4*4;
+    if (N - R >= 2) {
+        const wr_f2 *a = (const wr_f2 *)(p + R);
+        const wr_f2 t = *a;
+        v[R] = t.x;
+        v[R + 1] = t.y;
+    }
+    if (N % 2) v[N - 1] = p[N - 1];
 }
 
 // one-wave workgroups remapped so that each XCD owns runs of 32 consecutive
