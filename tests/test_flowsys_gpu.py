@@ -455,3 +455,78 @@ def test_lusgs_two_element_types(colored):
     assert sorted(got) == sorted(ref)
     for k, v in ref.items():
         assert np.array_equal(np.asarray(got[k]).reshape(v.shape), v), k
+
+
+# ------------------------------------------------------ edges of the wave kernels
+def layered_system(sizes, deg, nfv, nt, seed):
+    """A colour-ordered rank: len(sizes) ranges of cells, each cell with deg faces
+    to random cells of every later range (so the cells have any number of faces,
+    some of the last range none).  Elements map to the cells at random."""
+    from ucfd_sparse_amd.mesh import FlowSysMesh
+    rng = np.random.default_rng(seed)
+    start = np.concatenate([[0], np.cumsum(sizes)])
+    N = int(start[-1])
+    faces = []
+    for a in range(len(sizes)):
+        for b in range(a + 1, len(sizes)):
+            for i in range(start[a], start[a + 1]):
+                for j in rng.choice(np.arange(start[b], start[b + 1]),
+                                    size=min(deg, sizes[b]), replace=False):
+                    faces.append((i, int(j)))
+    rows = [[] for _ in range(N)]
+    for f, (i, j) in enumerate(faces):
+        rows[i].append((j, f, 1))
+        rows[j].append((i, f, -1))
+    pos = [x for r in rows for x in r]
+    rowptr = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    colidx, slots = (np.array([x[k] for x in pos], np.int32) for k in (0, 1))
+    sides = np.array([x[2] for x in pos], np.int8)
+    F, nvars, ND = len(faces), nfv + nt, 2 if nfv == 4 else 3
+    up = rng.uniform(0.1, 0.3, (nvars, N))
+    up[0] += 1.0
+    up[nfv - 1] += 2.5
+    el = {"cell_ids": rng.permutation(N).astype(np.int32), "uptsb": up,
+          "rhs": rng.normal(0.0, 1e-3, (nvars, N)), "dt": rng.uniform(0.5, 1.0, N),
+          "dsrc": rng.uniform(0.0, 1.0, (nvars, N)), "vol": rng.uniform(0.5, 2.0, N)}
+    fs = FlowSysMesh(N, F, rowptr, colidx, slots, sides, rng.uniform(0.5, 1.0, F),
+                     rng.normal(0.0, 1.0, (ND, F)), rng.uniform(0.5, 1.0, N),
+                     rng.normal(0.0, 0.02, (2, nfv, nfv, F)))
+    tj = rng.normal(0.0, 0.02, (2, nt, nt, F)) if nt else None
+    return fs, tj, el, rng.uniform(0.5, 2.0, F), rng.uniform(0.2, 1.0, F)
+
+
+@pytest.mark.parametrize("sizes, deg, nfv, nt", [((1, 63, 1), 1, 4, 0), ((63, 1, 64), 4, 4, 1),
+                                                 ((64, 65, 66), 8, 5, 0),
+                                                 ((129, 64, 66), 9, 5, 1),
+                                                 ((64, 127, 65), 20, 5, 2),
+                                                 ((30, 200, 3), 3, 5, 3),
+                                                 ((65, 63, 130), 30, 5, 4)])
+def test_wave_kernels_at_range_and_chunk_edges(sizes, deg, nfv, nt):
+    """Ranges of 1, 63, 64, 65, ... cells and more positions a wave of 64 cells
+    than it handles at a time, 4 to 9 variables: the scalar method's Prepare,
+    sweeps and Update and the block method's SubResidual and Update, bit for bit
+    against the oracle."""
+    from ucfd_sparse_amd import flowsys as FS
+    fs, tj, el, fspr, tfspr = layered_system(sizes, deg, nfv, nt, seed=sum(sizes) + deg)
+    most = max(int(fs.rowptr[min(i + 64, fs.nlocal)] - fs.rowptr[i]) for i in range(fs.nlocal))
+    say(f"ranges {sizes}, up to {most} positions per 64 cells, {nfv}+{nt} variables")
+    ref = O.flowsys_lusgs_run(fs, fspr, tfspr, el, nfv + nt, nfv, a0=0.2, turb_factor=1.7,
+                              kappa=1.1, iterations=2)
+    fsd, tjd, eld = on_device(fs, tj if nt else np.zeros(1), el)
+    S = FS.FlowSysLUSGS(fsd, nfv + nt, nfv, torch.from_numpy(fspr).cuda(),
+                        torch.from_numpy(tfspr).cuda(), ndims=2 if nfv == 4 else 3)
+    S.set_element(0, {k: v.clone() for k, v in eld.items()})
+    got = FS.run_lusgs(S, a0=0.2, turb_factor=1.7, kappa=1.1, iterations=2)
+    S.close()
+    for k, v in ref.items():
+        assert np.array_equal(np.asarray(got[k]).reshape(v.shape), v), k
+    if nt > 2:
+        return
+    ref = O.flowsys_run(fs, tj, el, nfv + nt, nfv, kind="sa" if nt == 1 else "kwsst",
+                        iterations=2)
+    S = FS.FlowSys(fsd, nfv + nt, nfv, ndims=2 if nfv == 4 else 3, tjmat=tjd if nt else None)
+    S.set_element(0, eld)
+    got = FS.run(S, kind="sa" if nt == 1 else "kwsst", iterations=2)
+    S.close()
+    for k, v in ref.items():
+        assert np.array_equal(np.asarray(got[k]).reshape(v.shape), v), k
