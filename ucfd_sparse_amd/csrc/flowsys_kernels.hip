@@ -978,15 +978,20 @@ __global__ __launch_bounds__(FB) void k_lsweep(int base, int cnt, const int *__r
 // cell's records in position order (coalesced) instead of gathering five
 // values through the slot index; every stored value is the product the
 // sweep itself forms (lusgs.c:185-195), so the results do not change by a
-// bit.  A wave's 64 cells own one contiguous range of positions: the
-// records of its first LPCAP positions are staged in LDS and written out
-// with consecutive lanes on consecutive records (one lane per cell would
-// write 32-byte pieces at the position stride, partial cache lines that
-// measured 2.15x the record bytes in HBM writes); positions beyond LPCAP
-// (cells with many faces) are written directly.
-constexpr int LPCAP = 256;   // staged positions per wave (64 tets)
+// bit.  A wave's 64 cells own one contiguous range of positions, which its
+// lanes take a position each: slots, sides and the records are met with
+// consecutive lanes on consecutive positions, the gathers of LPB positions a lane
+// are issued at once whatever the cells' face counts, and the cells sum their
+// positions' terms from LDS in position order.  Bound by the latency of slot ->
+// gathers.  A thread per cell with
+// the records exchanged in LDS took hexes beyond their first four faces one by
+// one: 166K hexes 35.5 -> 25.8 us, 343K hexes 82.7 -> 58.3, 356K tets 32.5 ->
+// 31.8, 1.3M tets 153 -> 143; without records (turbulence) 11.4 -> 10.6, 24.2 ->
+// 19.1, 12.8 -> 12.6, 39.0 -> 37.8.
+constexpr int LPCAP = 512;   // positions a wave handles at a time
+constexpr int LPB = 4;       // positions of a lane whose loads are issued together
 
-template <int ND>
+template <int ND, bool GEO>
 __global__ __launch_bounds__(FB) void k_lprep_pos(int nlocal, int64_t nfaces, int nv0, int nv1,
                                                   double kappa, const int *__restrict__ rowptr,
                                                   const int *__restrict__ slots,
@@ -998,8 +1003,8 @@ __global__ __launch_bounds__(FB) void k_lprep_pos(int nlocal, int64_t nfaces, in
                                                   double *diag, double4 *__restrict__ geo,
                                                   double *__restrict__ lam)
 {
-    __shared__ double4 sgeo[FB/64][LPCAP];
-    __shared__ double slam[FB/64][LPCAP];
+    __shared__ double sterm[FB/64][LPCAP], srv[FB/64][64];
+    __shared__ unsigned char scell[FB/64][LPCAP];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int w0 = fxcd()*FB + wv*64;   // the wave's first cell
     if (w0 >= nlocal) return;
@@ -1007,73 +1012,68 @@ __global__ __launch_bounds__(FB) void k_lprep_pos(int nlocal, int64_t nfaces, in
     const bool act = r < nlocal;
     const int P0 = rowptr[w0], P1 = rowptr[min(w0 + 64, nlocal)];
     const int p0 = act ? rowptr[r] : 0, p1 = act ? rowptr[r + 1] : 0;
-    const double rv = act ? rcp_vol[r] : 0.0;
-    // the slot indices of the first LKP positions together, then all their
-    // gathers, then the face terms in position order
-    int64_t sl[LKP];
-    double lf[LKP], fa[LKP], fn[LKP][ND], side[LKP];
+    double *term = sterm[wv], *rvs = srv[wv];
+    unsigned char *cell = scell[wv];
+    rvs[lane] = act ? rcp_vol[r] : 0.0;
+    double sd = 0.0;
+    for (int c0 = P0; c0 < P1; c0 += LPCAP) {
+        const int n = min(LPCAP, P1 - c0);
+        const int q0 = max(p0, c0), q1 = min(p1, c0 + n);
+        for (int p = q0; p < q1; ++p) cell[p - c0] = (unsigned char)lane;
+        ucfd::wave_lds_sync();
+        for (int b = lane; b < n; b += 64*LPB) {
+            int64_t sl[LPB];
+            double lf[LPB], fa[LPB], fn[LPB][ND], side[LPB];
 #pragma unroll
-    for (int k = 0; k < LKP; ++k) {
-        sl[k] = 0;
-        lf[k] = fa[k] = side[k] = 0.0;
+            for (int k = 0; k < LPB; ++k)
+                if (b + k*64 < n) {
+                    sl[k] = slots[c0 + b + k*64];
+                    if (GEO) side[k] = (double)sides[c0 + b + k*64];
+                }
 #pragma unroll
-        for (int d = 0; d < ND; ++d) fn[k][d] = 0.0;
-        if (p0 + k < p1) sl[k] = slots[p0 + k];
-    }
+            for (int k = 0; k < LPB; ++k)
+                if (b + k*64 < n) {
+                    lf[k] = lambdaf[sl[k]];
+                    fa[k] = face_area[sl[k]];
+                    if (GEO)
 #pragma unroll
-    for (int k = 0; k < LKP; ++k)
-        if (p0 + k < p1) {
-            lf[k] = lambdaf[sl[k]];
-            fa[k] = face_area[sl[k]];
-            if (geo) {
-                side[k] = (double)sides[p0 + k];
+                        for (int d = 0; d < ND; ++d) fn[k][d] = face_normal[sl[k] + (int64_t)d*nfaces];
+                }
 #pragma unroll
-                for (int d = 0; d < ND; ++d) fn[k][d] = face_normal[sl[k] + (int64_t)d*nfaces];
+            for (int k = 0; k < LPB; ++k) {
+                const int j = b + k*64;
+                if (j >= n) continue;
+                const double rv = rvs[cell[j]];
+                term[j] = 0.5*(lf[k]*kappa)*fa[k]*rv;
+                lam[c0 + j] = lf[k];
+                if (GEO) {
+                    double g[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                    for (int d = 0; d < ND; ++d) g[d] = side[k]*fn[k][d];
+                    g[ND] = fa[k]*rv;
+                    geo[c0 + j] = double4{g[0], g[1], g[2], g[3]};
+                }
             }
         }
-    double sd = 0.0;
-    auto face = [&](int p, double lfk, double fak, const double *fnk, double sidek) {
-        sd += 0.5*(lfk*kappa)*fak*rv;
-        const int j = p - P0;
-        if (geo) {
-            double g[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int d = 0; d < ND; ++d) g[d] = sidek*fnk[d];
-            g[ND] = fak*rv;
-            const double4 gv = double4{g[0], g[1], g[2], g[3]};
-            if (j < LPCAP) sgeo[wv][j] = gv;
-            else geo[p] = gv;
-        }
-        if (j < LPCAP) slam[wv][j] = lfk;
-        else lam[p] = lfk;
-    };
-#pragma unroll
-    for (int k = 0; k < LKP; ++k)
-        if (p0 + k < p1) face(p0 + k, lf[k], fa[k], fn[k], side[k]);
-    for (int p = p0 + LKP; p < p1; ++p) {
-        const int64_t s2 = slots[p];
-        double f2[ND] = {};
-        double sd2 = 0.0;
-        if (geo) {
-            sd2 = (double)sides[p];
-#pragma unroll
-            for (int d = 0; d < ND; ++d) f2[d] = face_normal[s2 + (int64_t)d*nfaces];
-        }
-        face(p, lambdaf[s2], face_area[s2], f2, sd2);
+        ucfd::wave_lds_sync();
+        for (int p = q0; p < q1; ++p) sd += term[p - c0];
+        ucfd::wave_lds_sync();
     }
-    if (act)
-        for (int k = nv0; k < nv1; ++k) diag[r + (int64_t)k*nlocal] += sd;
-    ucfd::wave_lds_sync();
-    const int nst = min(P1 - P0, LPCAP);
-    for (int j = lane; j < nst; j += 64) {
-        if (geo) geo[P0 + j] = sgeo[wv][j];
-        lam[P0 + j] = slam[wv][j];
+    if (!act) return;
+    for (int k0 = nv0; k0 < nv1; k0 += 4) {
+        double d[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (k0 + k < nv1) d[k] = diag[r + (int64_t)(k0 + k)*nlocal];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (k0 + k < nv1) diag[r + (int64_t)(k0 + k)*nlocal] = d[k] + sd;
     }
 }
 
-// k_lsweep reading the per-position records of k_lprep_pos
+// k_lsweep reading the per-position records of k_lprep_pos, for a list of cells
 template <int ND, int NT, bool UPPER>
-__global__ __launch_bounds__(FB) void k_lsweep_p(int base, int cnt, const int *__restrict__ order,
+__global__ __launch_bounds__(FB) void k_lsweep_p(const int *__restrict__ cells, int cnt,
                                                  int nfvars, double kappa, int nlocal,
                                                  const int *__restrict__ rowptr,
                                                  const int *__restrict__ colidx,
@@ -1144,6 +1144,103 @@ __global__ __launch_bounds__(FB) void k_lsweep_p(int base, int cnt, const int *_
         const int64_t l = r + (int64_t)(k + nv0)*nlocal;
         if (UPPER) du[l] = odu[k] - (0.5*df[k]/odg[k]);
         else du[l] = (odu[k] - 0.5*df[k])/odg[k];
+    }
+}
+
+// The same for a contiguous range of cells (every level of a renumbered mesh)
+// with a thread per position: a workgroup serves 64 cells with LSW waves, which
+// form the face terms of their positions (any number, LPCAP at a time) side by
+// side; thread (cell, k) then sums row k of its cell over the positions in order
+// from LDS (a position not taken adds +0.0 to a sum that is never -0.0: the same
+// bits).  Bound by the latency of the chain colidx -> u, du of the neighbour: a
+// thread per cell holds LKP faces at once in 173 VGPRs (2 waves a SIMD) and takes
+// the fifth and sixth of a hex after them.  A lower and an upper sweep of 5 flow
+// / 1 turbulence row: 4.9K hexes 24.1 -> 16.8 / 17.2 -> 16.4 us, 166K hexes
+// 40.9 -> 33.4 / 29.8 -> 20.6, 356K tets 47.8 -> 43.7 / 31.2 -> 24.3, 1.3M tets
+// 169.6 -> 170.4 / 112.8 -> 89.5.
+constexpr int LSW = 4;
+
+template <int ND, int NT, bool UPPER>
+__global__ __launch_bounds__(64*LSW) void k_lsweep_w(int base, int cnt, int nfvars, double kappa,
+                                                     int nlocal, const int *__restrict__ rowptr,
+                                                     const int *__restrict__ colidx,
+                                                     const double4 *__restrict__ geo,
+                                                     const double *__restrict__ lam,
+                                                     const double *__restrict__ diag,
+                                                     const double *__restrict__ u, double *du)
+{
+    constexpr int NF = ND + 2, DNV = LFace<ND, NT>::DNV, KW = (DNV + LSW - 1)/LSW;
+    constexpr int CAP = LPCAP;
+    __shared__ double sterm[DNV][CAP];
+    __shared__ unsigned char scell[CAP];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int nv0 = NT > 0 ? nfvars : 0;
+    const int b0 = fxcd()*64, ncell = min(64, cnt - b0);
+    const int r0 = base + b0, r = r0 + lane;
+    const bool act = lane < ncell;
+    const int P0 = rowptr[r0], P1 = rowptr[r0 + ncell];
+    const int p0 = act ? rowptr[r] : 0, p1 = act ? rowptr[r + 1] : 0;
+    double odu[KW], odg[KW], df[KW];
+#pragma unroll
+    for (int q = 0; q < KW; ++q) {
+        const int k = w + q*LSW;
+        df[q] = 0.0;
+        if (k < DNV && act) {
+            const int64_t l = r + (int64_t)(k + nv0)*nlocal;
+            odu[q] = du[l];
+            odg[q] = diag[l];
+        }
+    }
+    for (int c0 = P0; c0 < P1; c0 += CAP) {
+        const int n = min(CAP, P1 - c0);
+        const int q0 = max(p0, c0), q1 = min(p1, c0 + n);
+        if (w == 0)
+            for (int p = q0; p < q1; ++p) scell[p - c0] = (unsigned char)lane;
+        __syncthreads();
+        for (int j = threadIdx.x; j < n; j += 64*LSW) {
+            const int p = c0 + j, cell = r0 + scell[j];
+            const int64_t nb = colidx[p];
+            double t[DNV];
+#pragma unroll
+            for (int k = 0; k < DNV; ++k) t[k] = 0.0;
+            if (UPPER ? nb > cell : nb < cell) {
+                LFace<ND, NT> G;
+                const double4 g = geo[p];
+                const double gv[4] = {g.x, g.y, g.z, g.w};
+#pragma unroll
+                for (int d = 0; d < ND; ++d) G.nf[d] = gv[d];
+                G.fv = gv[ND];
+                G.lam = kappa*lam[p];
+#pragma unroll
+                for (int k = 0; k < NF; ++k) G.uf[k] = u[nb + (int64_t)k*nlocal];
+#pragma unroll
+                for (int k = 0; k < DNV; ++k) G.dnb[k] = du[nb + (int64_t)(k + nv0)*nlocal];
+                if (NT > 0) {
+#pragma unroll
+                    for (int k = 0; k < DNV; ++k) G.ut[k] = u[nb + (int64_t)(nfvars + k)*nlocal];
+                }
+                lface_add<ND, NT>(G, t);
+            }
+#pragma unroll
+            for (int k = 0; k < DNV; ++k) sterm[k][j] = t[k];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < KW; ++q) {
+            const int k = w + q*LSW;
+            if (k < DNV)
+                for (int p = q0; p < q1; ++p) df[q] += sterm[k][p - c0];
+        }
+        __syncthreads();
+    }
+    if (!act) return;
+#pragma unroll
+    for (int q = 0; q < KW; ++q) {
+        const int k = w + q*LSW;
+        if (k >= DNV) continue;
+        const int64_t l = r + (int64_t)(k + nv0)*nlocal;
+        if (UPPER) du[l] = odu[q] - (0.5*df[q]/odg[q]);
+        else du[l] = (odu[q] - 0.5*df[q])/odg[q];
     }
 }
 
@@ -1479,16 +1576,17 @@ int fs_launch_lprep_pos(hipStream_t s, int ndims, int nlocal, int64_t nfaces, in
                         const double *lambdaf, double *diag, void *geo, double *lam)
 {
     if (nlocal <= 0) return UCFD_OK;
-    if (ndims == 3)
-        hipLaunchKernelGGL(k_lprep_pos<3>, grid(nlocal), dim3(FB), 0, s, nlocal, nfaces, nv0, nv1,
-                           kappa, rowptr, slots, sides, face_area, face_normal, rcp_vol, lambdaf,
-                           diag, (double4 *)geo, lam);
-    else if (ndims == 2)
-        hipLaunchKernelGGL(k_lprep_pos<2>, grid(nlocal), dim3(FB), 0, s, nlocal, nfaces, nv0, nv1,
-                           kappa, rowptr, slots, sides, face_area, face_normal, rcp_vol, lambdaf,
-                           diag, (double4 *)geo, lam);
+#define LPREP(ND, GEO) \
+    hipLaunchKernelGGL((k_lprep_pos<ND, GEO>), grid(nlocal), dim3(FB), 0, s, nlocal, nfaces, nv0, \
+                       nv1, kappa, rowptr, slots, sides, face_area, face_normal, rcp_vol, \
+                       lambdaf, diag, (double4 *)geo, lam)
+    if (ndims == 3 && geo) LPREP(3, true);
+    else if (ndims == 3) LPREP(3, false);
+    else if (ndims == 2 && geo) LPREP(2, true);
+    else if (ndims == 2) LPREP(2, false);
     else
         return UCFD_ERR_ARG;
+#undef LPREP
     return ok();
 }
 
@@ -1500,12 +1598,21 @@ int lsweep_p_nt(hipStream_t s, bool upper, int nt, int base, int cnt, const int 
                 const double4 *geo, const double *lam, const double *diag, const double *u,
                 double *du)
 {
+    // the order of a level that is not a range of cells is met a cell to a thread
+    const dim3 gw((unsigned)((cnt + 63)/64));
 #define LP(NT) do { \
-    if (upper) hipLaunchKernelGGL((k_lsweep_p<ND, NT, true>), grid(cnt), dim3(FB), 0, s, base, \
-                                  cnt, order, nfvars, kappa, nlocal, rowptr, colidx, geo, lam, \
-                                  diag, u, du); \
-    else hipLaunchKernelGGL((k_lsweep_p<ND, NT, false>), grid(cnt), dim3(FB), 0, s, base, cnt, \
-                            order, nfvars, kappa, nlocal, rowptr, colidx, geo, lam, diag, u, du); \
+    if (!order && upper) \
+        hipLaunchKernelGGL((k_lsweep_w<ND, NT, true>), gw, dim3(64*LSW), 0, s, base, cnt, nfvars, \
+                           kappa, nlocal, rowptr, colidx, geo, lam, diag, u, du); \
+    else if (!order) \
+        hipLaunchKernelGGL((k_lsweep_w<ND, NT, false>), gw, dim3(64*LSW), 0, s, base, cnt, nfvars, \
+                           kappa, nlocal, rowptr, colidx, geo, lam, diag, u, du); \
+    else if (upper) \
+        hipLaunchKernelGGL((k_lsweep_p<ND, NT, true>), grid(cnt), dim3(FB), 0, s, order + base, cnt, \
+                           nfvars, kappa, nlocal, rowptr, colidx, geo, lam, diag, u, du); \
+    else \
+        hipLaunchKernelGGL((k_lsweep_p<ND, NT, false>), grid(cnt), dim3(FB), 0, s, order + base, cnt, \
+                           nfvars, kappa, nlocal, rowptr, colidx, geo, lam, diag, u, du); \
     return ok(); } while (0)
     switch (nt) {
     case 0: LP(0);
