@@ -246,9 +246,8 @@ def test_serial_matches_oracle(name):
 
 
 def test_serial_schedule_follows_table_changes():
-    """The serial sweeps keep their level schedule for the last neighbour
-    table, keyed by a content hash: a table changed in place (same pointer)
-    gets a new schedule, an unchanged one reuses it; both match the oracle."""
+    """A neighbour table changed in place (same pointer) is followed by the next
+    serial sweeps, as is an unchanged one: both match the oracle."""
     say("serial sweeps: neighbour table changed in place")
     mesh = M.tet_mesh(4, seed=97, permute=True)
     flow = M.flow_fields(mesh, seed=97)
@@ -267,6 +266,54 @@ def test_serial_schedule_follows_table_changes():
                                         flow.upts, flow.rhsb)
         say(f"  {label} table")
         assert np.array_equal(dub.cpu().numpy(), oq), label
+
+
+@pytest.mark.parametrize("N, F, D, kind", [
+    (1, 6, 3, "random"), (255, 4, 3, "random"), (256, 6, 3, "random"), (257, 3, 2, "random"),
+    (600, 4, 3, "line"), (700, 6, 3, "before"), (700, 6, 3, "after"), (513, 1, 3, "line"),
+    (1000, 5, 3, "random"), (1300, 9, 2, "random"), (900, 4, 2, "random"), (3000, 6, 2, "near"),
+    (3000, 6, 3, "nan")])
+def test_serial_sweeps_at_workgroup_edges(N, F, D, kind):
+    """The sequential sweeps on tables of any shape: a line (every cell waits for
+    the one before it), all neighbours before or after, near and far ones, cells
+    with more taken faces than wait at a time, one and many workgroups, face
+    counts with a kernel of their own and without; and with solutions that are
+    NaN, one of them with the bits that mark a value as not there yet."""
+    say(f"serial sweeps, {N} cells, {F} faces, {D}-D, {kind}")
+    rng = np.random.default_rng(N + F)
+    i = np.arange(N)
+    nei = {"random": lambda: rng.integers(0, N, (F, N)), "nan": lambda: rng.integers(0, N, (F, N)),
+           "line": lambda: np.stack([np.clip(i + (1 if f % 2 else -1), 0, N - 1) for f in range(F)]),
+           "before": lambda: rng.integers(0, i + 1, (F, N)),
+           "after": lambda: rng.integers(i, N, (F, N)),
+           "near": lambda: np.clip(i + rng.integers(-70, 70, (F, N)), 0, N - 1)}[kind]()
+    nei = np.ascontiguousarray(nei, np.int32)
+    fnv, fspr = rng.uniform(0.5, 1.0, (F, N)), rng.uniform(0.5, 2.0, (F, N))
+    vfn = np.ascontiguousarray(rng.normal(0.0, 0.6, (F, D, N)))
+    upts = rng.uniform(0.1, 0.3, (D + 2, N))
+    upts[0] += 1.0
+    upts[-1] += 2.5
+    rhs, dt = rng.normal(0.0, 1e-3, (D + 2, N)), rng.uniform(0.1, 0.2, N)
+    if kind == "nan":
+        rhs[1, 40] = np.nan
+        rhs.view(np.uint64)[2, 17] = 0xFFF8A5C35A3C0F1E
+        rhs[3, 90] = np.inf
+    L.call("ucfd_set_config", D + 2, D + 2, D)
+    od, os_, oq, ou = O.serial_pass(nei, fnv, vfn, fspr, dt, upts, rhs)
+    cv = torch_dev()
+    dn, df, dv, ds, ddt = (cv(a) for a in (nei, fnv, vfn, fspr, dt))
+    for two in (False, True):
+        u, r, diag = cv(upts.copy()), cv(rhs.copy()), cv(np.zeros(N))
+        b = cv(np.zeros_like(rhs)) if two else r
+        L.call("serial_pre_lusgs", N, F, 1.0, df, ddt, diag, ds)
+        pre = "ns_serial" if two else "serial_ns"
+        args = (u, r, b, diag, ds) if two else (u, r, diag, ds)
+        L.call(f"{pre}_lower_sweep", N, F, dn, df, dv, *args)
+        low = b.cpu().numpy().copy()
+        L.call(f"{pre}_upper_sweep", N, F, dn, df, dv, *args)
+        assert np.array_equal(low, os_, equal_nan=True), "dQ*"
+        assert np.array_equal(r.cpu().numpy(), oq, equal_nan=True), "dQ"
+    L.call("ucfd_set_config", 5, 5, 3)
 
 
 def test_hex32_ten_iterations_match_reference_fixture():

@@ -165,59 +165,6 @@ int do_colored(const char *fn, int dir, int n0, int ne, int neles, int nface, co
     return sg.leave(rc);
 }
 
-// Level schedules of the serial sweeps, one per direction, kept for the
-// last neighbour table seen: the key is the array's address, the sizes and a
-// content hash of nei_ele (about 0.1 ms on the device), so a schedule is
-// reused only for the same table and rebuilt whenever an entry changes.
-struct SerialSchedule {
-    const void *nei = nullptr;
-    int neles = -1, nface = -1;
-    bool dev = false;
-    unsigned long long hash = 0;
-    std::vector<int> off;
-    int *order_d = nullptr;     // device copy of the level order
-    size_t cap = 0;
-};
-SerialSchedule g_serial[2];
-std::mutex g_serial_mu;
-unsigned long long *g_hash_d = nullptr;
-
-// Dependency levels of the sequential sweep: lower (nb < i) or upper (nb > i).
-// order[] lists cells level by level, off[l]..off[l+1] is level l.
-void build_levels(int dir, int N, int F, const int *nei, std::vector<int> &order,
-                  std::vector<int> &off)
-{
-    std::vector<int> lev(N, 0);
-    int maxl = 0;
-    if (dir == 0) {
-        for (int i = 0; i < N; ++i) {
-            int l = 0;
-            for (int f = 0; f < F; ++f) {
-                const int nb = nei[(size_t)f*N + i];
-                if (nb >= 0 && nb < i) l = std::max(l, lev[nb] + 1);
-            }
-            lev[i] = l;
-            maxl = std::max(maxl, l);
-        }
-    } else {
-        for (int i = N - 1; i >= 0; --i) {
-            int l = 0;
-            for (int f = 0; f < F; ++f) {
-                const int nb = nei[(size_t)f*N + i];
-                if (nb > i && nb < N) l = std::max(l, lev[nb] + 1);
-            }
-            lev[i] = l;
-            maxl = std::max(maxl, l);
-        }
-    }
-    off.assign(maxl + 2, 0);
-    for (int i = 0; i < N; ++i) off[lev[i] + 1]++;
-    for (int l = 0; l <= maxl; ++l) off[l + 1] += off[l];
-    order.resize(N);
-    std::vector<int> pos(off.begin(), off.end() - 1);
-    for (int i = 0; i < N; ++i) order[pos[lev[i]]++] = i;
-}
-
 int do_serial(const char *fn, int dir, int neles, int nface, const int *nei,
               const double *fnorm_vol, const double *vec_fnorm, const double *upts,
               const double *in, double *out, const double *diag, const double *fspr,
@@ -230,64 +177,8 @@ int do_serial(const char *fn, int dir, int neles, int nface, const int *nei,
     const UcfdConfig &c = ucfd_config();
     const size_t N = (size_t)neles, F = (size_t)nface, D = (size_t)c.ndims,
                  V = rans ? (size_t)c.nvars : (size_t)c.nfvars;
-    int rc = ucfd_ensure_device(fn);
-    if (rc) return rc;
-
-    // the level schedule is built on the host from nei_ele, or reused; one
-    // lock covers the hash buffer, the hash and the schedule cache, so
-    // concurrent serial calls neither allocate nor read the hash twice
-    if (!nei) return ucfd_report(UCFD_ERR_ARG, fn, "NULL nei_ele");
-    std::lock_guard<std::mutex> lock(g_serial_mu);
-    const bool dev = ucfd_is_device_ptr(nei);
-    unsigned long long h = 0;
-    if (dev) {
-        if (!g_hash_d && (rc = ucfd_check_hip(hipMalloc((void **)&g_hash_d, 64), fn,
-                                              "hipMalloc(hash)")))
-            return rc;
-        rc = ucfd_launch_hash(ucfd_stream(), nei, (int64_t)(F*N), g_hash_d);
-        if (!rc) rc = ucfd_check_hip(hipMemcpyAsync(&h, g_hash_d, sizeof h, hipMemcpyDeviceToHost,
-                                                    ucfd_stream()), fn, "hipMemcpyAsync(hash)");
-        if (!rc) rc = ucfd_check_hip(hipStreamSynchronize(ucfd_stream()), fn, "sync");
-        if (rc) return rc;
-    } else {
-        h = ucfd_hash_host(nei, (int64_t)(F*N));
-    }
-    SerialSchedule &C = g_serial[dir];
-    if (!(C.nei == nei && C.neles == neles && C.nface == nface && C.dev == dev && C.hash == h)) {
-        std::vector<int> hnei;
-        const int *nei_h = nei;
-        if (dev) {
-            hnei.resize(F*N);
-            rc = ucfd_check_hip(hipMemcpy(hnei.data(), nei, F*N*4, hipMemcpyDeviceToHost), fn,
-                                "hipMemcpy(nei_ele)");
-            if (rc) return rc;
-            nei_h = hnei.data();
-        }
-        std::vector<int> order;
-        C.nei = nullptr;
-        build_levels(dir, neles, nface, nei_h, order, C.off);
-        if (C.cap < N) {
-            if (C.order_d) (void)hipFree(C.order_d);
-            C.order_d = nullptr;
-            C.cap = 0;
-            if ((rc = ucfd_check_hip(hipMalloc((void **)&C.order_d, N*4), fn, "hipMalloc(order)")))
-                return rc;
-            C.cap = N;
-        }
-        if ((rc = ucfd_check_hip(hipMemcpy(C.order_d, order.data(), N*4, hipMemcpyHostToDevice),
-                                 fn, "hipMemcpy(order)")))
-            return rc;
-        C.nei = nei;
-        C.neles = neles;
-        C.nface = nface;
-        C.dev = dev;
-        C.hash = h;
-    }
-    const std::vector<int> &off = C.off;
-
     UcfdStage sg(fn);
     const int a_nei = sg.add(nei, F*N*4, UCFD_IN);
-    const int a_ord = sg.add(C.order_d, N*4, UCFD_IN);
     const int a_fnv = sg.add(fnorm_vol, F*N*8, UCFD_IN);
     const int a_vfn = sg.add(vec_fnorm, F*D*N*8, UCFD_IN);
     const int a_u = sg.add(upts, V*N*8, UCFD_IN);
@@ -295,28 +186,16 @@ int do_serial(const char *fn, int dir, int neles, int nface, const int *nei,
     const int a_out = sg.add(out, V*N*8, UCFD_INOUT);
     const int a_dg = sg.add(diag, N*8, UCFD_IN);
     const int a_sp = sg.add(fspr, F*N*8, UCFD_IN);
-    rc = sg.enter();
+    const int a_ws = sg.add(nullptr, ucfd_serial_scratch(neles, nt ? nt : c.ndims + 2),
+                            UCFD_SCRATCH);
+    int rc = sg.enter();
     if (rc) return rc;
-    const int nlev = (int)off.size() - 1;
-    for (int l = 0; l < nlev && !rc; ++l) {
-        if (rans)
-            rc = ucfd_launch_rans_sweep(ucfd_stream(), dir, UCFD_SWEEP_ORDERED, off[l], off[l + 1],
-                                        neles, nface, c.ndims, nt, (const int *)sg.dev(a_nei),
-                                        (const int *)sg.dev(a_ord), nullptr,
-                                        (const double *)sg.dev(a_fnv),
-                                        (const double *)sg.dev(a_vfn),
-                                        (const double *)sg.dev(a_u), (const double *)sg.dev(a_in),
-                                        (double *)sg.dev(a_out), (const double *)sg.dev(a_dg),
-                                        (const double *)sg.dev(a_sp), ucfd_device_flag(), 0);
-        else
-            rc = ucfd_launch_sweep(ucfd_stream(), dir, UCFD_SWEEP_ORDERED, off[l], off[l + 1],
-                                   neles, nface, c.ndims, c.nfvars, (const int *)sg.dev(a_nei),
-                                   (const int *)sg.dev(a_ord), nullptr,
-                                   (const double *)sg.dev(a_fnv), (const double *)sg.dev(a_vfn),
-                                   (const double *)sg.dev(a_u), (const double *)sg.dev(a_in),
-                                   (double *)sg.dev(a_out), (const double *)sg.dev(a_dg),
-                                   (const double *)sg.dev(a_sp), ucfd_device_flag(), 0);
-    }
+    rc = ucfd_launch_serial(ucfd_stream(), dir, neles, nface, c.ndims, nt,
+                            (const int *)sg.dev(a_nei), (const double *)sg.dev(a_fnv),
+                            (const double *)sg.dev(a_vfn), (const double *)sg.dev(a_u),
+                            (const double *)sg.dev(a_in), (double *)sg.dev(a_out),
+                            (const double *)sg.dev(a_dg), (const double *)sg.dev(a_sp),
+                            sg.dev(a_ws), ucfd_device_flag());
     if (rc) ucfd_report(rc, fn, "kernel launch failed");
     return sg.leave(rc);
 }

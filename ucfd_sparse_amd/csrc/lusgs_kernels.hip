@@ -1,5 +1,5 @@
 // FP64 LU-SGS kernels behind the legacy array API: pre (diagonal), the
-// lower / upper sweep over one colour (or one dependency level) and the
+// lower / upper sweep over one colour and the
 // solution update.
 //
 // Sweep: one thread per cell of the launched range; the cell reads its own
@@ -101,7 +101,6 @@ template <typename T> __device__ __forceinline__ T ld_stream(const T *p)
 // DIR 1: upper, out_i = in_i - (0.5 df)/diag_i
 // MODE 0 (colored):  cell i = order[n0 + t]; neighbour taken iff
 //                    lcolor[nb] </> lcolor[i]
-// MODE 1 (ordered):  cell i = order[n0 + t]; neighbour taken iff nb </> i
 // MODE 2 (range):    colour-contiguous layout, cell i = n0 + t; neighbour
 //                    taken iff nb < n0 (lower) / nb >= ne (upper), which is
 //                    the colour test when [n0, ne) is one whole colour of a
@@ -176,8 +175,6 @@ __global__ __launch_bounds__(kSweepBlock) void k_sweep(
         } else if (MODE == 0) {
             const int cn = lcolor[nb];
             tk[f] = DIR == 0 ? (cn < ci) : (cn > ci);
-        } else if (MODE == 1) {
-            tk[f] = DIR == 0 ? (nb < i) : (nb > i);
         } else {
             tk[f] = DIR == 0 ? (nb < n0) : (nb >= n0 + cnt);
         }
@@ -287,8 +284,6 @@ __global__ __launch_bounds__(64*FC) void k_sweep_wf(
         } else if (MODE == 0) {
             const int cn = lcolor[nb];
             tk = DIR == 0 ? (cn < ci) : (cn > ci);
-        } else if (MODE == 1) {
-            tk = DIR == 0 ? (nb < i) : (nb > i);
         } else {
             tk = DIR == 0 ? (nb < n0) : (nb >= n0 + cnt);
         }
@@ -420,8 +415,6 @@ __global__ __launch_bounds__(kBlock) void k_sweep_any(
         if (MODE == 0) {
             const int cn = lcolor[nb];
             take = DIR == 0 ? (cn < ci) : (cn > ci);
-        } else if (MODE == 1) {
-            take = DIR == 0 ? (nb < i) : (nb > i);
         } else {
             take = DIR == 0 ? (nb < n0) : (nb >= n0 + cnt);
         }
@@ -506,8 +499,6 @@ __global__ __launch_bounds__(kSweepBlock) void k_rans_sweep(
         } else if (MODE == 0) {
             const int cn = lcolor[nb];
             tk[f] = DIR == 0 ? (cn < ci) : (cn > ci);
-        } else if (MODE == 1) {
-            tk[f] = DIR == 0 ? (nb < i) : (nb > i);
         } else {
             tk[f] = DIR == 0 ? (nb < n0) : (nb >= n0 + cnt);
         }
@@ -606,8 +597,6 @@ __global__ __launch_bounds__(64*FC) void k_rans_wf(
         } else if (MODE == 0) {
             const int cn = lcolor[nb];
             tk = DIR == 0 ? (cn < ci) : (cn > ci);
-        } else if (MODE == 1) {
-            tk = DIR == 0 ? (nb < i) : (nb > i);
         } else {
             tk = DIR == 0 ? (nb < n0) : (nb >= n0 + cnt);
         }
@@ -661,7 +650,7 @@ __global__ __launch_bounds__(64*FC) void k_rans_wf(
 // chain and spreads it.  Large launches of tets on a declared layout are bound
 // by the rate of their mixed streams and gathers, where the thread per cell
 // with every load of the cell in flight is ahead.  On a caller's own numbering
-// (MODE 0, 1) it is not: each launch touches most lines of every array, and the
+// (MODE 0) it is not: each launch touches most lines of every array, and the
 // extra waves hide more of it.  Times of a whole pass, us, thread per cell ->
 // wave per face (flow rows; cells in the mesh, two colours unless said):
 //   tets, declared: 197K 40.7 -> 37.2, 547K 88.0 -> 84.1, 1.6M (4-5 colours)
@@ -671,7 +660,6 @@ __global__ __launch_bounds__(64*FC) void k_rans_wf(
 //   hexes, declared: 101K 32.9 -> 31.5, 486K 90.1 -> 87.9, 2.1M 350 -> 342
 //   hexes, own numbering: 101K 48.6 -> 45.1, 246K 81.7 -> 84.3,
 //     486K 150.9 -> 148.7, 1.0M 303 -> 291
-//   sequential sweeps of a 41x37x33 grid: 20.1 -> 10.0 us per level
 // kWfRound: the cells the chip holds at once as six-wave workgroups (5 per
 // CU); between one and three such rounds of hexes the last, partly filled one
 // costs what the extra waves bring.  With turbulence rows hexes gain below one
@@ -879,52 +867,8 @@ int ucfd_launch_sweep(hipStream_t s, int dir, int mode, int n0, int ne, int nele
     if (dir == 0 && mode == UCFD_SWEEP_RANGE)
         return launch_sweep_d<0, 2>(s, ndims, n0, cnt, neles, nface, nei, order, lcolor, fnorm_vol,
                                     vec_fnorm, upts, in, out, diag, fspr, flag, lc_expect);
-    if (dir == 1 && mode == UCFD_SWEEP_RANGE)
-        return launch_sweep_d<1, 2>(s, ndims, n0, cnt, neles, nface, nei, order, lcolor, fnorm_vol,
-                                    vec_fnorm, upts, in, out, diag, fspr, flag, lc_expect);
-    if (dir == 0)
-        return launch_sweep_d<0, 1>(s, ndims, n0, cnt, neles, nface, nei, order, lcolor, fnorm_vol,
-                                    vec_fnorm, upts, in, out, diag, fspr, flag, lc_expect);
-    return launch_sweep_d<1, 1>(s, ndims, n0, cnt, neles, nface, nei, order, lcolor, fnorm_vol,
+    return launch_sweep_d<1, 2>(s, ndims, n0, cnt, neles, nface, nei, order, lcolor, fnorm_vol,
                                 vec_fnorm, upts, in, out, diag, fspr, flag, lc_expect);
-}
-
-// Content hash of an int array: sum over k of splitmix64(k, a[k]) mod 2^64.
-// The sum is order independent, so the block partials can be added with
-// atomics and the result is still deterministic.
-__device__ __forceinline__ unsigned long long hash_mix(unsigned long long k, int v)
-{
-    unsigned long long z = k*0x9E3779B97F4A7C15ull + (unsigned long long)(unsigned)v;
-    z = (z ^ (z >> 30))*0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27))*0x94D049BB133111EBull;
-    return z ^ (z >> 31);
-}
-
-__global__ void k_hash_zero(unsigned long long *out)
-{
-    if (threadIdx.x == 0) out[0] = 0ull;
-}
-
-__global__ __launch_bounds__(kBlock) void k_hash(const int *__restrict__ a, int64_t n,
-                                                 unsigned long long *out)
-{
-    unsigned long long s = 0ull;
-    const int64_t st = (int64_t)gridDim.x*kBlock;
-    for (int64_t k = (int64_t)blockIdx.x*kBlock + threadIdx.x; k < n; k += st)
-        s += hash_mix((unsigned long long)k, a[k]);
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if ((threadIdx.x & 63) == 0) atomicAdd(out, s);
-}
-
-int ucfd_launch_hash(hipStream_t s, const int *a, int64_t n, unsigned long long *out)
-{
-    hipLaunchKernelGGL(k_hash_zero, dim3(1), dim3(64), 0, s, out);
-    if (n > 0) {
-        int64_t blocks = (n + kBlock - 1)/kBlock;
-        if (blocks > 2048) blocks = 2048;
-        hipLaunchKernelGGL(k_hash, dim3((unsigned)blocks), dim3(kBlock), 0, s, a, n, out);
-    }
-    return hipGetLastError() == hipSuccess ? UCFD_OK : UCFD_ERR_HIP;
 }
 
 int ucfd_launch_update(hipStream_t s, int neles, int nrows, double *y, const double *x)
@@ -947,7 +891,6 @@ int ucfd_launch_rans_sweep(hipStream_t s, int dir, int mode, int n0, int ne, int
                                             lcolor, fnorm_vol, vec_fnorm, upts, in, out, tdiag, \
                                             tfspr, flag, lc_expect)
     if (mode == UCFD_SWEEP_COLORED) { if (dir == 0) RM(0, 0); RM(1, 0); }
-    if (mode == UCFD_SWEEP_ORDERED) { if (dir == 0) RM(0, 1); RM(1, 1); }
     // every face taken, as in ucfd_launch_sweep
     if (dir == 0 ? ne == neles : n0 == 0) { if (dir == 0) RM(0, 3); RM(1, 3); }
     if (dir == 0) RM(0, 2);

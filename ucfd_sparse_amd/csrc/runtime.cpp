@@ -153,6 +153,9 @@ int ucfd_sync_and_check(const char *fn)
         if (f & UCFD_KFLAG_INDEX)
             return ucfd_report(UCFD_ERR_INDEX, fn, "an index array holds an entry outside "
                                                    "[0, neles); the affected cells were skipped");
+        if (f & UCFD_KFLAG_STALL)
+            return ucfd_report(UCFD_ERR_HIP, fn, "a sequential sweep waited too long for an earlier "
+                                                 "cell and was given up; its results are undefined");
         if (f & UCFD_KFLAG_DUP)
             return ucfd_report(UCFD_ERR_INDEX, fn, "cell_ids maps two elements to the same cell; "
                                                    "the rank rows of that cell are undefined");
@@ -201,6 +204,11 @@ int UcfdStage::enter()
     for (int k = 0; k < nargs; ++k) {
         Arg &a = args[k];
         a.owner = -1;
+        if (a.dir == UCFD_SCRATCH) {
+            a.staged = true;
+            a.owner = k;
+            continue;
+        }
         if (!a.host) {
             s.mu.unlock();
             return ucfd_report(UCFD_ERR_ARG, fn, "NULL array argument");
@@ -238,7 +246,7 @@ int UcfdStage::enter()
     for (int k = 0; k < nargs; ++k) {
         Arg &a = args[k];
         if (!a.staged) continue;
-        any_staged = true;
+        (a.dir == UCFD_SCRATCH ? scratch : any_staged) = true;
         if (a.owner == k) {
             a.dev = (char *)s.ws + off;
             off += (a.bytes + 255) & ~(size_t)255;
@@ -277,22 +285,13 @@ int UcfdStage::leave(int status)
     } else {
         int r = ucfd_check_hip(hipGetLastError(), fn, "kernel launch");
         if (!rc) rc = r;
+        if (scratch) {
+            r = ucfd_check_hip(hipStreamSynchronize(s.stream), fn, "hipStreamSynchronize");
+            if (!rc) rc = r;
+        }
     }
     s.mu.unlock();
     return rc;
-}
-
-unsigned long long ucfd_hash_host(const int *a, int64_t n)
-{
-    unsigned long long s = 0ull;
-    for (int64_t k = 0; k < n; ++k) {
-        unsigned long long z = (unsigned long long)k*0x9E3779B97F4A7C15ull +
-                               (unsigned long long)(unsigned)a[k];
-        z = (z ^ (z >> 30))*0xBF58476D1CE4E5B9ull;
-        z = (z ^ (z >> 27))*0x94D049BB133111EBull;
-        s += z ^ (z >> 31);
-    }
-    return s;
 }
 
 // ---------------------------------------------------------------- extensions

@@ -21,8 +21,9 @@ enum {
 };
 
 // Error bits raised by kernels, one word each (error_word.h).
-enum { UCFD_KFLAG_INDEX = 1, UCFD_KFLAG_PIVOT = 2, UCFD_KFLAG_LAYOUT = 4, UCFD_KFLAG_DUP = 8 };
-constexpr int UCFD_KFLAG_COUNT = 4;
+enum { UCFD_KFLAG_INDEX = 1, UCFD_KFLAG_PIVOT = 2, UCFD_KFLAG_LAYOUT = 4, UCFD_KFLAG_DUP = 8,
+       UCFD_KFLAG_STALL = 16 };
+constexpr int UCFD_KFLAG_COUNT = 5;
 
 // Flow-variable configuration of the legacy API (compile-time in the
 // reference: NVARS / NFVARS / NDIMS, Makefile.inc:21-24).
@@ -55,13 +56,15 @@ UCFD_HIDDEN int ucfd_poll(const unsigned long long *word, unsigned long long wan
 // Staging of host arrays for one call.  Device (or managed) pointers are used
 // in place; host pointers are copied to a library workspace on entry and
 // copied back on exit when written.  Arguments that alias share one buffer.
-enum { UCFD_IN = 1, UCFD_OUT = 2, UCFD_INOUT = 3 };
+// UCFD_SCRATCH: no array, space in the workspace while the call lasts (leave()
+// waits for the stream, so that the next call on any stream may use it).
+enum { UCFD_IN = 1, UCFD_OUT = 2, UCFD_INOUT = 3, UCFD_SCRATCH = 4 };
 
 struct UcfdStage {
     struct Arg { const void *host; size_t bytes; int dir; void *dev; bool staged; int owner; };
     Arg args[24];
     int nargs = 0;
-    bool any_staged = false;
+    bool any_staged = false, scratch = false;
     const char *fn;
     explicit UcfdStage(const char *name) : fn(name) {}
     // register an argument; returns its index
@@ -81,15 +84,14 @@ UCFD_HIDDEN int ucfd_colored_mode(const int *icolor, const int *lcolor, int nele
                                   int *lc_value);
 
 // ---- kernel launchers (lusgs_kernels.hip)
-enum { UCFD_SWEEP_COLORED = 0, UCFD_SWEEP_ORDERED = 1, UCFD_SWEEP_RANGE = 2 };
+enum { UCFD_SWEEP_COLORED = 0, UCFD_SWEEP_RANGE = 2 };
 
 UCFD_HIDDEN int ucfd_launch_pre(hipStream_t s, int neles, int nface, double factor,
                                 const double *fnorm_vol, const double *dt, double *diag,
                                 const double *fspr);
 
 // dir 0 = lower, 1 = upper.  mode COLORED: cells order[n0:ne), neighbour
-// taken iff lcolor[nb] </> lcolor[i].  mode ORDERED: cells order[n0:ne),
-// neighbour taken iff nb </> i (sequential semantics, level scheduled).
+// taken iff lcolor[nb] </> lcolor[i].
 // mode RANGE: cells n0..ne-1 of a declared colour-contiguous layout,
 // neighbour taken iff nb < n0 / nb >= ne; order (= icolor) and lcolor are
 // only sampled, one cell per workgroup, against the declared layout
@@ -114,8 +116,14 @@ UCFD_HIDDEN int ucfd_launch_rans_sweep(hipStream_t s, int dir, int mode, int n0,
 
 // y += x over nrows rows of neles cells ([nrows][neles])
 UCFD_HIDDEN int ucfd_launch_update(hipStream_t s, int neles, int nrows, double *y, const double *x);
-// *out = sum over k < n of a mix of (k, a[k]) mod 2^64 (device array a; out
-// device memory): a content hash, order independent and deterministic.
-UCFD_HIDDEN int ucfd_launch_hash(hipStream_t s, const int *a, int64_t n, unsigned long long *out);
-// the same hash of a host array
-UCFD_HIDDEN unsigned long long ucfd_hash_host(const int *a, int64_t n);
+
+// ---- sequential sweeps (serial_kernels.hip): every cell after its neighbours
+// earlier in the sweep (dir 0 ascending, 1 descending).  nt = 0: the flow rows, any
+// nface; nt 1 or 2: the turbulence rows (nface 3, 4 or 6).  scratch holds
+// ucfd_serial_scratch bytes, rows = nt or ndims + 2.
+UCFD_HIDDEN size_t ucfd_serial_scratch(int neles, int rows);
+UCFD_HIDDEN int ucfd_launch_serial(hipStream_t s, int dir, int neles, int nface, int ndims, int nt,
+                                   const int *nei, const double *fnorm_vol,
+                                   const double *vec_fnorm, const double *upts, const double *in,
+                                   double *out, const double *diag, const double *fspr,
+                                   void *scratch, int *flag);
