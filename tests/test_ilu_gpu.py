@@ -277,3 +277,53 @@ def test_errors_are_reported(K):
     with pytest.raises(L.UCFDError):
         K.Precon(A.rowptr, A.colidx, A.diagslots, np.array(A.values), A.bn, 1, kind="bilu",
                  fp32=True)
+
+
+def with_zero_upper_block(A):
+    """A copy of A whose last row has one more block behind its diagonal: zeros at
+    the first row's column."""
+    z = np.zeros((1, A.blk, A.blk))
+    rowptr = A.rowptr.copy()
+    rowptr[-1] += 1
+    return M.BSR(A.bn, A.blk, rowptr, np.append(A.colidx, np.int32(0)), A.diagslots,
+                 np.concatenate([A.values, z]))
+
+
+@pytest.mark.parametrize("blk", [2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("bn, ncolors, per_row", [(131, 2, 5), (64, 2, 3), (200, 3, 20), (90, 5, 12),
+                                                  (40, 0, 1)])
+def test_joined_levels_and_rows_beyond_the_held_columns(K, blk, bn, ncolors, per_row):
+    """The last rows of a coloured matrix have no block above the diagonal: one
+    launch updates them for both sweeps.  Against the oracle for block ILU(0) (rows
+    of up to some 40 blocks, more than the factorisation holds the columns of) and
+    FP64 block LU-SGS; FP32 block LU-SGS equals that of the matrix with a zero block
+    above the diagonal of the last row, where the two updates are separate launches."""
+    if ncolors:
+        A, off, b = random_case(bn, blk, per_row, 900 + bn, ncolors=ncolors)
+    else:
+        A, off, b = random_case(bn, blk, per_row, 900 + bn)
+    say(f"joined levels: {bn} rows of {blk}x{blk}, {ncolors} colours, "
+        f"up to {int(np.diff(A.rowptr).max())} blocks a row")
+    for icolors in ((off, None) if ncolors else (None,)):
+        kind = "pbilu" if icolors is not None else "bilu"
+        D = Dev(A)
+        pc = K.Precon.from_bsr(D, icolors=icolors, kind="bilu")
+        f = O.ilu_prepare(A, kind)
+        assert np.array_equal(D.values.cpu().numpy(), f.reshape(A.values.shape))
+        x = dev(b)
+        pc.apply(x)
+        assert np.array_equal(x.cpu().numpy(), O.ilu_apply(A, f, b, kind, icolors))
+        pc = K.Precon.from_bsr(Dev(A), icolors=icolors)
+        pc.prepare()
+        x = dev(b)
+        pc.apply(x)
+        assert np.array_equal(x.cpu().numpy(),
+                              O.blusgs_apply(A, O.blusgs_prepare(A), b, icolors))
+        got = []
+        for m in (A, with_zero_upper_block(A)):
+            pc = K.Precon.from_bsr(Dev(m), icolors=icolors, fp32=True)
+            pc.prepare()
+            x = dev(b)
+            pc.apply(x)
+            got.append(x.cpu().numpy())
+        assert np.array_equal(got[0], got[1])

@@ -57,6 +57,7 @@ struct _Precon {
     float *vals32;           // device, nnz*blk*blk (fp32 only)
     float *x32;              // device, bn*blk (fp32 only)
     bool init32;             // the lower pass reads rows it has not yet produced
+    bool joined;             // the last lower launch does the first upper level's rows too
     UcfdSchedule lower, upper;
 };
 
@@ -198,30 +199,26 @@ int pc_apply(hipStream_t s, Precon pc, const PcDev &d, double *b)
     const int kind = pc_kind(pc);
     if (kind < 0) return UCFD_OK;
     int rc = UCFD_OK;
-    if (!pc->fp32) {
-        for (const UcfdLevel &l : pc->lower.lv)
-            if ((rc = kry_bsgs_sweep64(s, kind, 0, pc->blk, l.base, l.cnt,
-                                       l.ordered ? pc->lower.order : nullptr, d.rowptr, d.colidx,
-                                       d.diagslots, d.values, pc->diagvalues, b, l.empty)))
-                return rc;
-        for (const UcfdLevel &l : pc->upper.lv)
-            if ((rc = kry_bsgs_sweep64(s, kind, 1, pc->blk, l.base, l.cnt,
-                                       l.ordered ? pc->upper.order : nullptr, d.rowptr, d.colidx,
-                                       d.diagslots, d.values, pc->diagvalues, b, l.empty)))
-                return rc;
-        return UCFD_OK;
+    const std::vector<UcfdLevel> &lo = pc->lower.lv, &up = pc->upper.lv;
+    if (pc->fp32 && pc->init32 && (rc = kry_cast32(s, (int64_t)pc->bn*pc->blk, b, pc->x32)))
+        return rc;
+    for (int upper = 0; upper < 2; ++upper) {
+        const std::vector<UcfdLevel> &lv = upper ? up : lo;
+        int *const order = upper ? pc->upper.order : pc->lower.order;
+        for (size_t k = upper && pc->joined ? 1 : 0; k < lv.size(); ++k) {
+            const UcfdLevel &l = lv[k];
+            const bool join = pc->joined && !upper && k + 1 == lv.size();
+            if (pc->fp32)
+                rc = kry_bsgs_sweep32(s, upper, pc->blk, l.base, l.cnt, l.ordered ? order : nullptr,
+                                      d.rowptr, d.colidx, d.diagslots, pc->vals32, pc->diagvalues,
+                                      pc->x32, b, l.empty, join);
+            else
+                rc = kry_bsgs_sweep64(s, kind, upper, pc->blk, l.base, l.cnt,
+                                      l.ordered ? order : nullptr, d.rowptr, d.colidx, d.diagslots,
+                                      d.values, pc->diagvalues, b, l.empty, join);
+            if (rc) return rc;
+        }
     }
-    if (pc->init32 && (rc = kry_cast32(s, (int64_t)pc->bn*pc->blk, b, pc->x32))) return rc;
-    for (const UcfdLevel &l : pc->lower.lv)
-        if ((rc = kry_bsgs_sweep32(s, 0, pc->blk, l.base, l.cnt,
-                                   l.ordered ? pc->lower.order : nullptr, d.rowptr, d.colidx,
-                                   d.diagslots, pc->vals32, pc->diagvalues, pc->x32, b, l.empty)))
-            return rc;
-    for (const UcfdLevel &l : pc->upper.lv)
-        if ((rc = kry_bsgs_sweep32(s, 1, pc->blk, l.base, l.cnt,
-                                   l.ordered ? pc->upper.order : nullptr, d.rowptr, d.colidx,
-                                   d.diagslots, pc->vals32, pc->diagvalues, pc->x32, b, l.empty)))
-            return rc;
     return UCFD_OK;
 }
 
@@ -250,6 +247,16 @@ void mark_empty_levels(UcfdSchedule &S, bool upper, const std::vector<int> &rp,
         for (int i = l.base; i < l.base + l.cnt && l.empty; ++i)
             l.empty = (upper ? rp[i + 1] - ds[i] - 1 : ds[i] - rp[i]) == 0;
     }
+}
+
+// The last lower level and the first upper one are the same rows, which take
+// blocks in the lower sweep only (as the last colour of a coloured numbering): one
+// launch does both updates of a row (the block kernels of contiguous levels).
+bool levels_join(const Precon pc)
+{
+    if (pc->blk < 2 || pc->init32 || pc->lower.lv.empty() || pc->upper.lv.empty()) return false;
+    const UcfdLevel &l = pc->lower.lv.back(), &u = pc->upper.lv.front();
+    return !l.ordered && !l.empty && !u.ordered && u.empty && l.base == u.base && l.cnt == u.cnt;
 }
 
 int make_schedules(Precon pc, const char *fn)
@@ -315,6 +322,7 @@ int make_schedules(Precon pc, const char *fn)
         mark_empty_levels(pc->lower, false, rp, ds);
         mark_empty_levels(pc->upper, true, rp, ds);
         pc->init32 = unvis_l;
+        pc->joined = levels_join(pc);
         return UCFD_OK;
     }
     std::vector<std::vector<int>> levels;
@@ -334,6 +342,7 @@ int make_schedules(Precon pc, const char *fn)
     mark_empty_levels(pc->lower, false, rp, ds);
     mark_empty_levels(pc->upper, true, rp, ds);
     pc->init32 = unvis_l;
+    pc->joined = levels_join(pc);
     return UCFD_OK;
 }
 

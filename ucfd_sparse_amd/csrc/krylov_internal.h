@@ -49,18 +49,21 @@ enum { KRY_SW_LUSGS = 0, KRY_SW_BILU = 1, KRY_SW_ILU = 2 };
 // KRY_SW_BILU (factored values): lower x_i = b_i - sum_{j<diag} L_ij x_j,
 // upper x_i = U_ii^-1 (x_i - sum_{j>diag} U_ij x_j) with diagvalues the
 // factored U_ii.  KRY_SW_ILU: the scalar form (blk 1), dividing by the pivot.
-// empty: no row of the (contiguous) level has a block in this direction.
+// empty: no row of the (contiguous) level has a block in this direction.  join (a
+// lower sweep of a contiguous level, blk > 1): each row's update of the upper sweep
+// follows at once, for rows with no block above the diagonal.
 UCFD_HIDDEN int kry_bsgs_sweep64(hipStream_t s, int kind, int upper, int blk, int base, int cnt,
                                  const int *order, const int *rowptr, const int *colidx,
                                  const int *diagslots, const double *values,
-                                 const double *diagvalues, double *b, bool empty);
+                                 const double *diagvalues, double *b, bool empty, bool join);
 // Mixed form: block products in FP32 on FP32 values and an FP32 work vector
 // x32, the diagonal solve in FP64.  lower reads the right-hand side b (FP64)
 // and writes x32; upper updates x32 and writes the final value to b (FP64).
 UCFD_HIDDEN int kry_bsgs_sweep32(hipStream_t s, int upper, int blk, int base, int cnt,
                                  const int *order, const int *rowptr, const int *colidx,
                                  const int *diagslots, const float *vals32,
-                                 const double *diagvalues, float *x32, double *b, bool empty);
+                                 const double *diagvalues, float *x32, double *b, bool empty,
+                                 bool join);
 
 // Scalars posted to the host by the kernel that forms them: values at out (the
 // device address of pinned memory), then seq at word (0: not yet the last).
