@@ -28,6 +28,7 @@ __device__ __forceinline__ int fxcd()
     return x*per + (x < rem ? x : rem) + k;
 }
 
+inline dim3 waves(int64_t n) { return dim3((unsigned)((n + 63)/64)); }   // of 64 lanes
 inline dim3 grid(int64_t n) { return dim3((unsigned)((n + FB - 1)/FB)); }
 
 int ok() { return hipGetLastError() == hipSuccess ? UCFD_OK : UCFD_ERR_HIP; }
@@ -41,6 +42,60 @@ int ok() { return hipGetLastError() == hipSuccess ? UCFD_OK : UCFD_ERR_HIP; }
 // up to 64 cache lines).
 constexpr int PACK_MAXV = 16;
 typedef double fs_d2 __attribute__((ext_vector_type(2)));
+
+// the rank row of element e; -1 beyond the last one or, reported, with no valid row
+__device__ __forceinline__ int elem_row(int e, int neles, int nlocal,
+                                        const int *__restrict__ cell_ids, int *flag)
+{
+    if (e >= neles) return -1;
+    const int r = cell_ids[e];
+    if ((unsigned)r < (unsigned)nlocal) return r;
+    ucfd::raise(flag, UCFD_KFLAG_INDEX);
+    return -1;
+}
+
+// A wave writes one W-word record a lane (v, at row r of rec; r < 0: none) or reads
+// the n consecutive records from row r0 on: the records are turned in LDS (s: 64*W
+// words), so that consecutive lanes meet consecutive words in pairs.  A lane that
+// writes its own record touches 64 lines with each of its W/2 stores.  W is even.
+// Pack of 356K tets, 6 variables (8-word records): the element kernel 26.8 -> 17.4 us
+// (read back through LDS too, its other half 22.5 -> 25.6: left).  Scalar Pack
+// (18-word records; 22 with 7 variables) and Update, whole calls: 166K hexes 42.0 ->
+// 40.1 and 23.8 -> 23.8 us, 343K hexes 89.3 -> 75.1 and 35.0 -> 31.7, 1.3M tets 244
+// -> 235 and 86.9 -> 82.4.
+template <int W>
+__device__ __forceinline__ void put_records(double *s, const double *v, int r, double *rec)
+{
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int q = 0; q < W/2; ++q) ((fs_d2 *)s)[lane*(W/2) + q] = fs_d2{v[2*q], v[2*q + 1]};
+    ucfd::wave_lds_sync();
+#pragma unroll
+    for (int k = 0; k < W/2; ++k) {
+        const int f = k*64 + lane, el = f/(W/2), re = __shfl(r, el, 64);
+        if (re >= 0) ((fs_d2 *)rec)[(int64_t)re*(W/2) + (f - el*(W/2))] = ((fs_d2 *)s)[f];
+    }
+}
+
+template <int W>
+__device__ __forceinline__ void get_records(double *s, int r0, int n, const double *rec, double *v)
+{
+    const int lane = threadIdx.x & 63;
+    const fs_d2 *in = (const fs_d2 *)rec + (int64_t)r0*(W/2);
+    fs_d2 t[W/2];
+#pragma unroll
+    for (int k = 0; k < W/2; ++k)
+        if (k*64 + lane < n*(W/2)) t[k] = in[k*64 + lane];
+#pragma unroll
+    for (int k = 0; k < W/2; ++k) ((fs_d2 *)s)[k*64 + lane] = t[k];
+    ucfd::wave_lds_sync();
+#pragma unroll
+    for (int q = 0; q < W/2; ++q) {
+        const fs_d2 x = ((fs_d2 *)s)[lane*(W/2) + q];
+        v[2*q] = x.x;
+        v[2*q + 1] = x.y;
+    }
+}
 
 __global__ __launch_bounds__(64) void k_pack(int neles, int nlocal, int nvars, int nfvars, double a0,
                                              const int *__restrict__ cell_ids,
@@ -97,7 +152,7 @@ __global__ __launch_bounds__(64) void k_pack(int neles, int nlocal, int nvars, i
 // element to one record of (nvars + 2) & ~1 doubles (nvars 4-9; k_pack
 // otherwise).
 template <int NV>
-__global__ __launch_bounds__(FB) void k_bpack_rec(int neles, int nlocal, double a0,
+__global__ __launch_bounds__(64) void k_bpack_rec(int neles, int nlocal, double a0,
                                                   const int *__restrict__ cell_ids,
                                                   int *__restrict__ inv,
                                                   const double *__restrict__ rhs,
@@ -105,22 +160,17 @@ __global__ __launch_bounds__(FB) void k_bpack_rec(int neles, int nlocal, double 
                                                   double *__restrict__ rec, int *flag)
 {
     constexpr int W = (NV + 2) & ~1;
-    const int e = fxcd()*FB + threadIdx.x;
-    if (e >= neles) return;
-    const int r = cell_ids[e];
-    if ((unsigned)r >= (unsigned)nlocal) {
-        ucfd::raise(flag, UCFD_KFLAG_INDEX);
-        return;
+    __shared__ __align__(16) double s[64*W];
+    const int e = ucfd::wave_xcd_index()*64 + threadIdx.x;
+    const int r = elem_row(e, neles, nlocal, cell_ids, flag);
+    double v[W] = {};
+    if (r >= 0) {
+        inv[r] = e;
+        v[0] = 1/dt[e] + a0;
+#pragma unroll
+        for (int k = 0; k < NV; ++k) v[1 + k] = rhs[e + (int64_t)k*neles];
     }
-    inv[r] = e;
-    double v[W];
-    v[0] = 1/dt[e] + a0;
-#pragma unroll
-    for (int k = 0; k < NV; ++k) v[1 + k] = rhs[e + (int64_t)k*neles];
-    if (W > NV + 1) v[W - 1] = 0.0;
-    fs_d2 *o = (fs_d2 *)(rec + (int64_t)r*W);
-#pragma unroll
-    for (int q = 0; q < W/2; ++q) o[q] = fs_d2{v[2*q], v[2*q + 1]};
+    put_records<W>(s, v, r, rec);
 }
 
 template <int NV>
@@ -277,16 +327,6 @@ __global__ __launch_bounds__(FB) void k_subres(int neles, int nlocal, int nvars,
 // SubResidual of 356K cells and 6 variables 77.5 -> 26.0 us (7 variables 90 ->
 // 29.6), 91K cells 17.9 -> 9.9; Update 22.2 -> 13.8, 25 -> 15.5 and 6.5 -> 4.4
 // (with the scalar method's records of 166K cells: 26.6 -> 23.6 for its two passes).
-__device__ __forceinline__ int elem_row(int e, int neles, int nlocal,
-                                        const int *__restrict__ cell_ids, int *flag)
-{
-    if (e >= neles) return -1;
-    const int r = cell_ids[e];
-    if ((unsigned)r < (unsigned)nlocal) return r;
-    ucfd::raise(flag, UCFD_KFLAG_INDEX);
-    return -1;
-}
-
 // W: words of a row in du (NV, or a padded record of the scalar method)
 template <int NV, int W>
 __global__ __launch_bounds__(64) void k_update_w(int neles, int nlocal,
@@ -741,7 +781,7 @@ template <int NV> constexpr int rec_w(int per) { return (per*NV + 1) & ~1; }
 
 
 template <int NV>
-__global__ __launch_bounds__(FB) void k_lpack_rec(int neles, int nlocal, int nfvars,
+__global__ __launch_bounds__(64) void k_lpack_rec(int neles, int nlocal, int nfvars,
                                                   double turb_factor, double a0,
                                                   const int *__restrict__ cell_ids,
                                                   int *__restrict__ inv,
@@ -752,48 +792,40 @@ __global__ __launch_bounds__(FB) void k_lpack_rec(int neles, int nlocal, int nfv
                                                   double *__restrict__ rec, int *flag)
 {
     constexpr int W = rec_w<NV>(3);
-    const int e = fxcd()*FB + threadIdx.x;
-    if (e >= neles) return;
-    const int r = cell_ids[e];
-    if ((unsigned)r >= (unsigned)nlocal) {
-        ucfd::raise(flag, UCFD_KFLAG_INDEX);
-        return;
-    }
-    if (atomicExch(inv + r, e) >= 0) ucfd::raise(flag, UCFD_KFLAG_DUP);
-    const double dte = dt[e];
-    double v[W];
+    __shared__ __align__(16) double s[64*W];
+    const int e = ucfd::wave_xcd_index()*64 + threadIdx.x;
+    const int r = elem_row(e, neles, nlocal, cell_ids, flag);
+    double v[W] = {};
+    if (r >= 0) {
+        if (atomicExch(inv + r, e) >= 0) ucfd::raise(flag, UCFD_KFLAG_DUP);
+        const double dte = dt[e];
 #pragma unroll
-    for (int k = 0; k < NV; ++k) {
-        const int64_t ei = e + (int64_t)k*neles;
-        const double factor = k < nfvars ? 1.0 : turb_factor;
-        v[k] = upts[ei];
-        v[NV + k] = rhs[ei];
-        v[2*NV + k] = 1.0/(dte*factor) + a0 + dsrc[ei];
+        for (int k = 0; k < NV; ++k) {
+            const int64_t ei = e + (int64_t)k*neles;
+            const double factor = k < nfvars ? 1.0 : turb_factor;
+            v[k] = upts[ei];
+            v[NV + k] = rhs[ei];
+            v[2*NV + k] = 1.0/(dte*factor) + a0 + dsrc[ei];
+        }
     }
-    if (W > 3*NV) v[W - 1] = 0.0;
-    fs_d2 *o = (fs_d2 *)(rec + (int64_t)r*W);
-#pragma unroll
-    for (int q = 0; q < W/2; ++q) o[q] = fs_d2{v[2*q], v[2*q + 1]};
+    put_records<W>(s, v, r, rec);
 }
 
 template <int NV>
-__global__ __launch_bounds__(FB) void k_lpack_from_rec(int nlocal, const int *__restrict__ inv,
+__global__ __launch_bounds__(64) void k_lpack_from_rec(int nlocal, const int *__restrict__ inv,
                                                        const double *__restrict__ rec,
                                                        double *__restrict__ u,
                                                        double *__restrict__ du,
                                                        double *__restrict__ diag)
 {
     constexpr int W = rec_w<NV>(3);
-    const int r = fxcd()*FB + threadIdx.x;
-    if (r >= nlocal || inv[r] < 0) return;      // a cell of another element type
-    const fs_d2 *in = (const fs_d2 *)(rec + (int64_t)r*W);
+    __shared__ __align__(16) double s[64*W];
+    const int r0 = ucfd::wave_xcd_index()*64, r = r0 + threadIdx.x;
+    if (r0 >= nlocal) return;
+    const bool has = r < nlocal && inv[r] >= 0;
     double v[W];
-#pragma unroll
-    for (int q = 0; q < W/2; ++q) {
-        const fs_d2 t = in[q];
-        v[2*q] = t.x;
-        v[2*q + 1] = t.y;
-    }
+    get_records<W>(s, r0, min(64, nlocal - r0), rec, v);
+    if (!has) return;                           // a cell of another element type
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
         const int64_t ri = r + (int64_t)k*nlocal;
@@ -804,19 +836,17 @@ __global__ __launch_bounds__(FB) void k_lpack_from_rec(int nlocal, const int *__
 }
 
 template <int NV>
-__global__ __launch_bounds__(FB) void k_lupdate_rec(int nlocal, const double *__restrict__ du,
+__global__ __launch_bounds__(64) void k_lupdate_rec(int nlocal, const double *__restrict__ du,
                                                     double *__restrict__ rec)
 {
     constexpr int W = rec_w<NV>(1);
-    const int r = fxcd()*FB + threadIdx.x;
-    if (r >= nlocal) return;
-    double v[W];
+    __shared__ __align__(16) double s[64*W];
+    const int r = ucfd::wave_xcd_index()*64 + threadIdx.x;
+    double v[W] = {};
+    if (r < nlocal)
 #pragma unroll
-    for (int k = 0; k < NV; ++k) v[k] = du[r + (int64_t)k*nlocal];
-    if (W > NV) v[W - 1] = 0.0;
-    fs_d2 *o = (fs_d2 *)(rec + (int64_t)r*W);
-#pragma unroll
-    for (int q = 0; q < W/2; ++q) o[q] = fs_d2{v[2*q], v[2*q + 1]};
+        for (int k = 0; k < NV; ++k) v[k] = du[r + (int64_t)k*nlocal];
+    put_records<W>(s, v, r < nlocal ? r : -1, rec);
 }
 
 // rank_lusgs_update (lusgs.c:54-70)
@@ -1353,7 +1383,7 @@ int fs_launch_pack(hipStream_t s, int neles, int nlocal, int nvars, int nfvars, 
                            (int64_t)nlocal, inv, -1);
 #define FS_BPACK(NVC) \
         case NVC: \
-            hipLaunchKernelGGL(k_bpack_rec<NVC>, grid(neles), dim3(FB), 0, s, neles, nlocal, a0, \
+            hipLaunchKernelGGL(k_bpack_rec<NVC>, waves(neles), dim3(64), 0, s, neles, nlocal, a0, \
                                cell_ids, inv, rhs, dt, rec, flag); \
             hipLaunchKernelGGL(k_bpack_from_rec<NVC>, dim3((unsigned)((nlocal + 63)/64)), dim3(64), \
                                0, s, nlocal, nfvars, inv, rec, rank_rhs, diag); \
@@ -1467,9 +1497,9 @@ int fs_launch_lpack(hipStream_t s, int neles, int nlocal, int nvars, int nfvars,
                        (int64_t)nlocal, inv, -1);
 #define FS_PACK_REC(NVC) \
     case NVC: \
-        hipLaunchKernelGGL(k_lpack_rec<NVC>, grid(neles), dim3(FB), 0, s, neles, nlocal, nfvars, \
+        hipLaunchKernelGGL(k_lpack_rec<NVC>, waves(neles), dim3(64), 0, s, neles, nlocal, nfvars, \
                            turb_factor, a0, cell_ids, inv, upts, rhs, dt, dsrc, rec, flag); \
-        hipLaunchKernelGGL(k_lpack_from_rec<NVC>, grid(nlocal), dim3(FB), 0, s, nlocal, inv, rec, \
+        hipLaunchKernelGGL(k_lpack_from_rec<NVC>, waves(nlocal), dim3(64), 0, s, nlocal, inv, rec, \
                            u, du, diag); \
         return ok();
     if (rec) {
@@ -1492,7 +1522,7 @@ int fs_launch_lupdate(hipStream_t s, int neles, int nlocal, int nvars, const int
     if (neles <= 0) return UCFD_OK;
 #define FS_UPD_REC(NVC) \
     case NVC: \
-        hipLaunchKernelGGL(k_lupdate_rec<NVC>, grid(nlocal), dim3(FB), 0, s, nlocal, du, rec); \
+        hipLaunchKernelGGL(k_lupdate_rec<NVC>, waves(nlocal), dim3(64), 0, s, nlocal, du, rec); \
         hipLaunchKernelGGL((k_update_w<NVC, rec_w<NVC>(1)>), dim3((unsigned)((neles + 63)/64)), \
                            dim3(64), 0, s, neles, nlocal, cell_ids, rec, upts, flag); \
         return ok();
