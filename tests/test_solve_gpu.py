@@ -172,3 +172,45 @@ def test_solves_at_workgroup_edges_and_on_both_sides_of_the_kernel_choice(kind, 
         assert no <= 2e-10 * np.linalg.norm(f.rhsb[:5])
     assert np.abs(out[1] - out[0]).max() <= 1e-8 * np.abs(out[0]).max()
     s.close()
+
+
+@pytest.mark.parametrize("kind,dims", [("hex", (6, 5, 4)),        # two colours: a pass ahead
+                                       ("hex", (42, 40, 39)),     # 65520 cells, two colours
+                                       ("hex", (42, 40, 40)),     # 67200: FP64 waits
+                                       ("tet", (5,)),             # more colours: waits
+                                       ("hex", (1, 1, 1))])       # one cell, one colour
+def test_solve_stops_where_the_oracle_does(kind, dims):
+    """The lower launch of the next pass is enqueued before the norm of a pass is
+    known: a solve that meets its tolerance after n passes returns, bit for bit, the
+    increment of one bounded to n passes (nothing is enqueued behind the last pass
+    allowed), and n is the oracle's; two handles, so also that nothing stays from a
+    solve before."""
+    mesh = M.tet_mesh(*dims, seed=12) if kind == "tet" else M.hex_mesh(*dims, seed=12)
+    mesh.key = M.hilbert_keys(mesh, kind, dims)
+    lay = colored_layout(mesh, M.flow_fields(mesh, seed=12),
+                         coloring="greedy" if kind == "tet" else "greedy-bfs")
+    m, f = lay.mesh, lay.flow
+    say(f"{kind} {dims}: {m.neles} cells, {lay.ncolors} colours")
+    b = dev(f.rhsb[:5])
+    for handle in range(2):
+        s = LUSGSSolver.from_layout(lay)
+
+        def solve(mode, rtol, maxiter):
+            dq = dev(np.zeros((5, m.neles)))
+            st = s.solve(b, dq, mode, rtol, maxiter)
+            return st, dq.cpu().numpy()
+
+        for rtol in (0.5, 1e-1, 1e-2, 1e-3):
+            # the pass whose norm meets the tolerance is still done
+            n = O.dc_solve(m.nei_ele, lay.icolor, lay.lcolor, m.fnorm_vol, m.vec_fnorm,
+                           f.fspr, f.dt, f.upts, f.rhsb, rtol, 50)[1] + 1
+            st, got = solve("fp64", rtol, 50)
+            assert st.passes == n and st.converged
+            st, bounded = solve("fp64", 0.0, n)
+            assert st.passes == n
+            assert np.array_equal(got, bounded), rtol
+            st, got = solve("mixed", rtol, 50)
+            assert st.converged and st.passes < 50
+            st2, bounded = solve("mixed", rtol, st.passes)
+            assert st2.passes == st.passes and np.array_equal(got, bounded), rtol
+        s.close()

@@ -232,16 +232,27 @@ __device__ __forceinline__ double sum_parts(const double *part, int n)
 // The norm of a pass: partials of the launches before this one, and where the
 // result goes: pinned host memory, the value and then the sequence number that
 // the host polls while the launches behind run (no copy, no wait for the
-// stream).  n = 0: nothing to sum.
+// stream).  n = 0: nothing to sum.  ctl given: whether the solve ends with this
+// pass is decided here too, for the launches behind (ctl[1]) and the host (hout[2]);
+// ctl[0] holds the norm of the first pass.
 struct NormJob {
     const double *part;
     int n;
     double *hout;
     unsigned long long seq;
+    double *ctl = nullptr, tol = 0.0;
+    bool first = false;
 };
 
 __device__ __forceinline__ void publish(const NormJob &job, double t)
 {
+    if (job.ctl) {
+        const double nrm = sqrt(t), base = job.first ? nrm : job.ctl[0];
+        const double stop = base == 0.0 || nrm <= job.tol*base ? 1.0 : 0.0;
+        if (job.first) job.ctl[0] = nrm;
+        job.ctl[1] = stop;
+        __hip_atomic_store(job.hout + 2, stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
     __hip_atomic_store(job.hout, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __hip_atomic_store((unsigned long long *)job.hout + 1, job.seq, __ATOMIC_RELEASE,
                        __HIP_MEMORY_SCOPE_SYSTEM);
@@ -537,9 +548,11 @@ template <typename T, int FC, bool WITH_RES, bool LAST>
 __global__ __launch_bounds__(64*FC) void k_lower_res_wf(
     int n0, int cnt, int N, const int *__restrict__ nei, const Face4<T> *__restrict__ geo,
     const T *__restrict__ diag, const T *__restrict__ qb, const T *__restrict__ rhs, T *e,
-    T *dstar, double *part, int pofs, T *delta)
+    T *dstar, double *part, int pofs, T *delta, const double *stop)
 {
     constexpr int KW = (NV + FC - 1)/FC;
+    // launched ahead of the decision: e stays what the last pass made it
+    const bool halt = LAST && stop && *stop != 0.0;
     __shared__ T slow[FC][NV][64], sres[WITH_RES ? FC : 1][NV][64];
     const int lane = threadIdx.x & 63, f = threadIdx.x >> 6;
     const int b = xcd_remap(), t = b*64 + lane, i = n0 + t;
@@ -594,7 +607,7 @@ __global__ __launch_bounds__(64*FC) void k_lower_res_wf(
             if (LAST) {
                 const T acc0 = T(0), dlt = o - T(0.5)*acc0/dg;
                 *at_split(delta, N, i, q) = dlt;
-                *at_split(e, N, i, q) = ei[w] + dlt;
+                if (!halt) *at_split(e, N, i, q) = ei[w] + dlt;
             } else {
                 *at_split(dstar, N, i, q) = o;
             }
@@ -976,7 +989,8 @@ inline bool wave_per_face(int F, int cnt) { return F == 6 || cnt <= kWfTets; }
 // colour's upper step, writing delta and e (upper_pass then skips it).
 template <typename T>
 int lower_pass(ucfd_lusgs_solver *s, hipStream_t st, bool with_res, const T *qb, const T *rhs,
-               T *e, T *dstar, T *delta, const Face4<T> *geo, const T *diag, bool pre0 = false)
+               T *e, T *dstar, T *delta, const Face4<T> *geo, const T *diag, bool pre0 = false,
+               const double *stop = nullptr)
 {
     int pofs = 0;
     for (int c = 0; c < s->nc; ++c) {
@@ -989,11 +1003,12 @@ int lower_pass(ucfd_lusgs_solver *s, hipStream_t st, bool with_res, const T *qb,
             continue;
         }
         const bool last = s->nc > 1 && c == s->nc - 1;
-#define LRK(K, B) hipLaunchKernelGGL(K, g, dim3(B), 0, st, n0, cnt, s->N, s->nei, geo, diag, qb, \
-                                     rhs, e, dstar, s->parts[s->cur], pofs, delta)
+#define LRK(K, B, ...) hipLaunchKernelGGL(K, g, dim3(B), 0, st, n0, cnt, s->N, s->nei, geo, diag, \
+                                          qb, rhs, e, dstar, s->parts[s->cur], pofs, delta, \
+                                          ##__VA_ARGS__)
 // hexes always take the wave-per-face form
 #define LR(FC, RES, LAST) do { \
-        if (FC == 6 || wf) LRK((k_lower_res_wf<T, FC, RES, LAST>), 64*FC); \
+        if (FC == 6 || wf) LRK((k_lower_res_wf<T, FC, RES, LAST>), 64*FC, stop); \
         else if constexpr (FC == 4) LRK((k_lower_res<T, 4, RES, LAST>), kSB); } while (0)
         if (s->F == 4) {
             if (last) { if (with_res) LR(4, true, true); else LR(4, false, true); }
@@ -1017,9 +1032,10 @@ int lower_pass(ucfd_lusgs_solver *s, hipStream_t st, bool with_res, const T *qb,
 // (more than one colour).
 template <typename T>
 int upper_pass(ucfd_lusgs_solver *s, hipStream_t st, const T *qb, T *dstar, T *delta, T *e,
-               const Face4<T> *geo, const T *diag, const T *rhs = nullptr)
+               const Face4<T> *geo, const T *diag, const T *rhs = nullptr, bool first = false,
+               double tol = 0.0)
 {
-    NormJob job{s->parts[s->cur], s->np, s->hnorm_dev, ++s->seq};
+    NormJob job{s->parts[s->cur], s->np, s->hnorm_dev, ++s->seq, s->norm + 2, tol, first};
     double *next = s->parts[s->cur ^ 1];
     bool summed = false;
     for (int c = s->nc - 1; c >= 0; --c) {
@@ -1088,12 +1104,29 @@ int residual64(ucfd_lusgs_solver *s, hipStream_t st, const double *b, const doub
 // The norm last requested, as soon as the kernel that sums it has written it:
 // the rest of that launch and those behind it run while the host decides and
 // enqueues the next pass.
-int read_norm(ucfd_lusgs_solver *s, hipStream_t st, double *out, const char *fn)
+int read_norm(ucfd_lusgs_solver *s, hipStream_t st, double *out, const char *fn,
+              bool *stop = nullptr)
 {
     int rc = ucfd_poll((const unsigned long long *)s->hnorm + 1, s->seq, st, fn,
                        "norm of the residual");
-    *out = sqrt(*(volatile double *)s->hnorm);
+    const volatile double *h = s->hnorm;
+    *out = sqrt(h[0]);
+    if (stop) *stop = h[2] != 0.0;
     return rc;
+}
+
+// Whether the next pass's lower launch is enqueued before the norm of this one is
+// known (it leaves the increment alone if the solve turns out to have ended), so
+// that the chip does not wait for the host.  A large upper launch hides the host by
+// itself, and the launch too many at the end of a loop costs what it saves
+// elsewhere; with more than two colours there are several.  Solves, us: FP64 900
+// hexes 160 -> 149, 8.8K 195 -> 186, 45K 286 -> 264, 123K 512 -> 521; 6K tets 213
+// -> 184; 48K tets of 4 colours 530 -> 543; mixed 900 hexes 225 -> 204, 8.8K 263 ->
+// 237, 45K 341 -> 301, 123K 423 -> 406, 258K 629 -> 641; 6K tets 280 -> 247, 197K
+// 580 -> 562, 511K 1145 -> 1176.
+bool lower_ahead(const ucfd_lusgs_solver *s, int mode)
+{
+    return s->nc <= 2 && s->N <= (mode == UCFD_SOLVE_FP64 ? 65536 : 200000);
 }
 
 }  // namespace
@@ -1252,23 +1285,30 @@ UCFD_API int ucfd_lusgs_solve(ucfd_lusgs_solver *s, int mode, const double *b, d
     hipLaunchKernelGGL(k_fill<double>, grid1(n), dim3(kB), 0, st, (int64_t)n, E, 0.0);
     double bnorm = 0.0, rn = 0.0;
 
+    const bool ahead = lower_ahead(s, mode);
     auto record = [&](double v) {
         if (info.nhist < UCFD_SOLVE_HIST) info.history[info.nhist++] = v;
     };
 
     if (mode == UCFD_SOLVE_FP64) {
         // e = dq; iteration j: s = b - A(e) (in the lower launches), e += M^-1 s
+        bool stop = false;
+        auto lower = [&](int it) {
+            return lower_pass<double>(s, st, it > 0, s->q64, B, E, s->dstar64, s->delta64, s->g64,
+                                      s->d64, it > 0, it > 0 ? s->norm + 3 : nullptr);
+        };
+        rc = lower(0);
         for (int it = 0; it < maxiter && !rc; ++it) {
-            rc = lower_pass<double>(s, st, it > 0, s->q64, B, E, s->dstar64, s->delta64, s->g64,
-                                    s->d64, it > 0);
+            if (it > 0 && !ahead) rc = lower(it);
             if (!rc) rc = upper_pass<double>(s, st, s->q64, s->dstar64, s->delta64, E, s->g64,
-                                             s->d64, B);
-            if (!rc) rc = read_norm(s, st, &rn, fn);
+                                             s->d64, B, it == 0, rtol);
+            if (!rc && ahead && it + 1 < maxiter) rc = lower(it + 1);
+            if (!rc) rc = read_norm(s, st, &rn, fn, &stop);
             if (rc) break;
             if (it == 0) bnorm = rn;
             record(bnorm > 0 ? rn/bnorm : 0.0);
             info.passes++;
-            if (bnorm == 0.0 || rn <= rtol*bnorm) break;
+            if (stop) break;
         }
         // the last check saw the iterate before its update; report the
         // residual of the dq actually returned
@@ -1289,17 +1329,21 @@ UCFD_API int ucfd_lusgs_solve(ucfd_lusgs_solver *s, int mode, const double *b, d
             // accuracy FP32 can deliver
             const double inner_tol = std::max(1e-5, 0.5*rtol*bnorm/rn);
             hipLaunchKernelGGL(k_fill<float>, grid1(n), dim3(kB), 0, st, (int64_t)n, s->e32, 0.0f);
-            double s0 = 0.0;
-            for (int j = 0; info.passes < maxiter && !rc; ++j) {
-                rc = lower_pass<float>(s, st, j > 0, s->qb32, s->r32, s->e32, s->dstar32,
-                                       s->delta32, s->g32, s->d32, j > 0);
+            auto lower = [&](int j) {
+                return lower_pass<float>(s, st, j > 0, s->qb32, s->r32, s->e32, s->dstar32,
+                                         s->delta32, s->g32, s->d32, j > 0,
+                                         j > 0 ? s->norm + 3 : nullptr);
+            };
+            rc = lower(0);
+            bool stop = false;
+            for (int j = 0; info.passes < maxiter && !rc && !stop; ++j) {
+                if (j > 0 && !ahead) rc = lower(j);
                 if (!rc) rc = upper_pass<float>(s, st, s->qb32, s->dstar32, s->delta32, s->e32,
-                                                s->g32, s->d32, s->r32);
+                                                s->g32, s->d32, s->r32, j == 0, inner_tol);
+                if (!rc && ahead && info.passes + 1 < maxiter) rc = lower(j + 1);
                 double sn = 0.0;
-                if (!rc) rc = read_norm(s, st, &sn, fn);
+                if (!rc) rc = read_norm(s, st, &sn, fn, &stop);
                 info.passes++;
-                if (j == 0) s0 = sn;
-                if (s0 == 0.0 || sn <= inner_tol*s0) break;
             }
             // dq64 and e32 share the split layout: elementwise over 5N
             hipLaunchKernelGGL(k_add32, grid1(n), dim3(kB), 0, st, (int64_t)n, E, s->e32);
