@@ -8,13 +8,11 @@
 //
 // Colored calls launch one kernel over the cells icolor[n0:ne); a neighbour is
 // "lower" iff lcolor[nb] < lcolor[i] (upper: >).  Serial calls keep the
-// sequential semantics of src/lusgs/lusgs.c:175,227 (lower iff nb < i) and run
-// them level by level: a cell's level is one more than the highest level of
-// its lower neighbours, so each level is independent and the result equals
-// the sequential sweep exactly.
+// sequential semantics of src/lusgs/lusgs.c:175,227 (lower iff nb < i): one launch
+// in which a cell waits for its earlier neighbours (serial_kernels.hip), so the
+// result equals the sequential sweep exactly.
 #include "ucfd_internal.h"
 
-#include <algorithm>
 #include <mutex>
 #include <vector>
 
