@@ -316,6 +316,49 @@ def test_serial_sweeps_at_workgroup_edges(N, F, D, kind):
     L.call("ucfd_set_config", 5, 5, 3)
 
 
+@pytest.mark.parametrize("F", [4, 5, 6])
+def test_serial_sweeps_report_a_bad_index_and_follow_a_stream(F):
+    """An entry outside the table is reported by both sequential sweeps (status 3)
+    and its face skipped, as if the cell were its own neighbour there; on a caller's
+    stream the sweeps give the same bits as without one."""
+    say(f"serial sweeps, {F} faces: bad entries, caller's stream")
+    rng = np.random.default_rng(F)
+    N, D = 700, 3
+    good = rng.integers(0, N, (F, N)).astype(np.int32)
+    bad = good.copy()
+    for f, i, v in ((0, 5, N), (1, 300, -1), (F - 1, 699, 2**31 - 1), (2, 256, -2**31)):
+        bad[f, i], good[f, i] = v, i
+    fnv, fspr = rng.uniform(0.5, 1.0, (F, N)), rng.uniform(0.5, 2.0, (F, N))
+    vfn = np.ascontiguousarray(rng.normal(0.0, 0.6, (F, D, N)))
+    upts = rng.uniform(0.1, 0.3, (D + 2, N))
+    upts[0] += 1.0
+    upts[-1] += 2.5
+    rhs, dt = rng.normal(0.0, 1e-3, (D + 2, N)), rng.uniform(0.1, 0.2, N)
+    od, os_, oq, ou = O.serial_pass(good, fnv, vfn, fspr, dt, upts, rhs)
+    cv = torch_dev()
+    args = [cv(a) for a in (fnv, vfn, upts)]
+    diag, sp, lib = cv(od), cv(fspr), L.load()
+    for nei, want in ((bad, 3), (good, 0)):
+        dub, n = cv(rhs.copy()), cv(nei)
+        p = [L.ptr(a) for a in (n, *args, dub, diag, sp)]
+        assert lib.serial_ns_lower_sweep(N, F, *p) == want
+        assert np.array_equal(dub.cpu().numpy(), os_)
+        assert lib.serial_ns_upper_sweep(N, F, *p) == want
+        assert np.array_equal(dub.cpu().numpy(), oq)
+    import torch
+    st = torch.cuda.Stream()
+    dub, n = cv(rhs.copy()), cv(good)
+    torch.cuda.synchronize()
+    L.call("ucfd_set_stream", st.cuda_stream)
+    try:
+        L.call("serial_ns_lower_sweep", N, F, n, *args, dub, diag, sp)
+        L.call("serial_ns_upper_sweep", N, F, n, *args, dub, diag, sp)
+        st.synchronize()
+    finally:
+        L.call("ucfd_set_stream", None)
+    assert np.array_equal(dub.cpu().numpy(), oq)
+
+
 def test_hex32_ten_iterations_match_reference_fixture():
     say("32^3 permuted hex, 10 iterations, rhsb restored each iteration")
     z, mesh, flow = load_case("hex32p")
