@@ -16,13 +16,16 @@ extern "C" {
  * By default every call is synchronous.  After ucfd_set_stream(s) (a
  * hipStream_t), calls whose arrays are all device resident only enqueue on
  * s; ucfd_synchronize() waits for s and reports kernel-detected errors.
- * ucfd_set_stream(NULL) restores the synchronous default. */
+ * ucfd_set_stream(NULL) restores the synchronous default.  The sequential
+ * sweeps share one scratch space, so those enqueued on different streams run
+ * one after the other, and they cannot be captured into a graph. */
 int ucfd_set_stream(void *hip_stream);
 void *ucfd_get_stream(void);
 int ucfd_synchronize(void);
 /* number of visible HIP devices (0: every compute entry point will fail) */
 int ucfd_device_available(void);
-/* free the staging workspace used for host-pointer calls */
+/* free the workspace (staged host arrays, scratch of the sequential sweeps);
+ * waits for the calls that use it */
 int ucfd_release_workspace(void);
 
 /* ---- configuration --------------------------------------------------------

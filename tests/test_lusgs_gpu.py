@@ -359,6 +359,89 @@ def test_serial_sweeps_report_a_bad_index_and_follow_a_stream(F):
     assert np.array_equal(dub.cpu().numpy(), oq)
 
 
+def random_system(N, F, D, seed):
+    """(nei, fnv, vfn, fspr, dt, upts, rhs) with neighbours anywhere in the table."""
+    rng = np.random.default_rng(seed)
+    upts = rng.uniform(0.1, 0.3, (D + 2, N))
+    upts[0] += 1.0
+    upts[-1] += 2.5
+    return (rng.integers(0, N, (F, N)).astype(np.int32), rng.uniform(0.5, 1.0, (F, N)),
+            np.ascontiguousarray(rng.normal(0.0, 0.6, (F, D, N))), rng.uniform(0.5, 2.0, (F, N)),
+            rng.uniform(0.1, 0.2, N), upts, rng.normal(0.0, 1e-3, (D + 2, N)))
+
+
+def test_serial_sweeps_only_enqueue_on_a_callers_stream():
+    """On a caller's stream the sequential sweeps return before the work ahead of
+    them has run.  Their scratch is shared: a sweep on another stream, one that
+    needs more of it, and a call with host arrays, all issued meanwhile, give the
+    oracle's bits, as do the sweeps themselves."""
+    import torch
+    say("serial sweeps enqueued on two streams, host arrays between")
+    cv, lib, F = torch_dev(), L.load(), 6
+    systems = [random_system(N, F, 3, N) for N in (700, 900, 40000, 800)]
+    want = [O.serial_pass(s[0], s[1], s[2], s[3], s[4], s[5], s[6]) for s in systems]
+    dev = [[cv(a) for a in s] + [cv(w[0])] for s, w in zip(systems, want)]
+
+    def sweep(k, which):
+        nei, fnv, vfn, fspr, _, upts, b, diag = dev[k]
+        L.call(f"serial_ns_{which}_sweep", nei.shape[1], F, nei, fnv, vfn, upts, b, diag, fspr)
+
+    L.call("ucfd_release_workspace")
+    sweep(0, "lower")                   # the workspace is there, and small
+    dev[0][6] = cv(systems[0][6])
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    try:
+        with torch.cuda.stream(streams[0]):
+            torch.cuda._sleep(200_000_000)
+        L.call("ucfd_set_stream", streams[0].cuda_stream)
+        sweep(0, "lower")
+        sweep(0, "upper")
+        assert not streams[0].query(), "the sweeps waited for the stream"
+        L.call("ucfd_set_stream", streams[1].cuda_stream)
+        sweep(1, "lower")
+        sweep(2, "lower")               # the workspace grows
+        sweep(1, "upper")
+        L.call("ucfd_set_stream", streams[0].cuda_stream)
+        sweep(2, "upper")
+        L.call("ucfd_set_stream", None)
+        nei, fnv, vfn, fspr, _, upts, rhs = systems[3]
+        b = rhs.copy()
+        for which in ("lower", "upper"):
+            L.call(f"serial_ns_{which}_sweep", 800, F, nei, fnv, vfn, upts, b, want[3][0], fspr)
+        torch.cuda.synchronize()
+        L.call("ucfd_synchronize")
+    finally:
+        L.call("ucfd_set_stream", None)
+    assert np.array_equal(b, want[3][2])
+    for k in range(3):
+        assert np.array_equal(dev[k][6].cpu().numpy(), want[k][2]), k
+
+
+def test_serial_sweeps_refuse_capture():
+    """A captured sequential sweep is refused (status 2) and leaves the stream usable."""
+    import torch
+    say("serial sweeps under capture")
+    cv = torch_dev()
+    nei, fnv, vfn, fspr, dt, upts, rhs = random_system(600, 4, 3, 11)
+    od, os_, _, _ = O.serial_pass(nei, fnv, vfn, fspr, dt, upts, rhs)
+    args = [cv(a) for a in (nei, fnv, vfn, upts)]
+    b, diag, sp, lib = cv(rhs), cv(od), cv(fspr), L.load()
+    p = [L.ptr(a) for a in (*args, b, diag, sp)]
+    g, st, x = torch.cuda.CUDAGraph(), torch.cuda.Stream(), torch.zeros(8, device="cuda")
+    L.call("ucfd_set_stream", st.cuda_stream)
+    try:
+        with torch.cuda.graph(g, stream=st):
+            x += 1.0
+            rc = lib.serial_ns_lower_sweep(600, 4, *p)
+        assert rc == 2
+        assert lib.serial_ns_lower_sweep(600, 4, *p) == 0
+        L.call("ucfd_synchronize")
+    finally:
+        L.call("ucfd_set_stream", None)
+    assert np.array_equal(b.cpu().numpy(), os_)
+
+
 def test_hex32_ten_iterations_match_reference_fixture():
     say("32^3 permuted hex, 10 iterations, rhsb restored each iteration")
     z, mesh, flow = load_case("hex32p")

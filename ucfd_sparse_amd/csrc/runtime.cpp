@@ -29,8 +29,12 @@ struct State {
     int device = -1;
     int *words = nullptr;        // error words (error_word.h): pinned host memory
     int *words_dev = nullptr;    // their device address
-    void *ws = nullptr;          // staging workspace (grow only)
+    void *ws = nullptr;          // workspace: staged arrays and scratch (grow only)
     size_t ws_bytes = 0;
+    // recorded behind a call that was only enqueued with scratch in the workspace;
+    // whoever uses the workspace next, on any stream, waits for it (ws_busy)
+    hipEvent_t ws_event = nullptr;
+    bool ws_busy = false;
     UcfdConfig cfg{0, 0, 0};
     bool cfg_set = false;
 };
@@ -194,6 +198,33 @@ int UcfdStage::add(const void *p, size_t bytes, int dir)
     return nargs++;
 }
 
+// Before this call's use of the workspace: the stream (the host, if the
+// workspace is to grow) waits for the last call that was only enqueued with it.
+int UcfdStage::claim_ws(bool grow)
+{
+    State &s = st();
+    int rc;
+    if (scratch && s.user_stream) {
+        // replays would use the workspace in no order with the calls around them
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if ((rc = ucfd_check_hip(hipStreamIsCapturing(s.stream, &cap), fn, "hipStreamIsCapturing")))
+            return rc;
+        if (cap != hipStreamCaptureStatusNone)
+            return ucfd_report(UCFD_ERR_HIP, fn, "this call cannot be captured into a graph");
+        if (!s.ws_event &&
+            (rc = ucfd_check_hip(hipEventCreateWithFlags(&s.ws_event, hipEventDisableTiming), fn,
+                                 "hipEventCreate(workspace)")))
+            return rc;
+    }
+    if (!s.ws_busy) return UCFD_OK;
+    if (!grow)
+        return ucfd_check_hip(hipStreamWaitEvent(s.stream, s.ws_event, 0), fn,
+                              "hipStreamWaitEvent(workspace)");
+    rc = ucfd_check_hip(hipEventSynchronize(s.ws_event), fn, "hipEventSynchronize(workspace)");
+    if (!rc) s.ws_busy = false;
+    return rc;
+}
+
 int UcfdStage::enter()
 {
     State &s = st();
@@ -230,7 +261,14 @@ int UcfdStage::enter()
     // pass 2: place owners in the workspace
     size_t need = 0;
     for (int k = 0; k < nargs; ++k)
-        if (args[k].staged && args[k].owner == k) need += (args[k].bytes + 255) & ~(size_t)255;
+        if (args[k].staged) {
+            (args[k].dir == UCFD_SCRATCH ? scratch : any_staged) = true;
+            if (args[k].owner == k) need += (args[k].bytes + 255) & ~(size_t)255;
+        }
+    if (need && (rc = claim_ws(need > s.ws_bytes))) {
+        s.mu.unlock();
+        return rc;
+    }
     if (need > s.ws_bytes) {
         if (s.ws) (void)hipFree(s.ws);
         s.ws = nullptr;
@@ -246,7 +284,6 @@ int UcfdStage::enter()
     for (int k = 0; k < nargs; ++k) {
         Arg &a = args[k];
         if (!a.staged) continue;
-        (a.dir == UCFD_SCRATCH ? scratch : any_staged) = true;
         if (a.owner == k) {
             a.dev = (char *)s.ws + off;
             off += (a.bytes + 255) & ~(size_t)255;
@@ -282,11 +319,15 @@ int UcfdStage::leave(int status)
     if (any_staged || !s.user_stream) {
         int r = ucfd_sync_and_check(fn);
         if (!rc) rc = r;
+        if (any_staged || scratch) s.ws_busy = false;
     } else {
         int r = ucfd_check_hip(hipGetLastError(), fn, "kernel launch");
         if (!rc) rc = r;
         if (scratch) {
-            r = ucfd_check_hip(hipStreamSynchronize(s.stream), fn, "hipStreamSynchronize");
+            r = ucfd_check_hip(hipEventRecord(s.ws_event, s.stream), fn,
+                               "hipEventRecord(workspace)");
+            if (r) (void)hipStreamSynchronize(s.stream);
+            else s.ws_busy = true;
             if (!rc) rc = r;
         }
     }
@@ -342,7 +383,10 @@ UCFD_API int ucfd_release_workspace(void)
     std::lock_guard<std::recursive_mutex> g(s.mu);
     if (s.ws) {
         int rc = ucfd_check_hip(hipStreamSynchronize(s.stream), "ucfd_release_workspace", "sync");
+        if (!rc && s.ws_busy)
+            rc = ucfd_check_hip(hipEventSynchronize(s.ws_event), "ucfd_release_workspace", "sync");
         if (rc) return rc;
+        s.ws_busy = false;
         (void)hipFree(s.ws);
     }
     s.ws = nullptr;

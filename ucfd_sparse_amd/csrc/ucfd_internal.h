@@ -56,8 +56,8 @@ UCFD_HIDDEN int ucfd_poll(const unsigned long long *word, unsigned long long wan
 // Staging of host arrays for one call.  Device (or managed) pointers are used
 // in place; host pointers are copied to a library workspace on entry and
 // copied back on exit when written.  Arguments that alias share one buffer.
-// UCFD_SCRATCH: no array, space in the workspace while the call lasts (leave()
-// waits for the stream, so that the next call on any stream may use it).
+// UCFD_SCRATCH: no array, space in the workspace for the kernels of the call
+// (those of the next call that uses the workspace wait for them, on any stream).
 enum { UCFD_IN = 1, UCFD_OUT = 2, UCFD_INOUT = 3, UCFD_SCRATCH = 4 };
 
 struct UcfdStage {
@@ -74,6 +74,9 @@ struct UcfdStage {
     // copy outputs back and synchronise as the call contract requires
     int leave(int status);
     void *dev(int idx) const { return args[idx].dev; }
+
+private:
+    int claim_ws(bool grow);
 };
 
 // ---- legacy API (legacy_api.cpp)
