@@ -418,6 +418,27 @@ def test_serial_sweeps_only_enqueue_on_a_callers_stream():
         assert np.array_equal(dev[k][6].cpu().numpy(), want[k][2]), k
 
 
+@pytest.mark.parametrize("N, F, D", [(200_000, 6, 3), (250_000, 5, 3), (200_000, 3, 2)])
+def test_serial_sweeps_of_one_long_chain(N, F, D):
+    """Every cell waits for the one before it, over more cells than the chip holds at
+    once: the last workgroups to be resident wait for as long as a wave can."""
+    say(f"serial sweeps, a chain of {N} cells, {F} faces, {D}-D")
+    _, fnv, vfn, fspr, dt, upts, rhs = random_system(N, F, D, F)
+    i = np.arange(N)
+    nei = np.stack([np.clip(i + (1 if f % 2 else -1), 0, N - 1) for f in range(F)]).astype(np.int32)
+    od, os_, oq, _ = O.serial_pass(nei, fnv, vfn, fspr, dt, upts, rhs)
+    cv = torch_dev()
+    b, args = cv(rhs), [cv(a) for a in (nei, fnv, vfn, upts)]
+    diag, sp = cv(od), cv(fspr)
+    L.call("ucfd_set_config", D + 2, D + 2, D)
+    try:
+        for which, want in (("lower", os_), ("upper", oq)):
+            L.call(f"serial_ns_{which}_sweep", N, F, *args, b, diag, sp)
+            assert np.array_equal(b.cpu().numpy(), want), which
+    finally:
+        L.call("ucfd_set_config", 5, 5, 3)
+
+
 def test_serial_sweeps_refuse_capture():
     """A captured sequential sweep is refused (status 2) and leaves the stream usable."""
     import torch

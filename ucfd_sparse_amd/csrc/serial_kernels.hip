@@ -15,8 +15,12 @@
 // workgroup draws its cells by a ticket when it starts, so the earliest unfinished
 // cell is always ready and belongs to a workgroup that runs, or to the next one to
 // start once those before it have ended.  No lane stops while another lane of its
-// wave can go on.  A wait of more than kPolls rounds (seconds) raises
-// UCFD_KFLAG_STALL, and the launch drains.
+// wave can go on.  A wave that ends counts itself in ctl->ended, so a long wait in a
+// sweep that goes on is told from one that does not: kPolls idle rounds (0.2 us each
+// or more: a second) in which no wave of the launch has ended raise UCFD_KFLAG_STALL,
+// and the launch drains.  The first unfinished wave ends after at most 64 hops, 0.3
+// ms; a wave may wait for all that the chip holds, 0.8 s in a chain of 200K cells of
+// k_serial_any.
 //
 // What bounds it is the longest chain of cells; a hop costs a round of the loop
 // below, about 2 us (the loads of the awaited words, up to KS fluxes, the divisions
@@ -43,11 +47,17 @@ constexpr int kPolls = 1 << 22;
 typedef unsigned long long word;
 constexpr word kUnset = 0xFFF8A5C35A3C0F1Eull;
 
-// the words of pub, then the ticket and the stall word
+// behind the words of pub
+struct Control {
+    word ticket;            // workgroups started
+    unsigned stall, ended;  // a wave has given up; waves that ended
+};
+constexpr int kControl = sizeof(Control)/sizeof(word);
+
 __global__ __launch_bounds__(256) void k_unset(int64_t n, word *pub)
 {
     const int64_t st = (int64_t)gridDim.x*256;
-    for (int64_t k = (int64_t)blockIdx.x*256 + threadIdx.x; k < n + 2; k += st)
+    for (int64_t k = (int64_t)blockIdx.x*256 + threadIdx.x; k < n + kControl; k += st)
         pub[k] = k < n ? kUnset : 0ull;
 }
 
@@ -133,15 +143,32 @@ __device__ __forceinline__ int draw(word *ticket, int *sb)
     return *sb;
 }
 
-__device__ __forceinline__ bool given_up(int polls, word *stall, int *flag)
-{
-    if (polls == kPolls) {
+// The idle rounds of a wave since the launch last made progress
+struct Idle {
+    int rounds = 0;
+    unsigned ended = 0;
+    // after a round without progress: whether to give up
+    __device__ __forceinline__ bool give_up(Control *ctl, int *flag)
+    {
+        if (++rounds & 1023) return false;
+        if (__hip_atomic_load(&ctl->stall, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return true;
+        const unsigned e = __hip_atomic_load(&ctl->ended, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (e != ended) {
+            ended = e;
+            rounds = 0;
+        }
+        if (rounds < kPolls) return false;
         ucfd::raise(flag, UCFD_KFLAG_STALL);
-        __hip_atomic_store(stall, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&ctl->stall, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return true;
     }
-    return (polls & 1023) == 1023 &&
-           __hip_atomic_load(stall, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0ull;
+};
+
+// by every wave whose cells are all done
+__device__ __forceinline__ void count_end(Control *ctl)
+{
+    if ((threadIdx.x & 63) == 0)
+        __hip_atomic_fetch_add(&ctl->ended, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 template <int R> struct Chain {   // one lane's view of the published values
@@ -191,8 +218,8 @@ __global__ __launch_bounds__(KB) void k_serial(int N, const int *__restrict__ ne
     __shared__ int sb;
 #pragma unroll
     for (int k = 0; k < R; ++k) lds[k][threadIdx.x] = kUnset;
-    word *ticket = pub + (int64_t)R*N, *stall = ticket + 1;
-    const int b = draw(ticket, &sb);
+    Control *ctl = (Control *)(pub + (int64_t)R*N);
+    const int b = draw(&ctl->ticket, &sb);
     const Chain<R> C{lds, pub, N, (int64_t)b*KB};
     const int64_t q = C.q0 + threadIdx.x, i = DIR == 0 ? q : N - 1 - q;
     bool wait = q < N;
@@ -221,7 +248,7 @@ __global__ __launch_bounds__(KB) void k_serial(int N, const int *__restrict__ ne
             if ((DIR == 0 ? nb[f] : N - 1 - nb[f]) < q) rest |= 1 << f;
         }
     }
-    for (int polls = 0; __any(wait); ) {
+    for (Idle idle; __any(wait); ) {
         if (wait && pend == 0 && rest) {
 #pragma unroll
             for (int s = 0; s < KS; ++s) {
@@ -274,8 +301,9 @@ __global__ __launch_bounds__(KB) void k_serial(int N, const int *__restrict__ ne
             }
             wait = false;
         }
-        if (!__any(before != pend || done) && given_up(polls++, stall, flag)) return;
+        if (!__any(before != pend || done) && idle.give_up(ctl, flag)) return;
     }
+    count_end(ctl);
 }
 
 // Any face count: a lane takes its faces one after the other.
@@ -295,8 +323,8 @@ __global__ __launch_bounds__(KB) void k_serial_any(int N, int nface, const int *
     __shared__ int sb;
 #pragma unroll
     for (int k = 0; k < R; ++k) lds[k][threadIdx.x] = kUnset;
-    word *ticket = pub + (int64_t)R*N, *stall = ticket + 1;
-    const int b = draw(ticket, &sb);
+    Control *ctl = (Control *)(pub + (int64_t)R*N);
+    const int b = draw(&ctl->ticket, &sb);
     const Chain<R> C{lds, pub, N, (int64_t)b*KB};
     const int64_t q = C.q0 + threadIdx.x, i = DIR == 0 ? q : N - 1 - q;
     bool wait = q < N;
@@ -321,7 +349,7 @@ __global__ __launch_bounds__(KB) void k_serial_any(int N, int nface, const int *
         }
     };
     if (wait) next();
-    for (int polls = 0; __any(wait); ) {
+    for (Idle idle; __any(wait); ) {
         bool got = false;
         if (wait && f < nface) {
             word v[R];
@@ -350,15 +378,16 @@ __global__ __launch_bounds__(KB) void k_serial_any(int N, int nface, const int *
             wait = false;
             got = true;
         }
-        if (!__any(got) && given_up(polls++, stall, flag)) return;
+        if (!__any(got) && idle.give_up(ctl, flag)) return;
     }
+    count_end(ctl);
 }
 
 }  // namespace
 
 size_t ucfd_serial_scratch(int neles, int rows)
 {
-    return ((size_t)neles*(size_t)rows + 2)*sizeof(word);
+    return ((size_t)neles*(size_t)rows + kControl)*sizeof(word);
 }
 
 int ucfd_launch_serial(hipStream_t s, int dir, int neles, int nface, int ndims, int nt,
@@ -370,7 +399,7 @@ int ucfd_launch_serial(hipStream_t s, int dir, int neles, int nface, int ndims, 
     if ((ndims != 2 && ndims != 3) || nt < 0 || nt > 2) return UCFD_ERR_ARG;
     word *pub = (word *)scratch;
     const int64_t n = (int64_t)neles*(nt ? nt : ndims + 2);
-    const int64_t fb = (n + 2 + 255)/256;
+    const int64_t fb = (n + kControl + 255)/256;
     hipLaunchKernelGGL(k_unset, dim3((unsigned)(fb > 4096 ? 4096 : fb)), dim3(256), 0, s, n, pub);
     const dim3 g((unsigned)(((int64_t)neles + KB - 1)/KB)), b(KB);
 #define SER(DIR, ND, NT, FC) \
