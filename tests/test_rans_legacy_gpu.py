@@ -196,6 +196,38 @@ def test_serial_rans_sweeps_match_flowsys_oracle(kind, m, nt):
         assert_close(dq[nfv:], oq, f"serial {kind} nt={nt} dQ ({tag})")
 
 
+@pytest.mark.parametrize("N, F, D, nt, kind", [
+    (1, 3, 2, 1, "random"), (255, 3, 2, 2, "random"), (257, 4, 2, 1, "near"),
+    (900, 6, 2, 2, "random"), (3000, 3, 2, 1, "near"), (256, 3, 3, 1, "random"),
+    (700, 4, 3, 2, "random"), (3000, 6, 3, 1, "near"), (1300, 6, 3, 2, "random"),
+    (513, 4, 2, 2, "line"), (400_000, 4, 3, 1, "line"), (300_000, 6, 3, 2, "line")])
+def test_serial_rans_sweeps_at_workgroup_edges(N, F, D, nt, kind):
+    """The sequential turbulence sweeps on tables of any shape, every face count and
+    dimension with a kernel: one and many workgroups of 256 cells, neighbours near
+    and far, and lines (every cell waits for the one before it), two of them longer
+    than the chip holds at once.  Bit for bit."""
+    say(f"serial RANS sweeps, {N} cells, {F} faces, {D}-D, {nt} rows, {kind}")
+    rng = np.random.default_rng(N + F + nt)
+    i = np.arange(N)
+    nei = {"random": lambda: rng.integers(0, N, (F, N)),
+           "line": lambda: np.stack([np.clip(i + (1 if f % 2 else -1), 0, N - 1) for f in range(F)]),
+           "near": lambda: np.clip(i + rng.integers(-70, 70, (F, N)), 0, N - 1)}[kind]()
+    mesh = M.Mesh(np.ascontiguousarray(nei, np.int32), rng.uniform(0.5, 1.0, (F, N)),
+                  np.ascontiguousarray(rng.normal(0.0, 0.6, (F, D, N))), None, None)
+    upts = rng.uniform(0.1, 0.3, (D + 2 + nt, N))
+    upts[0] += 1.0
+    upts[D + 1] += 2.5
+    flow = M.Flow(upts, rng.uniform(0.5, 2.0, (F, N)), rng.uniform(0.1, 0.2, N),
+                  np.zeros((D + 2 + nt, N)))
+    flow, tfspr = with_turbulence(mesh, flow, nt, N)
+    L.call("ucfd_set_config", D + 2 + nt, D + 2, D)
+    od, os_, oq = bridge_oracle(mesh, flow, tfspr, D + 2)
+    for two in (False, True):
+        td, ds, dq = run_gpu(mesh, flow, tfspr, D + 2, False, None, two)
+        assert np.array_equal(td, od), "tdiag"
+        assert np.array_equal(ds, os_) and np.array_equal(dq[D + 2:], oq), two
+
+
 def test_rans_sweeps_refuse_a_configuration_without_turbulence_rows():
     mesh = M.tet_mesh(3, seed=3)
     flow = M.flow_fields(mesh, seed=3)
