@@ -986,7 +986,8 @@ inline bool wave_per_face(int F, int cnt) { return F == 6 || cnt <= kWfTets; }
 // previous pass's upper launch formed the first colour's residual, block
 // partials and dstar (k_upper_upd_res), so the pass starts at the second
 // colour.  With more than one colour the last colour's launch also does that
-// colour's upper step, writing delta and e (upper_pass then skips it).
+// colour's upper step, writing delta and e (upper_pass then skips it); stop
+// (lower_ahead): e only if *stop is still zero when the launch runs.
 template <typename T>
 int lower_pass(ucfd_lusgs_solver *s, hipStream_t st, bool with_res, const T *qb, const T *rhs,
                T *e, T *dstar, T *delta, const Face4<T> *geo, const T *diag, bool pre0 = false,
@@ -1124,9 +1125,12 @@ int read_norm(ucfd_lusgs_solver *s, hipStream_t st, double *out, const char *fn,
 // -> 184; 48K tets of 4 colours 530 -> 543; mixed 900 hexes 225 -> 204, 8.8K 263 ->
 // 237, 45K 341 -> 301, 123K 423 -> 406, 258K 629 -> 641; 6K tets 280 -> 247, 197K
 // 580 -> 562, 511K 1145 -> 1176.
+// Only the wave-per-face launch of the last colour reads the decision (stop): with
+// the thread-per-cell one the solve would end with a pass too many.
 bool lower_ahead(const ucfd_lusgs_solver *s, int mode)
 {
-    return s->nc <= 2 && s->N <= (mode == UCFD_SOLVE_FP64 ? 65536 : 200000);
+    return s->nc <= 2 && s->N <= (mode == UCFD_SOLVE_FP64 ? 65536 : 200000) &&
+           wave_per_face(s->F, s->off[s->nc] - s->off[s->nc - 1]);
 }
 
 }  // namespace
