@@ -6,9 +6,11 @@
  * reference call sites.  Semantics are the sequential sweeps of
  * src/lusgs/lusgs.c:157-257: the lower sweep visits cells in ascending id and
  * uses neighbours nb < i, the upper sweep visits them in descending id and
- * uses neighbours nb > i.  On the GPU the sweep runs level by level (a cell's
- * level is one more than the highest level of the neighbours it depends on),
- * which gives exactly the sequential result.
+ * uses neighbours nb > i.  On the GPU a sweep is one launch in which the cells
+ * start in that order and each waits for the earlier neighbours it uses, which
+ * gives exactly the sequential result.  The waits are bounded: a launch that
+ * makes no progress for about a second is given up and reported with status 2
+ * (its results are undefined).
  *
  * Layouts, pointer kinds and return values as in coloredlusgs.h.
  */

@@ -334,6 +334,27 @@ def test_status_codes(K, tet3):
     assert (st, it) == (K.RHOBREAKDOWN, 0)
 
 
+@pytest.mark.parametrize("bn", [1000, 40_000])
+def test_pi_breakdown_leaves_x(K, bn):
+    """BiCGSTAB with rt.(A p) = 0 in the first iteration (skew blocks, a residual of
+    equal entries): the breakdown status, and x as it was, where the kernels sum
+    the partials of a reduction themselves (8 of them) and where a launch of its
+    own does (313)."""
+    say(f"pi breakdown, {bn} blocks")
+    rng = np.random.default_rng(bn)
+    rows = np.arange(bn + 1, dtype=np.int32)
+    mat = K.SpMat(dev(rows), dev(rows[:-1]), dev(np.tile([0.0, 1.0, -1.0, 0.0], bn)), bn, 2)
+    x0 = rng.integers(-9, 10, 2 * bn).astype(np.float64)    # every sum below is exact
+    r = np.repeat(rng.integers(1, 8, bn), 2).astype(np.float64)
+    b = r + np.stack([x0[1::2], -x0[::2]], 1).reshape(-1)
+    s = K.Solver("bicgstab", 2 * bn, 5, 1e-10)
+    for _ in range(2):
+        x = dev(x0)
+        st, it, _ = s.solve(K.Precon.none(), mat, x, dev(b))
+        assert (st, it) == (K.PIBREAKDOWN, 0)
+        assert np.array_equal(x.cpu().numpy(), x0)
+
+
 def test_errors_are_reported_not_faulted(K, tet3):
     say("index and pivot errors")
     from ucfd_sparse_amd import lib as L

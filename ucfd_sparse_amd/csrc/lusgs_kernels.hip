@@ -661,15 +661,18 @@ __global__ __launch_bounds__(64*FC) void k_rans_wf(
 //   hexes, own numbering: 101K 48.6 -> 45.1, 246K 81.7 -> 84.3,
 //     486K 150.9 -> 148.7, 1.0M 303 -> 291
 // kWfRound: the cells the chip holds at once as six-wave workgroups (5 per
-// CU); between one and three such rounds of hexes the last, partly filled one
-// costs what the extra waves bring.  With turbulence rows hexes gain below one
-// round only (101K 57.0 -> 53.8, 246K 89.0 -> 88.7, 1.0M 303.7 -> 309.7).
+// CU); between one and three such rounds of hexes (246K and 486K above, whose
+// launches are of 123K and 243K cells, stay with the thread per cell) the last,
+// partly filled one costs what the extra waves bring.  Declared hexes always take
+// the wave per face (launch_sweep_f).  With turbulence rows hexes gain below one
+// round only (101K 57.0 -> 53.8, 246K 89.0 -> 88.7, 1.0M 303.7 -> 309.7:
+// launch_rans_f).
 constexpr int kWfRound = 256*5*64;
 constexpr int kWfTets = 400000;
 
 inline bool wave_per_face(int mode, int nface, int cnt)
 {
-    if (nface == 6) return mode >= 2 || cnt <= kWfRound || cnt >= 3*kWfRound;
+    if (nface == 6) return cnt <= kWfRound || cnt >= 3*kWfRound;
     return mode < 2 || cnt <= kWfTets;
 }
 

@@ -140,8 +140,8 @@ bool ucfd_is_device_ptr(const void *p)
 }
 
 // Wait for the stream and turn a raised error bit into a status.  A wait and
-// four host reads: a synchronous sweep of 365 cells takes 15.5 us where it
-// took 17.9 with an error word copied back from device memory.
+// a host read per error word: a synchronous sweep of 365 cells takes 15.5 us where
+// it took 17.9 with an error word copied back from device memory.
 int ucfd_sync_and_check(const char *fn)
 {
     State &s = st();
