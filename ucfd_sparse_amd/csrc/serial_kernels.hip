@@ -15,12 +15,12 @@
 // workgroup draws its cells by a ticket when it starts, so the earliest unfinished
 // cell is always ready and belongs to a workgroup that runs, or to the next one to
 // start once those before it have ended.  No lane stops while another lane of its
-// wave can go on.  A wave that ends counts itself in ctl->ended, so a long wait in a
-// sweep that goes on is told from one that does not: kPolls idle rounds (0.2 us each
-// or more: a second) in which no wave of the launch has ended raise UCFD_KFLAG_STALL,
-// and the launch drains.  The first unfinished wave ends after at most 64 hops, 0.3
-// ms; a wave may wait for all that the chip holds, 0.8 s in a chain of 200K cells of
-// k_serial_any.
+// wave can go on.  A wave that ends after a long wait counts itself in ctl->ended, so
+// a wait in a sweep that goes on is told from one in a sweep that does not: kPolls
+// idle rounds (0.2 us each or more: a second) without a change there raise
+// UCFD_KFLAG_STALL, and the launch drains.  The first unfinished wave ends after at
+// most 64 hops, 0.3 ms; a wave may wait for all that the chip holds, 0.8 s in a chain
+// of 200K cells of k_serial_any.
 //
 // What bounds it is the longest chain of cells; a hop costs a round of the loop
 // below, about 2 us (the loads of the awaited words, up to KS fluxes, the divisions
@@ -50,7 +50,7 @@ constexpr word kUnset = 0xFFF8A5C35A3C0F1Eull;
 // behind the words of pub
 struct Control {
     word ticket;            // workgroups started
-    unsigned stall, ended;  // a wave has given up; waves that ended
+    unsigned stall, ended;  // a wave has given up; waves that waited long and ended
 };
 constexpr int kControl = sizeof(Control)/sizeof(word);
 
@@ -147,6 +147,7 @@ __device__ __forceinline__ int draw(word *ticket, int *sb)
 struct Idle {
     int rounds = 0;
     unsigned ended = 0;
+    __device__ __forceinline__ bool long_wait() const { return rounds >= 1024 || ended; }
     // after a round without progress: whether to give up
     __device__ __forceinline__ bool give_up(Control *ctl, int *flag)
     {
@@ -164,10 +165,12 @@ struct Idle {
     }
 };
 
-// by every wave whose cells are all done
-__device__ __forceinline__ void count_end(Control *ctl)
+// By a wave whose cells are all done, if it ever had to wait for long: those that did
+// not end within a millisecond, and counting every wave in one word cost 10 ns each
+// (5.3M cells in two levels 0.47 -> 1.27 ms).
+__device__ __forceinline__ void count_end(const Idle &idle, Control *ctl)
 {
-    if ((threadIdx.x & 63) == 0)
+    if (idle.long_wait() && (threadIdx.x & 63) == 0)
         __hip_atomic_fetch_add(&ctl->ended, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -248,7 +251,8 @@ __global__ __launch_bounds__(KB) void k_serial(int N, const int *__restrict__ ne
             if ((DIR == 0 ? nb[f] : N - 1 - nb[f]) < q) rest |= 1 << f;
         }
     }
-    for (Idle idle; __any(wait); ) {
+    Idle idle;
+    while (__any(wait)) {
         if (wait && pend == 0 && rest) {
 #pragma unroll
             for (int s = 0; s < KS; ++s) {
@@ -303,7 +307,7 @@ __global__ __launch_bounds__(KB) void k_serial(int N, const int *__restrict__ ne
         }
         if (!__any(before != pend || done) && idle.give_up(ctl, flag)) return;
     }
-    count_end(ctl);
+    count_end(idle, ctl);
 }
 
 // Any face count: a lane takes its faces one after the other.
@@ -349,7 +353,8 @@ __global__ __launch_bounds__(KB) void k_serial_any(int N, int nface, const int *
         }
     };
     if (wait) next();
-    for (Idle idle; __any(wait); ) {
+    Idle idle;
+    while (__any(wait)) {
         bool got = false;
         if (wait && f < nface) {
             word v[R];
@@ -380,7 +385,7 @@ __global__ __launch_bounds__(KB) void k_serial_any(int N, int nface, const int *
         }
         if (!__any(got) && idle.give_up(ctl, flag)) return;
     }
-    count_end(ctl);
+    count_end(idle, ctl);
 }
 
 }  // namespace
