@@ -324,11 +324,14 @@ int UcfdStage::leave(int status)
         int r = ucfd_check_hip(hipGetLastError(), fn, "kernel launch");
         if (!rc) rc = r;
         if (scratch) {
-            r = ucfd_check_hip(hipEventRecord(s.ws_event, s.stream), fn,
-                               "hipEventRecord(workspace)");
-            if (r) (void)hipStreamSynchronize(s.stream);
-            else s.ws_busy = true;
-            if (!rc) rc = r;
+            if (hipEventRecord(s.ws_event, s.stream) == hipSuccess) {
+                s.ws_busy = true;
+            } else {
+                // a stream of another device than the event's: wait for it instead
+                (void)hipGetLastError();
+                r = ucfd_check_hip(hipStreamSynchronize(s.stream), fn, "hipStreamSynchronize");
+                if (!rc) rc = r;
+            }
         }
     }
     s.mu.unlock();
